@@ -242,9 +242,7 @@ __global__ __launch_bounds__(MD_BLOCK) void k_md(MDArgs a) {
       float nl;
       if (!try_normalize(c.m1.t - c.m2.t, NCX_FLT_EPS, &dir, &nl)) dir = f3{1.f, 0.f, 0.f};
       Simplex sx;
-      sx_init(sx);
-      sx_reset(sx, cso_from<G>(c, dir, a.P, gl));
-      const GJKOut r = gjk<G>(c, NCX_FLT_MAX, sx, a.P, gl, 10000);
+      const GJKOut r = gjk<G>(c, dir, NCX_FLT_MAX, sx, a.P, gl, 10000);
       const float d = r.status == GJK_S_CLOSEST ? norm(r.p1 - r.p2) : 0.f;
       if (d < best) best = d;
     };
@@ -341,6 +339,7 @@ extern "C" int ncx_mesh_contact_batch(ncx_mesh* m, const ncx_pose* mesh_pose, nc
   hipLaunchKernelGGL(k_mc_tri_records, dim3(ceil_div(nt, 256)), dim3(256), 0, ctx->stream,
                      C->shapes.as<ncx_shape>() + ns, nt);
   C->n = nc;
+  C->buckets = s->buckets;  // a triangle changes no pair's bucket
   C->npts = s->npts;
   C->hx = s->hx; C->hy = s->hy; C->hz = s->hz;  // borrowed (never released through C)
   C->tri = m->tris.as<float4>();
@@ -388,7 +387,7 @@ extern "C" int ncx_mesh_contact_batch(ncx_mesh* m, const ncx_pose* mesh_pose, nc
   NCX_HIP_CHECK(hipGetLastError());
   if (total) {
     // query::contact(mesh pose, triangle, shape pose, shape, prediction) on every candidate
-    if ((rc = contact_tiers_reserve(C->tiers, total))) return rc;
+    if ((rc = contact_tiers_reserve(C->tiers, ctx, total, total))) return rc;
     if ((rc = contacts_launch_device_count(C, C->tiers, ctx, m->cposes.as<ncx_pose>(), m->ca.as<uint32_t>(),
                                            m->cb.as<uint32_t>(), m->ctot.as<uint32_t>(), total, prediction, nullptr,
                                            10000, m->chas.as<uint8_t>(), m->cw1.as<float>(), m->cw2.as<float>(),

@@ -71,7 +71,6 @@ __device__ __forceinline__ CSO vget(const Arena& A, uint32_t i) {
   CSO c;
   c.o1 = f3{f[0], f[1], f[2]};
   c.o2 = f3{f[3], f[4], f[5]};
-  c.p = c.o1 - c.o2;
   return c;
 }
 __device__ __forceinline__ f3 vpt(const Arena& A, uint32_t i) {
@@ -102,7 +101,7 @@ __device__ __forceinline__ void heap_sift_up(HeapE* h, uint32_t pos) {
 // (nearest first) is where the climb stops.  The ancestors below it each move down one level
 // along the path and the element takes the last one's slot, which is what the loop leaves.
 // Needs as many lanes as the heap has levels above pos.
-template <int G, bool GMEM>
+template <int G>
 __device__ __forceinline__ void heap_sift_up_par(HeapE* h, uint32_t pos, int gl) {
   const HeapE e = h[pos];
   const uint32_t k = pos + 1;
@@ -120,11 +119,11 @@ __device__ __forceinline__ void heap_sift_up_par(HeapE* h, uint32_t pos, int gl)
   __builtin_amdgcn_wave_barrier();
   if (gl == 0) h[s == 0 ? pos : (k >> s) - 1u] = e;
   __builtin_amdgcn_wave_barrier();
-  // A device-memory heap: the other lanes' stores must have landed before anyone reads the heap.
-  if constexpr (GMEM) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+  // the other lanes' stores must have landed before anyone reads the heap
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
 }
 
-template <int G, int PAR>
+template <int G>
 __device__ __forceinline__ bool heap_pop(HeapE* h, uint32_t& len, HeapE& out, int gl) {
   if (len == 0) return false;
   len -= 1;
@@ -143,8 +142,7 @@ __device__ __forceinline__ bool heap_pop(HeapE* h, uint32_t& len, HeapE& out, in
     }
     if (child == end - 1) { h[pos] = h[child]; pos = child; }
     h[pos] = e;
-    if constexpr (PAR != 0) heap_sift_up_par<G, PAR == 2>(h, pos, gl);
-    else heap_sift_up(h, pos);
+    heap_sift_up_par<G>(h, pos, gl);
   }
   out = item;
   return true;
@@ -191,7 +189,7 @@ __device__ __forceinline__ void face_points(const Arena& A, const FaceD& f, f3& 
   const CSO b = vget(A, f.pts[1]);
   const CSO c = vget(A, f.pts[2]);
   Loc loc;
-  proj_triangle(a.p, b.p, c.p, loc);
+  proj_triangle(a.pt(), b.pt(), c.pt(), loc);
   float b0 = 0.f, b1 = 0.f, b2 = 0.f;
   if (loc.kind == LOC_FACE) { b0 = loc.bc0; b1 = loc.bc1; b2 = loc.bc2; }
   p1 = a.o1 * b0 + b.o1 * b1 + c.o1 * b2;
@@ -229,25 +227,11 @@ __device__ __forceinline__ bool can_be_seen(const Arena& A, const FaceD& f, uint
 }
 
 // Suspending and resuming an EPA run between arena tiers.  A run that is about to outgrow its
-// arena at an iteration boundary (the vertex capacity reached, or fewer than SUSPEND_MARGIN free
-// face slots) saves its polytope -- vertices, faces, heap and loop scalars, bit for bit -- to
+// arena at an iteration boundary (no room for a usual iteration's vertex, faces and heap entries)
+// saves its polytope -- vertices, faces, heap and loop scalars, bit for bit -- to
 // slot i of the next tier's input, where i is its entry in the overflow list, and marks the
-// entry with ENTRY_SAVED.  The next tier replays the pair's GJK, which rebuilds the same simplex,
-// and continues the EPA from the saved state instead of from that simplex, so only a run that
-// outgrows a tier mid-iteration (a silhouette longer than the margin), or finds no free slot,
-// starts again.
-struct EpaIO {
-  const uint8_t* load;  // saved run to continue (null: build the polytope from the simplex)
-  uint8_t* save;        // slots for runs this launch suspends (null: it does not suspend)
-  size_t save_bytes;    // bytes per slot
-  uint32_t save_cap;    // slots
-  uint32_t* count;      // the overflow list's counter and entries
-  uint32_t* list;
-  uint32_t list_cap;
-  uint32_t k;           // the pair's index
-};
-#define EPA_SUSPENDED 3
-#define SUSPEND_MARGIN 16u
+// entry with ENTRY_SAVED.  The next tier continues from the saved state; only a run that
+// outgrows a tier mid-iteration, or finds no free slot, starts again from its simplex.
 #define ENTRY_SAVED 0x80000000u
 #define SAVE_HEADER_WORDS 8u
 
@@ -260,22 +244,6 @@ template <int G>
 __device__ __forceinline__ void copy_words(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, uint32_t n,
                                            int gl) {
   for (uint32_t w = (uint32_t)gl; w < n; w += G) dst[w] = src[w];
-}
-
-template <int G>
-__device__ __forceinline__ void epa_save(uint8_t* slot, const Arena& A, int gl, uint32_t nv, uint32_t nf, uint32_t hl,
-                                         int niter, int iters, HeapE best, float max_dist) {
-  uint32_t* d = (uint32_t*)slot;
-  if (gl == 0) {
-    d[0] = nv; d[1] = nf; d[2] = hl; d[3] = (uint32_t)niter; d[4] = (uint32_t)iters;
-    d[5] = __float_as_uint(best.neg_dist); d[6] = best.id; d[7] = __float_as_uint(max_dist);
-  }
-  d += SAVE_HEADER_WORDS;
-  copy_words<G>(d, (const uint32_t*)A.verts, nv * (uint32_t)(sizeof(VertA) / 4), gl);
-  d += nv * (sizeof(VertA) / 4);
-  copy_words<G>(d, (const uint32_t*)A.faces, nf * (uint32_t)(sizeof(FaceD) / 4), gl);
-  d += nf * (sizeof(FaceD) / 4);
-  copy_words<G>(d, (const uint32_t*)A.heap, hl * (uint32_t)(sizeof(HeapE) / 4), gl);
 }
 
 // Loads a saved run into A (whose capacities are at least the saving tier's); the caller
@@ -295,13 +263,13 @@ __device__ __forceinline__ void epa_load(const uint8_t* slot, const Arena& A, in
   copy_words<G>((uint32_t*)A.heap, s, hl * (uint32_t)(sizeof(HeapE) / 4), gl);
 }
 
-// EPA::closest_points (epa3.rs:219-430).  compute_silhouette's recursion
-// (:432-454) becomes an explicit stack visiting faces in the same order.  PAR picks how the
-// group's lanes share the work: 0 every lane runs the same sequential steps, 1 the lane-parallel
-// steps on an LDS arena, 2 the same on a device-memory arena (with workgroup fences).
-template <int G, int PAR>
-__device__ __forceinline__ int epa(const Ctx2& c, const Simplex& s, const Pool& P, int gl, const Arena& A, f3& p1, f3& p2, f3& n,
-                   int& iters, const EpaIO& io) {
+// EPA::closest_points (epa3.rs:219-430) on a device-memory arena, for the runs that outgrow every
+// LDS arena (ncx_epa.h).  compute_silhouette's recursion (:432-454) becomes an explicit stack
+// visiting faces in the same order; the group's lanes share the work, with workgroup fences
+// between their writes and each other's reads.
+template <int G>
+__device__ __forceinline__ int epa(const Ctx2& c, const Simplex& s, const Pool& P, int gl, const Arena& A, f3& p1,
+                                   f3& p2, f3& n, int& iters, const uint8_t* load) {
   const float eps_tol = NCX_FLT_EPS * 100.f;
   const float gjk_tol = NCX_FLT_EPS * 10.f;
   iters = 0;
@@ -309,8 +277,8 @@ __device__ __forceinline__ int epa(const Ctx2& c, const Simplex& s, const Pool& 
   int niter = 0;
   float max_dist = NCX_FLT_MAX;
   HeapE best;
-  if (io.load) {
-    epa_load<G>(io.load, A, gl, nv, nf, hl, niter, iters, best, max_dist);
+  if (load) {
+    epa_load<G>(load, A, gl, nv, nf, hl, niter, iters, best, max_dist);
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   } else {
     vset(A, nv++, s.v0);
@@ -352,13 +320,6 @@ __device__ __forceinline__ int epa(const Ctx2& c, const Simplex& s, const Pool& 
         }
       }
     } else {
-      if (s.dim == 1) {
-        f3 dpt = vpt(A, 1) - vpt(A, 0);
-        // nalgebra orthonormal_subspace_basis for one vector; epa3.rs:299-305 keeps a x dpt.
-        f3 a = fabsf(dpt.x) > fabsf(dpt.y) ? f3{dpt.z, 0.f, -dpt.x} : f3{0.f, -dpt.z, dpt.y};
-        a = normalize(a);
-        vset(A, nv++, cso_from<G>(c, cross(a, dpt), P, gl));
-      }
       FaceD f1, f2;
       f3 n1, n2;
       make_face(A, 0, 1, 2, 1, 1, 1, f1, n1);
@@ -373,18 +334,7 @@ __device__ __forceinline__ int epa(const Ctx2& c, const Simplex& s, const Pool& 
   }
   HeapE fid;
   for (;;) {
-    if constexpr (PAR != 0) {
-      if (io.save && (nv >= A.vcap || nf + SUSPEND_MARGIN > A.fcap)) {
-        uint32_t slot = 0;
-        if (gl == 0) slot = atomicAdd(io.count, 1u);
-        slot = (uint32_t)__shfl((int)slot, __lane_id() & ~(G - 1), 64);
-        const bool saved = slot < io.save_cap;
-        if (saved) epa_save<G>(io.save + (size_t)slot * io.save_bytes, A, gl, nv, nf, hl, niter, iters, best, max_dist);
-        if (gl == 0 && slot < io.list_cap) io.list[slot] = io.k | (saved ? ENTRY_SAVED : 0u);
-        return EPA_SUSPENDED;
-      }
-    }
-    if (!heap_pop<G, PAR>(A.heap, hl, fid, gl)) break;
+    if (!heap_pop<G>(A.heap, hl, fid, gl)) break;
     FaceD face = A.faces[fid.id];
     if (face.deleted) continue;
     if (nv >= A.vcap) return EPA_OVERFLOW;
@@ -393,7 +343,7 @@ __device__ __forceinline__ int epa(const Ctx2& c, const Simplex& s, const Pool& 
     iters += 1;
     uint32_t sp_id = nv;
     vset(A, nv++, cso);
-    float cand = dot(cso.p, face_n);
+    float cand = dot(cso.pt(), face_n);
     if (cand < max_dist) { best = fid; max_dist = cand; }
     float curr_dist = -fid.neg_dist;
     if (max_dist - curr_dist < eps_tol) {
@@ -405,159 +355,103 @@ __device__ __forceinline__ int epa(const Ctx2& c, const Simplex& s, const Pool& 
     A.faces[fid.id].deleted = 1;
     // compute_silhouette for the three neighbours, depth first.
     uint32_t ns = 0, sp = 0;
-    if constexpr (PAR != 0) {
-      // Each stack entry's visibility (can_be_seen through the entry's edge) is computed when it
-      // is pushed, the entries pushed together by different lanes of the group at once, and kept
-      // in bit 15 of the entry: it depends only on the face's vertices, the new point and the
-      // edge, none of which change during the search.  The pops, the deleted-face skips and the
-      // pushes are the search's own, so the silhouette comes out in the same order.
-      const int lane = __lane_id();
-      const int gbase = lane & ~(G - 1);
-      {
-        const int k = 2 - (gl % 3);  // lanes 0, 1, 2 take the entries in push order
-        // value selects, not an index into the register copy of the face (that would spill it)
-        const uint32_t adj = k == 0 ? face.adj[0] : (k == 1 ? face.adj[1] : face.adj[2]);
-        const uint32_t ptk = k == 0 ? face.pts[0] : (k == 1 ? face.pts[1] : face.pts[2]);
-        const bool v = can_be_seen(A, A.faces[adj], sp_id, next_ccw(A.faces[adj], ptk));
+    // Each stack entry's visibility (can_be_seen through the entry's edge) is computed when it
+    // is pushed, the entries pushed together by different lanes of the group at once, and kept
+    // in bit 15 of the entry: it depends only on the face's vertices, the new point and the
+    // edge, none of which change during the search.  The pops, the deleted-face skips and the
+    // pushes are the search's own, so the silhouette comes out in the same order.
+    const int lane = __lane_id();
+    const int gbase = lane & ~(G - 1);
+    {
+      const int k = 2 - (gl % 3);  // lanes 0, 1, 2 take the entries in push order
+      // value selects, not an index into the register copy of the face (that would spill it)
+      const uint32_t adj = k == 0 ? face.adj[0] : (k == 1 ? face.adj[1] : face.adj[2]);
+      const uint32_t ptk = k == 0 ? face.pts[0] : (k == 1 ? face.pts[1] : face.pts[2]);
+      const bool v = can_be_seen(A, A.faces[adj], sp_id, next_ccw(A.faces[adj], ptk));
+      const uint64_t vb = __ballot(v) >> gbase;
+      for (int j = 0; j < 3; ++j) {
+        const uint32_t adjj = face.adj[2 - j];
+        const uint32_t oj = next_ccw(A.faces[adjj], face.pts[2 - j]);
+        A.stack[sp++] = SilE{(uint16_t)adjj, (uint16_t)(oj | (((vb >> j) & 1ull) ? 0x8000u : 0u))};
+      }
+    }
+    while (sp > 0) {
+      const SilE e = A.stack[--sp];
+      const uint32_t opp = e.opp & 3u;
+      FaceD& fa = A.faces[e.face];
+      if (fa.deleted) continue;
+      if (!(e.opp & 0x8000u)) {
+        if (ns >= A.scap) return EPA_OVERFLOW;
+        A.sil[ns++] = SilE{e.face, (uint16_t)opp};
+      } else {
+        fa.deleted = 1;
+        const uint32_t i1 = (opp + 2) % 3, i2 = opp;
+        const uint32_t adj1 = fa.adj[i1], adj2 = fa.adj[i2];
+        const uint32_t o1 = next_ccw(A.faces[adj1], fa.pts[i1]);
+        const uint32_t o2 = next_ccw(A.faces[adj2], fa.pts[i2]);
+        if (sp + 2 > A.stcap) return EPA_OVERFLOW;
+        const bool odd = (gl & 1) != 0;  // even lanes: adj2 (pushed first), odd lanes: adj1
+        const bool v = can_be_seen(A, A.faces[odd ? adj1 : adj2], sp_id, odd ? o1 : o2);
         const uint64_t vb = __ballot(v) >> gbase;
-        for (int j = 0; j < 3; ++j) {
-          const uint32_t adjj = face.adj[2 - j];
-          const uint32_t oj = next_ccw(A.faces[adjj], face.pts[2 - j]);
-          A.stack[sp++] = SilE{(uint16_t)adjj, (uint16_t)(oj | (((vb >> j) & 1ull) ? 0x8000u : 0u))};
-        }
-      }
-      while (sp > 0) {
-        const SilE e = A.stack[--sp];
-        const uint32_t opp = e.opp & 3u;
-        FaceD& fa = A.faces[e.face];
-        if (fa.deleted) continue;
-        if (!(e.opp & 0x8000u)) {
-          if (ns >= A.scap) return EPA_OVERFLOW;
-          A.sil[ns++] = SilE{e.face, (uint16_t)opp};
-        } else {
-          fa.deleted = 1;
-          const uint32_t i1 = (opp + 2) % 3, i2 = opp;
-          const uint32_t adj1 = fa.adj[i1], adj2 = fa.adj[i2];
-          const uint32_t o1 = next_ccw(A.faces[adj1], fa.pts[i1]);
-          const uint32_t o2 = next_ccw(A.faces[adj2], fa.pts[i2]);
-          if (sp + 2 > A.stcap) return EPA_OVERFLOW;
-          const bool odd = (gl & 1) != 0;  // even lanes: adj2 (pushed first), odd lanes: adj1
-          const bool v = can_be_seen(A, A.faces[odd ? adj1 : adj2], sp_id, odd ? o1 : o2);
-          const uint64_t vb = __ballot(v) >> gbase;
-          A.stack[sp++] = SilE{(uint16_t)adj2, (uint16_t)(o2 | ((vb & 1ull) ? 0x8000u : 0u))};
-          A.stack[sp++] = SilE{(uint16_t)adj1, (uint16_t)(o1 | ((vb & 2ull) ? 0x8000u : 0u))};
-        }
-      }
-    } else {
-      for (int k = 2; k >= 0; --k) {
-        uint32_t adj = face.adj[k];
-        A.stack[sp++] = SilE{(uint16_t)adj, (uint16_t)next_ccw(A.faces[adj], face.pts[k])};
-      }
-      while (sp > 0) {
-        SilE e = A.stack[--sp];
-        FaceD& fa = A.faces[e.face];
-        if (fa.deleted) continue;
-        if (!can_be_seen(A, fa, sp_id, e.opp)) {
-          if (ns >= A.scap) return EPA_OVERFLOW;
-          A.sil[ns++] = e;
-        } else {
-          fa.deleted = 1;
-          uint32_t i1 = (e.opp + 2) % 3, i2 = e.opp;
-          uint32_t adj1 = fa.adj[i1], adj2 = fa.adj[i2];
-          uint32_t o1 = next_ccw(A.faces[adj1], fa.pts[i1]);
-          uint32_t o2 = next_ccw(A.faces[adj2], fa.pts[i2]);
-          if (sp + 2 > A.stcap) return EPA_OVERFLOW;
-          A.stack[sp++] = SilE{(uint16_t)adj2, (uint16_t)o2};
-          A.stack[sp++] = SilE{(uint16_t)adj1, (uint16_t)o1};
-        }
+        A.stack[sp++] = SilE{(uint16_t)adj2, (uint16_t)(o2 | ((vb & 1ull) ? 0x8000u : 0u))};
+        A.stack[sp++] = SilE{(uint16_t)adj1, (uint16_t)(o1 | ((vb & 2ull) ? 0x8000u : 0u))};
       }
     }
     uint32_t first_new = nf;
     if (ns == 0) return EPA_NONE;
-    if constexpr (PAR != 0) {
-      // The new faces are made in parallel, silhouette edge q by lane q mod G of the group, and
-      // then checked and pushed in edge order as the loop below does.  Which edges get a face
-      // (their silhouette face still live), and so every new face's id, is known before any face
-      // is made: making faces only appends faces and rewrites adjacency slots, never the deleted
-      // flags or vertex ids read here.  Each edge's results go to its silhouette entry (bit 14:
-      // has a face, bit 15: origin projects inside) and to the emptied search stack (the
-      // distance).  Lanes of one wavefront see each other's LDS writes in order; a device-memory
-      // arena (PAR 2) fences at workgroup scope before the edges' results are read back.
-      const int lane = __lane_id();
-      const uint64_t gmask = G == 64 ? ~0ull : (((1ull << (G & 63)) - 1ull) << (lane & ~(G - 1)));
-      const uint64_t below = (1ull << lane) - 1ull;
-      float* sdist = (float*)A.stack;
-      uint32_t nvalid = 0;
-      for (uint32_t base = 0; base < ns; base += G) {
-        const uint32_t q = base + (uint32_t)gl;
-        SilE edge = SilE{0, 0};
-        bool valid = false;
-        if (q < ns) {
-          edge = A.sil[q];
-          valid = !A.faces[edge.face].deleted;
-        }
-        const uint64_t vm = __ballot(valid) & gmask;
-        const uint32_t new_id = nf + nvalid + (uint32_t)__popcll(vm & below);
-        __builtin_amdgcn_wave_barrier();
-        if (valid && new_id < A.fcap) {
-          const uint32_t pt1 = A.faces[edge.face].pts[(edge.opp + 2) % 3];
-          const uint32_t pt2 = A.faces[edge.face].pts[(edge.opp + 1) % 3];
-          FaceD nfc;
-          f3 nfn;
-          const bool inside = make_face(A, pt1, pt2, sp_id, edge.face, new_id + 1, new_id - 1, nfc, nfn);
-          A.faces[edge.face].adj[(edge.opp + 1) % 3] = (uint16_t)new_id;
-          A.faces[new_id] = nfc;
-          sdist[q] = inside ? dot(nfn, vpt(A, pt1)) : 0.f;
-          A.sil[q].opp = (uint16_t)(edge.opp | 0x4000u | (inside ? 0x8000u : 0u));
-        }
-        nvalid += (uint32_t)__popcll(vm);
+    // The new faces are made in parallel, silhouette edge q by lane q mod G of the group, and
+    // then checked and pushed in edge order as the loop below does.  Which edges get a face
+    // (their silhouette face still live), and so every new face's id, is known before any face
+    // is made: making faces only appends faces and rewrites adjacency slots, never the deleted
+    // flags or vertex ids read here.  Each edge's results go to its silhouette entry (bit 14:
+    // has a face, bit 15: origin projects inside) and to the emptied search stack (the
+    // distance), fenced at workgroup scope before they are read back.
+    const uint64_t gmask = G == 64 ? ~0ull : (((1ull << (G & 63)) - 1ull) << (lane & ~(G - 1)));
+    const uint64_t below = (1ull << lane) - 1ull;
+    float* sdist = (float*)A.stack;
+    uint32_t nvalid = 0;
+    for (uint32_t base = 0; base < ns; base += G) {
+      const uint32_t q = base + (uint32_t)gl;
+      SilE edge = SilE{0, 0};
+      bool valid = false;
+      if (q < ns) {
+        edge = A.sil[q];
+        valid = !A.faces[edge.face].deleted;
       }
+      const uint64_t vm = __ballot(valid) & gmask;
+      const uint32_t new_id = nf + nvalid + (uint32_t)__popcll(vm & below);
       __builtin_amdgcn_wave_barrier();
-      if constexpr (PAR == 2) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-      if (nf + nvalid > A.fcap) return EPA_OVERFLOW;
-      for (uint32_t q = 0; q < ns; ++q) {
-        const uint32_t fl = A.sil[q].opp;
-        if (!(fl & 0x4000u)) continue;
-        const uint32_t new_id = nf++;
-        if (fl & 0x8000u) {
-          const float dist = sdist[q];
-          if (dist < curr_dist) {
-            face_points(A, face, p1, p2);
-            n = face_n;
-            return EPA_OK;
-          }
-          if (-dist > gjk_tol) return EPA_NONE;
-          A.heap[hl] = HeapE{-dist, new_id};
-          heap_sift_up_par<G, PAR == 2>(A.heap, hl, gl);
-          hl++;
-        }
+      if (valid && new_id < A.fcap) {
+        const uint32_t pt1 = A.faces[edge.face].pts[(edge.opp + 2) % 3];
+        const uint32_t pt2 = A.faces[edge.face].pts[(edge.opp + 1) % 3];
+        FaceD nfc;
+        f3 nfn;
+        const bool inside = make_face(A, pt1, pt2, sp_id, edge.face, new_id + 1, new_id - 1, nfc, nfn);
+        A.faces[edge.face].adj[(edge.opp + 1) % 3] = (uint16_t)new_id;
+        A.faces[new_id] = nfc;
+        sdist[q] = inside ? dot(nfn, vpt(A, pt1)) : 0.f;
+        A.sil[q].opp = (uint16_t)(edge.opp | 0x4000u | (inside ? 0x8000u : 0u));
       }
-    } else {
-      for (uint32_t q = 0; q < ns; ++q) {
-        SilE edge = A.sil[q];
-        if (!A.faces[edge.face].deleted) {
-          if (nf >= A.fcap || hl >= A.fcap) return EPA_OVERFLOW;
-          uint32_t new_id = nf;
-          uint32_t pt1 = A.faces[edge.face].pts[(edge.opp + 2) % 3];
-          uint32_t pt2 = A.faces[edge.face].pts[(edge.opp + 1) % 3];
-          FaceD nfc;
-          f3 nfn;
-          bool inside = make_face(A, pt1, pt2, sp_id, edge.face, new_id + 1, new_id - 1, nfc, nfn);
-          A.faces[edge.face].adj[(edge.opp + 1) % 3] = (uint16_t)new_id;
-          A.faces[nf++] = nfc;
-          if (inside) {
-            float dist = dot(nfn, vpt(A, nfc.pts[0]));
-            if (dist < curr_dist) {
-              face_points(A, face, p1, p2);
-              n = face_n;
-              return EPA_OK;
-            }
-            if (-dist > gjk_tol) return EPA_NONE;
-            A.heap[hl] = HeapE{-dist, new_id};
-            heap_sift_up(A.heap, hl);
-            hl++;
-          }
+      nvalid += (uint32_t)__popcll(vm);
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    if (nf + nvalid > A.fcap) return EPA_OVERFLOW;
+    for (uint32_t q = 0; q < ns; ++q) {
+      const uint32_t fl = A.sil[q].opp;
+      if (!(fl & 0x4000u)) continue;
+      const uint32_t new_id = nf++;
+      if (fl & 0x8000u) {
+        const float dist = sdist[q];
+        if (dist < curr_dist) {
+          face_points(A, face, p1, p2);
+          n = face_n;
+          return EPA_OK;
         }
+        if (-dist > gjk_tol) return EPA_NONE;
+        A.heap[hl] = HeapE{-dist, new_id};
+        heap_sift_up_par<G>(A.heap, hl, gl);
+        hl++;
       }
     }
     if (first_new == nf) return EPA_NONE;
@@ -574,7 +468,7 @@ __device__ __forceinline__ int epa(const Ctx2& c, const Simplex& s, const Pool& 
 
 // ------------------------------------------------------------------ per-pair queries
 struct PairOut {
-  int has;  // 1 = Some(contact); 0 = None; 2 = arena overflow (re-run); 3 = warm-start cap; 4 = suspended (listed)
+  int has;  // 1 = Some(contact); 0 = None; 3 = warm-start cap; 5 = the pair needs EPA
   f3 w1, w2, n;
   float depth;
   int gjk_iters;
@@ -585,46 +479,27 @@ struct PairOut {
   f3 fdir;
 };
 
-// contact_support_map_support_map_with_params (contact_support_map_support_map.rs:38-88)
-template <int G, int PAR>
-__device__ __forceinline__ PairOut contact_sm(const Ctx2& c, float prediction, bool has_init, f3 init_dir, const Pool& P,
-                              int gl, const Arena& A, int max_iter, const EpaIO& io) {
-  PairOut o;
+__device__ __forceinline__ void pair_none(PairOut& o) {
+  const f3 z = f3{0.f, 0.f, 0.f};
   o.has = 0;
+  o.w1 = o.w2 = o.n = o.fdir = z;
+  o.depth = 0.f;
   o.gjk_iters = 0;
-  o.fdir = f3{0.f, 0.f, 0.f};
-  f3 dir;
-  if (has_init) dir = init_dir;
-  else {
-    float nl;
-    if (!try_normalize(c.m2.t - c.m1.t, NCX_FLT_EPS, &dir, &nl)) dir = f3{1.f, 0.f, 0.f};
-  }
-  Simplex s;
-  sx_init(s);
-  sx_reset(s, cso_from<G>(c, dir, P, gl));
-  GJKOut r = gjk<G>(c, prediction, s, P, gl, max_iter);
-  o.gjk_iters = r.iters;
-  if (r.status == GJK_S_CAP && max_iter < 10000) {
-    o.has = 3;  // iteration cap of a warm-started run: the caller re-runs plain GJK
-    return o;
-  }
-  f3 w1, w2, n;
-  if (r.status == GJK_S_CLOSEST) { w1 = r.p1; w2 = r.p2; n = r.dir; }
-  else if (r.status == GJK_S_INTERSECTION) {
-    int it;
-    int e = epa<G, PAR>(c, s, P, gl, A, w1, w2, n, it, io);
-    if (e == EPA_OVERFLOW) { o.has = 2; return o; }
-    if (e == EPA_SUSPENDED) { o.has = 4; return o; }
-    if (e != EPA_OK) { o.fdir = f3{1.f, 0.f, 0.f}; return o; }  // NoIntersection(x_axis)
-  } else {
-    if (r.status == GJK_S_NOINTER || r.status == GJK_S_CAP) o.fdir = r.dir;
-    return o;
-  }
+}
+
+// How an EPA run's result completes its pair: contact_support_map_support_map, or the projection of
+// a ball (the first or the second shape) on the other.
+#define EPA_KIND_SM 0u
+#define EPA_KIND_BALL_FIRST 1u
+#define EPA_KIND_BALL_SECOND 2u
+
+// Contact of a support-map pair from its closest points (contact_support_map_support_map.rs:62-76,
+// Contact::new_wo_depth contact.rs:43-46).
+__device__ __forceinline__ void contact_sm_finish(PairOut& o, f3 w1, f3 w2, f3 n) {
   o.fdir = n;
   o.has = 1;
   o.w1 = w1; o.w2 = w2; o.n = n;
-  o.depth = -dot(n, w2 - w1);  // Contact::new_wo_depth (contact.rs:43-46)
-  return o;
+  o.depth = -dot(n, w2 - w1);
 }
 
 // AABB::local_point_projection + project_point_with_feature for a cuboid (point_aabb.rs:9-135), solid = false.
@@ -686,64 +561,26 @@ __device__ __forceinline__ f3 cuboid_feature_normal(int fkind, int fid) {
   return normalize(d);
 }
 
-// contact_ball_convex_polyhedron (contact_ball_convex_polyhedron.rs:11-58), Cuboid or ConvexHull.
-template <int G, int PAR>
-__device__ __forceinline__ PairOut contact_ball_convex(f3 c1, float r, const iso& m2, const ShapeD& g2, float prediction,
-                                       const Pool& P, int gl, const Arena& A, const EpaIO& io) {
-  PairOut o;
-  o.has = 0;
-  o.gjk_iters = 0;
-  o.fdir = f3{0.f, 0.f, 0.f};
-  bool inside;
-  int fkind = 3, fid = 0;
-  f3 world2;
-  f3 tri_n = f3{0.f, 1.f, 0.f};  // Triangle::feature_normal: its normal, or +y when degenerate
-  if (g2.type == NCX_CUBOID) {
-    world2 = project_cuboid(m2, f3{g2.a, g2.b, g2.c}, c1, inside, fkind, fid);
-  } else if (g2.type == SHAPE_SEGMENT) {
-    // a capsule's segment in the contact-manifold generators: Segment::project_point_with_feature
-    world2 = proj_segment_at(m2, f3{0.f, -g2.a, 0.f}, f3{0.f, g2.a, 0.f}, c1, fkind, fid, inside);
-  } else if (g2.type == SHAPE_TRIANGLE) {
-    // Triangle::project_point_with_feature, solid in 3D (src/query/point/point_triangle.rs:29-51);
-    // every location names a feature, so the zero-distance branch below always has a normal
-    f3 a, b, c;
-    tri_vertices(P, g2.off, a, b, c);
-    Loc loc;
-    world2 = proj_triangle_at(m2, a, b, c, c1, loc, inside);
-    fkind = 0;
-    f3 nn;
-    float nl;
-    if (try_normalize(cross(b - a, c - a), NCX_FLT_EPS, &nn, &nl)) tri_n = nn;  // triangle.rs:137-139, 367-374
-  } else {
-    // point_projection_on_support_map (point_support_map.rs:15-53), solid = false
-    Ctx2 c;
-    c.m1 = m2;
-    c.m1.t = (-c1) + m2.t;
-    c.g1 = g2;
-    c.m2 = iso_identity();
-    c.g2.type = SHAPE_ORIGIN;
-    f3 dir;
-    float nl;
-    if (!try_normalize(-c.m1.t, NCX_FLT_EPS, &dir, &nl)) dir = f3{1.f, 0.f, 0.f};
-    Simplex s;
-    sx_init(s);
-    sx_reset(s, cso_from<G>(c, dir, P, gl));
-    GJKOut r2 = gjk<G>(c, NCX_FLT_MAX, s, P, gl, 10000);
-    o.gjk_iters = r2.iters;
-    if (r2.status == GJK_S_CLOSEST) {
-      inside = false;
-      world2 = r2.p1 + c1;
-    } else {
-      f3 p1, p2, nn;
-      int it;
-      int e = r2.status == GJK_S_INTERSECTION ? epa<G, PAR>(c, s, P, gl, A, p1, p2, nn, it, io) : EPA_NONE;
-      if (e == EPA_OVERFLOW) { o.has = 2; return o; }
-      if (e == EPA_SUSPENDED) { o.has = 4; return o; }
-      inside = true;
-      world2 = e == EPA_OK ? p1 + c1 : c1;
-    }
-  }
-  f3 dpt = world2 - c1;
+// point_projection_on_support_map's two support maps (point_support_map.rs:15-53): the shape with
+// the point at the origin, and ConstantOrigin.
+__device__ __forceinline__ Ctx2 ball_projection_ctx(f3 c1, const iso& m2, const ShapeD& g2) {
+  Ctx2 c;
+  c.m1 = m2;
+  c.m1.t = (-c1) + m2.t;
+  c.g1 = g2;
+  c.m2 = iso_identity();
+  c.g2.type = SHAPE_ORIGIN;
+  c.g2.off = 0;
+  c.g2.cnt = 0;
+  c.g2.a = c.g2.b = c.g2.c = 0.f;
+  return c;
+}
+
+// The contact of a ball with the point it projects on (contact_ball_convex_polyhedron.rs:25-58).
+// no_feature: the shape has no normal to offer when the ball's centre is on its surface.
+__device__ __forceinline__ void ball_convex_finish(PairOut& o, f3 c1, float r, f3 world2, bool inside, bool no_feature,
+                                                   f3 feature_normal, float prediction) {
+  const f3 dpt = world2 - c1;
   f3 dir;
   float dist, depth;
   f3 normal;
@@ -751,17 +588,9 @@ __device__ __forceinline__ PairOut contact_ball_convex(f3 c1, float r, const iso
     if (inside) { depth = dist + r; normal = -dir; }
     else { depth = -dist + r; normal = dir; }
   } else {
-    if (g2.type == SHAPE_TRIANGLE) {
-      depth = r;
-      normal = -tri_n;
-    } else if (g2.type == SHAPE_SEGMENT) {  // a segment location always names a feature
-      depth = r;
-      normal = -segment_feature_normal(f3{0.f, -g2.a, 0.f}, f3{0.f, g2.a, 0.f}, fkind, fid);
-    } else {
-      if (g2.type != NCX_CUBOID || fkind == 3) return o;
-      depth = r;
-      normal = -cuboid_feature_normal(fkind, fid);
-    }
+    if (no_feature) return;
+    depth = r;
+    normal = -feature_normal;
   }
   if (depth >= -prediction) {
     o.has = 1;
@@ -770,27 +599,65 @@ __device__ __forceinline__ PairOut contact_ball_convex(f3 c1, float r, const iso
     o.n = normal;
     o.depth = depth;
   }
-  return o;
 }
 
-// query::contact dispatch (contact_shape_shape.rs:10-48).
-template <int G, int PAR>
-__device__ __forceinline__ PairOut contact_pair(const Ctx2& c, float prediction, bool has_init, f3 init_dir, const Pool& P,
-                                int gl, const Arena& A, int max_iter, const EpaIO& io) {
-  bool b1 = c.g1.type == NCX_BALL, b2 = c.g2.type == NCX_BALL;
+// Contact::flip (contact.rs:52-55)
+__device__ __forceinline__ void contact_flip(PairOut& o, bool flip) {
+  const f3 a = o.w1, b = o.w2;
+  o.w1 = sel3(flip, b, a);
+  o.w2 = sel3(flip, a, b);
+  o.n = sel3(flip, -o.n, o.n);
+}
+
+// contact_ball_convex_polyhedron (contact_ball_convex_polyhedron.rs:11-58) on a Cuboid, Triangle or
+// Segment, whose point projections are closed forms.
+__device__ __forceinline__ void contact_ball_closed(PairOut& o, f3 c1, float r, const iso& m2, const ShapeD& g2,
+                                                    float prediction, const Pool& P) {
+  bool inside;
+  int fkind = 3, fid = 0;
+  f3 world2, fn;
+  bool no_feature = false;
+  if (g2.type == NCX_CUBOID) {
+    world2 = project_cuboid(m2, f3{g2.a, g2.b, g2.c}, c1, inside, fkind, fid);
+    no_feature = fkind == 3;
+    fn = cuboid_feature_normal(fkind, fid);
+  } else if (g2.type == SHAPE_SEGMENT) {
+    // a capsule's segment in the contact-manifold generators: Segment::project_point_with_feature
+    const f3 a = f3{0.f, -g2.a, 0.f}, b = f3{0.f, g2.a, 0.f};
+    world2 = proj_segment_at(m2, a, b, c1, fkind, fid, inside);
+    fn = segment_feature_normal(a, b, fkind, fid);
+  } else {
+    // Triangle::project_point_with_feature, solid in 3D (src/query/point/point_triangle.rs:29-51);
+    // Triangle::feature_normal: its normal, or +y when degenerate (triangle.rs:137-139, 367-374)
+    f3 a, b, c;
+    tri_vertices(P, g2.off, a, b, c);
+    Loc loc;
+    world2 = proj_triangle_at(m2, a, b, c, c1, loc, inside);
+    float nl;
+    if (!try_normalize(cross(b - a, c - a), NCX_FLT_EPS, &fn, &nl)) fn = f3{0.f, 1.f, 0.f};
+  }
+  ball_convex_finish(o, c1, r, world2, inside, no_feature, fn, prediction);
+}
+
+// query::contact dispatch (contact_shape_shape.rs:10-48).  GJK runs at one place for every path:
+// contact_support_map_support_map_with_params (contact_support_map_support_map.rs:38-88) and a
+// ball's projection on a hull (point_support_map.rs:15-53).  has = 5: the pair intersects; s and
+// kind are EPA's input.
+template <int G>
+__device__ __forceinline__ PairOut contact_pair(const Ctx2& c, float prediction, bool has_init, f3 init_dir,
+                                                const Pool& P, int gl, int max_iter, Simplex& s, uint32_t& kind) {
+  const bool b1 = c.g1.type == NCX_BALL, b2 = c.g2.type == NCX_BALL;
   // ConvexPolyhedron shapes: a ball against one takes the point-projection path (a capsule's
   // segment appears only in the contact-manifold generators, where the ball-polyhedron
   // generator handles it the same way)
-  bool poly1 = c.g1.type == NCX_CUBOID || c.g1.type == NCX_CONVEX_HULL || c.g1.type == SHAPE_TRIANGLE ||
-               c.g1.type == SHAPE_SEGMENT;
-  bool poly2 = c.g2.type == NCX_CUBOID || c.g2.type == NCX_CONVEX_HULL || c.g2.type == SHAPE_TRIANGLE ||
-               c.g2.type == SHAPE_SEGMENT;
+  const bool poly1 = c.g1.type == NCX_CUBOID || c.g1.type == NCX_CONVEX_HULL || c.g1.type == SHAPE_TRIANGLE ||
+                     c.g1.type == SHAPE_SEGMENT;
+  const bool poly2 = c.g2.type == NCX_CUBOID || c.g2.type == NCX_CONVEX_HULL || c.g2.type == SHAPE_TRIANGLE ||
+                     c.g2.type == SHAPE_SEGMENT;
+  PairOut o;
+  pair_none(o);
   if (b1 && b2) {
     // contact_ball_ball (contact_ball_ball.rs:8-38)
-    PairOut o;
-    o.has = 0;
-    o.gjk_iters = 0;
-    o.fdir = f3{0.f, 0.f, 0.f};
     float r1 = c.g1.a, r2 = c.g2.a;
     f3 delta = c.m2.t - c.m1.t;
     float d2 = norm_sq(delta);
@@ -805,14 +672,42 @@ __device__ __forceinline__ PairOut contact_pair(const Ctx2& c, float prediction,
     }
     return o;
   }
-  if (b1 && poly2) return contact_ball_convex<G, PAR>(c.m1.t, c.g1.a, c.m2, c.g2, prediction, P, gl, A, io);
-  if (poly1 && b2) {
-    PairOut o = contact_ball_convex<G, PAR>(c.m2.t, c.g2.a, c.m1, c.g1, prediction, P, gl, A, io);
-    if (o.has == 1) {  // Contact::flip (contact.rs:52-55)
-      f3 t = o.w1; o.w1 = o.w2; o.w2 = t;
-      o.n = -o.n;
-    }
+  kind = b1 && poly2 ? EPA_KIND_BALL_FIRST : (poly1 && b2 ? EPA_KIND_BALL_SECOND : EPA_KIND_SM);
+  const bool swapped = kind == EPA_KIND_BALL_SECOND;
+  const f3 c1 = swapped ? c.m2.t : c.m1.t;  // the ball, where one is projected
+  const float r = swapped ? c.g2.a : c.g1.a;
+  if (kind != EPA_KIND_SM && (swapped ? c.g1.type : c.g2.type) != NCX_CONVEX_HULL) {
+    contact_ball_closed(o, c1, r, swapped ? c.m1 : c.m2, swapped ? c.g1 : c.g2, prediction, P);
+    contact_flip(o, swapped);
     return o;
   }
-  return contact_sm<G, PAR>(c, prediction, has_init, init_dir, P, gl, A, max_iter, io);
+  Ctx2 cc = c;
+  f3 dir;
+  float max_dist = prediction;
+  bool found;
+  float nl;
+  if (kind == EPA_KIND_SM) {
+    dir = init_dir;
+    found = has_init || try_normalize(c.m2.t - c.m1.t, NCX_FLT_EPS, &dir, &nl);
+  } else {
+    cc = ball_projection_ctx(c1, swapped ? c.m1 : c.m2, swapped ? c.g1 : c.g2);
+    found = try_normalize(-cc.m1.t, NCX_FLT_EPS, &dir, &nl);
+    max_dist = NCX_FLT_MAX;
+    max_iter = 10000;
+  }
+  if (!found) dir = f3{1.f, 0.f, 0.f};
+  const GJKOut g = gjk<G, true>(cc, dir, max_dist, s, P, gl, max_iter);
+  o.gjk_iters = g.iters;
+  if (g.status == GJK_S_INTERSECTION) {
+    o.has = 5;
+  } else if (kind == EPA_KIND_SM) {
+    if (g.status == GJK_S_CAP && max_iter < 10000) o.has = 3;  // a warm-started run's cap: the caller re-runs plain GJK
+    else if (g.status == GJK_S_CLOSEST) contact_sm_finish(o, g.p1, g.p2, g.dir);
+    else if (g.status == GJK_S_NOINTER || g.status == GJK_S_CAP) o.fdir = g.dir;
+  } else {
+    const bool inside = g.status != GJK_S_CLOSEST;
+    ball_convex_finish(o, c1, r, inside ? c1 : g.p1 + c1, inside, true, f3{0.f, 0.f, 0.f}, prediction);
+    contact_flip(o, swapped);
+  }
+  return o;
 }

@@ -61,19 +61,44 @@ __device__ __forceinline__ void tri_vertices(const Pool& P, uint32_t k, f3& a, f
   c = f3{C.x, C.y, C.z};
 }
 
+// The value of another lane for a reduction step over 2 O lanes whose O-lane halves hold equal
+// values already: lane ^ O for O = 1, 2; within 8 or 16 lanes the mirrored lane serves as well.
+// These are DPP moves (a few cycles); __shfl_xor goes through the LDS crossbar, whose latency the
+// support scans would pay up to four times per call.
+template <int O> __device__ __forceinline__ uint32_t lane_across(uint32_t v) {
+  if constexpr (O == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);        // quad_perm 1,0,3,2
+  else if constexpr (O == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);   // quad_perm 2,3,0,1
+  else if constexpr (O == 4) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true);  // row_half_mirror
+  else if constexpr (O == 8) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, true);  // row_mirror
+  else return (uint32_t)__shfl_xor((int)v, O, 64);
+}
+
+#define HULL_NONE 0xFFFFFFFFu
+// The lane reduction of a hull scan: the larger value and, on ties, the lower index.
+template <int G, int O = 1> __device__ __forceinline__ void hull_best(float& best, uint32_t& bi) {
+  if constexpr (O < G) {
+    const float ob = __uint_as_float(lane_across<O>(__float_as_uint(best)));
+    const uint32_t oi = lane_across<O>(bi);
+    if (oi != HULL_NONE && (bi == HULL_NONE || ob > best || (ob == best && oi < bi))) {
+      best = ob;
+      bi = oi;
+    }
+    hull_best<G, 2 * O>(best, bi);
+  }
+}
+
 // point_cloud_support_point_id (src/utils/point_cloud_support_point.rs:6-24), split over G lanes.
 // The reference keeps index 0 when dot(p_0, dir) is NaN and otherwise returns the first index of
 // the maximum over the non-NaN dots (NaN never compares greater).  Each lane scans vertices
 // gl, gl + G, ... in increasing order keeping its first maximum over non-NaN dots; the lane
-// reduction keeps the larger value and, on ties, the lower index.  U vertices' loads are issued
-// together so their latencies overlap.
+// reduction keeps the larger value and, on ties, the lower index (vertex 0 with a NaN dot enters
+// it as infinity).  U vertices' loads are issued together so their latencies overlap.
 template <int G>
 __device__ __forceinline__ uint32_t hull_support_id(const Pool& P, uint32_t off, uint32_t cnt, f3 dir, int gl) {
   constexpr int U = 4;
-  constexpr uint32_t NONE = 0xFFFFFFFFu;
   float best = 0.f;
-  uint32_t bi = NONE;
-  int nan0 = 0;
+  uint32_t bi = HULL_NONE;
+  bool nan0 = false;
   for (uint32_t v0 = gl; v0 < cnt; v0 += U * G) {
     float px[U], py[U], pz[U];
 #pragma unroll
@@ -90,24 +115,19 @@ __device__ __forceinline__ uint32_t hull_support_id(const Pool& P, uint32_t off,
       float d = dot(f3{px[u], py[u], pz[u]}, dir);
       if (v < cnt) {
         if (v == 0) nan0 = d != d;
-        if (d > best || (bi == NONE && d == d)) {
+        if (d > best || (bi == HULL_NONE && d == d)) {
           best = d;
           bi = v;
         }
       }
     }
   }
-#pragma unroll
-  for (int o = G / 2; o >= 1; o >>= 1) {
-    float ob = __shfl_xor(best, o, 64);
-    uint32_t oi = __shfl_xor(bi, o, 64);
-    if (oi != NONE && (bi == NONE || ob > best || (ob == best && oi < bi))) {
-      best = ob;
-      bi = oi;
-    }
+  if (nan0) {
+    best = __builtin_inff();
+    bi = 0;
   }
-  nan0 = __shfl(nan0, 0, G);  // lane 0 of the group scanned vertex 0
-  return (bi == NONE || nan0) ? 0u : bi;
+  hull_best<G>(best, bi);
+  return bi == HULL_NONE ? 0u : bi;
 }
 
 // SupportMap::support_point (src/shape/support_map.rs:26-29) and the overrides of
@@ -155,8 +175,15 @@ __device__ __forceinline__ f3 support(const ShapeD& g, const iso& m, f3 dir, con
   }
 }
 
+// A point of the Minkowski difference with the two support points it came from.
 struct CSO {
+  f3 o1, o2;
+  __device__ __forceinline__ f3 pt() const { return o1 - o2; }
+};
+// The same with the point kept apart: the ray cast moves it and leaves the support points.
+struct CSOR {
   f3 p, o1, o2;
+  __device__ __forceinline__ f3 pt() const { return p; }
 };
 
 struct Ctx2 {
@@ -169,7 +196,6 @@ __device__ __forceinline__ CSO cso_from(const Ctx2& c, f3 dir, const Pool& P, in
   CSO r;
   r.o1 = support<G>(c.g1, c.m1, dir, P, gl);
   r.o2 = support<G>(c.g2, c.m2, -dir, P, gl);
-  r.p = r.o1 - r.o2;
   return r;
 }
 
@@ -319,29 +345,34 @@ __device__ __forceinline__ f3 proj_tetrahedron(f3 A, f3 B, f3 C, f3 D, Loc& loc)
 // The four vertices are separate members and the "previous vertex" permutation is
 // packed 2 bits per slot, so no runtime index reaches an array: everything stays in
 // registers.
-struct Simplex {
-  CSO v0, v1, v2, v3;
+template <class V> struct SimplexT {
+  V v0, v1, v2, v3;
   uint32_t pv;  // prev_vertices, slot i in bits [2i, 2i+2)
   float proj0, proj1, proj2, pproj0, pproj1, pproj2;
   int dim, pdim;
 };
+typedef SimplexT<CSO> Simplex;
+typedef SimplexT<CSOR> SimplexR;
 
 // Value selects (never a select between addresses), so the simplex stays in registers.
 __device__ __forceinline__ f3 sel3(bool c, f3 a, f3 b) { return f3{c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z}; }
 __device__ __forceinline__ CSO csel(bool c, const CSO& a, const CSO& b) {
-  return CSO{sel3(c, a.p, b.p), sel3(c, a.o1, b.o1), sel3(c, a.o2, b.o2)};
+  return CSO{sel3(c, a.o1, b.o1), sel3(c, a.o2, b.o2)};
 }
-__device__ __forceinline__ CSO sx_get(const Simplex& s, int i) {
+__device__ __forceinline__ CSOR csel(bool c, const CSOR& a, const CSOR& b) {
+  return CSOR{sel3(c, a.p, b.p), sel3(c, a.o1, b.o1), sel3(c, a.o2, b.o2)};
+}
+template <class V> __device__ __forceinline__ V sx_get(const SimplexT<V>& s, int i) {
   return csel(i == 0, s.v0, csel(i == 1, s.v1, csel(i == 2, s.v2, s.v3)));
 }
-__device__ __forceinline__ void sx_set(Simplex& s, int i, const CSO& c) {
+template <class V> __device__ __forceinline__ void sx_set(SimplexT<V>& s, int i, const V& c) {
   s.v0 = csel(i == 0, c, s.v0);
   s.v1 = csel(i == 1, c, s.v1);
   s.v2 = csel(i == 2, c, s.v2);
   s.v3 = csel(i == 3, c, s.v3);
 }
-__device__ __forceinline__ void sx_swap(Simplex& s, int i, int j) {
-  CSO a = sx_get(s, i), b = sx_get(s, j);
+template <class V> __device__ __forceinline__ void sx_swap(SimplexT<V>& s, int i, int j) {
+  V a = sx_get(s, i), b = sx_get(s, j);
   sx_set(s, i, b);
   sx_set(s, j, a);
   uint32_t pi = (s.pv >> (2 * i)) & 3u, pj = (s.pv >> (2 * j)) & 3u;
@@ -351,7 +382,7 @@ __device__ __forceinline__ void sx_swap(Simplex& s, int i, int j) {
 
 #define PV_IDENTITY 0xE4u  // slots (0, 1, 2, 3)
 
-__device__ __forceinline__ void sx_init(Simplex& s) {
+template <class V> __device__ __forceinline__ void sx_init(SimplexT<V>& s) {
   s.pv = PV_IDENTITY;
   s.proj0 = s.proj1 = s.proj2 = 0.f;
   s.pproj0 = s.pproj1 = s.pproj2 = 0.f;
@@ -359,24 +390,24 @@ __device__ __forceinline__ void sx_init(Simplex& s) {
   s.pdim = 0;
 }
 
-__device__ __forceinline__ void sx_reset(Simplex& s, const CSO& p) {
+template <class V> __device__ __forceinline__ void sx_reset(SimplexT<V>& s, const V& p) {
   s.dim = 0;
   s.pdim = 0;
   s.v0 = p;
 }
 
-__device__ __forceinline__ bool sx_add(Simplex& s, const CSO& pt) {
+template <class V> __device__ __forceinline__ bool sx_add(SimplexT<V>& s, const V& pt) {
   const float tol = NCX_FLT_EPS * 10.f;
   s.pdim = s.dim;
   s.pproj0 = s.proj0; s.pproj1 = s.proj1; s.pproj2 = s.proj2;
   s.pv = PV_IDENTITY;
   if (s.dim == 0) {
-    if (norm_sq(s.v0.p - pt.p) < tol) return false;
+    if (norm_sq(s.v0.pt() - pt.pt()) < tol) return false;
   } else if (s.dim == 1) {
-    f3 ab = s.v1.p - s.v0.p, ac = pt.p - s.v0.p;
+    f3 ab = s.v1.pt() - s.v0.pt(), ac = pt.pt() - s.v0.pt();
     if (norm_sq(cross(ab, ac)) < tol) return false;
   } else {
-    f3 ab = s.v1.p - s.v0.p, ac = s.v2.p - s.v0.p, ap = pt.p - s.v0.p;
+    f3 ab = s.v1.pt() - s.v0.pt(), ac = s.v2.pt() - s.v0.pt(), ap = pt.pt() - s.v0.pt();
     f3 n = normalize(cross(ab, ac));
     if (fabsf(dot(n, ap)) < tol) return false;
   }
@@ -385,20 +416,20 @@ __device__ __forceinline__ bool sx_add(Simplex& s, const CSO& pt) {
   return true;
 }
 
-__device__ __forceinline__ f3 sx_project_reduce(Simplex& s) {
+template <class V> __device__ __forceinline__ f3 sx_project_reduce(SimplexT<V>& s) {
   if (s.dim == 0) {
     s.proj0 = 1.f;
-    return s.v0.p;
+    return s.v0.pt();
   } else if (s.dim == 1) {
     Loc loc;
-    f3 pr = proj_segment(s.v0.p, s.v1.p, loc);
+    f3 pr = proj_segment(s.v0.pt(), s.v1.pt(), loc);
     if (loc.kind == LOC_VERTEX && loc.id == 0) { s.proj0 = 1.f; s.dim = 0; }
     else if (loc.kind == LOC_VERTEX) { sx_swap(s, 0, 1); s.proj0 = 1.f; s.dim = 0; }
     else { s.proj0 = loc.bc0; s.proj1 = loc.bc1; }
     return pr;
   } else if (s.dim == 2) {
     Loc loc;
-    f3 pr = proj_triangle(s.v0.p, s.v1.p, s.v2.p, loc);
+    f3 pr = proj_triangle(s.v0.pt(), s.v1.pt(), s.v2.pt(), loc);
     if (loc.kind == LOC_VERTEX) { sx_swap(s, 0, loc.id); s.proj0 = 1.f; s.dim = 0; }
     else if (loc.kind == LOC_EDGE) {
       if (loc.id == 0) { s.proj0 = loc.bc0; s.proj1 = loc.bc1; }
@@ -411,7 +442,7 @@ __device__ __forceinline__ f3 sx_project_reduce(Simplex& s) {
     return pr;
   } else {
     Loc loc;
-    f3 pr = proj_tetrahedron(s.v0.p, s.v1.p, s.v2.p, s.v3.p, loc);
+    f3 pr = proj_tetrahedron(s.v0.pt(), s.v1.pt(), s.v2.pt(), s.v3.pt(), loc);
     if (loc.kind == LOC_VERTEX) { sx_swap(s, 0, loc.id); s.proj0 = 1.f; s.dim = 0; }
     else if (loc.kind == LOC_EDGE) {
       switch (loc.id) {
@@ -443,7 +474,7 @@ __device__ __forceinline__ f3 sx_project_reduce(Simplex& s) {
 }
 
 // gjk.rs:367-388
-__device__ __forceinline__ void gjk_result(const Simplex& s, bool prev, f3& p1, f3& p2) {
+template <class V> __device__ __forceinline__ void gjk_result(const SimplexT<V>& s, bool prev, f3& p1, f3& p2) {
   f3 r1 = f3{0.f, 0.f, 0.f}, r2 = f3{0.f, 0.f, 0.f};
   const int n = prev ? s.pdim : s.dim;
 #pragma unroll
@@ -451,7 +482,7 @@ __device__ __forceinline__ void gjk_result(const Simplex& s, bool prev, f3& p1, 
     if (i <= n) {
       float c = prev ? (i == 0 ? s.pproj0 : (i == 1 ? s.pproj1 : s.pproj2))
                      : (i == 0 ? s.proj0 : (i == 1 ? s.proj1 : s.proj2));
-      CSO pt = sx_get(s, prev ? (int)((s.pv >> (2 * i)) & 3u) : i);
+      const V pt = sx_get(s, prev ? (int)((s.pv >> (2 * i)) & 3u) : i);
       r1 = r1 + pt.o1 * c;
       r2 = r2 + pt.o2 * c;
     }
@@ -466,31 +497,83 @@ struct GJKOut {
   int iters;
 };
 
-// gjk::closest_points (gjk.rs:76-177), exact_dist = true.
-template <int G>
-__device__ __forceinline__ GJKOut gjk(const Ctx2& c, float max_dist, Simplex& s, const Pool& P, int gl, int max_iter) {
+// gjk::closest_points (gjk.rs:76-177), exact_dist = true, from the simplex of the support point
+// along dir.  The first point, the loop's points and (FOR_EPA) an intersecting segment's third
+// point (epa3.rs:294-305) are taken by one support call in the loop, so a kernel holds the support
+// functions of every shape once; with a call each, the contact kernel's GJK spilled 103 registers
+// more.
+template <int G, bool FOR_EPA = false>
+__device__ __forceinline__ GJKOut gjk(const Ctx2& c, f3 dir, float max_dist, Simplex& s, const Pool& P, int gl,
+                                      int max_iter) {
   GJKOut r;
   r.iters = 0;
   const float eps_tol = NCX_FLT_EPS * 10.f;
   const float eps_rel = __builtin_sqrtf(eps_tol);
-  f3 proj = sx_project_reduce(s);
-  f3 old_dir;
-  {
-    f3 pd;
-    float nl;
-    if (try_normalize(proj, 0.f, &pd, &nl)) old_dir = -pd;
-    else { r.status = GJK_S_INTERSECTION; return r; }
-  }
+  sx_init(s);
+  f3 old_dir = f3{0.f, 0.f, 0.f};
   float max_bound = NCX_FLT_MAX;
-  f3 dir;
-  int niter = 0;
+  int niter = -1;  // -1: the first point; -2: a segment's third point
   for (;;) {
-    float old_max_bound = max_bound;
-    {
-      f3 nd;
-      float dist;
-      if (try_normalize(-proj, eps_tol, &nd, &dist)) { dir = nd; max_bound = dist; }
-      else { r.status = GJK_S_INTERSECTION; return r; }
+    const CSO cso = cso_from<G>(c, dir, P, gl);
+    f3 proj;
+    if (FOR_EPA && niter == -2) {
+      s.v2 = cso;
+      s.dim = 2;
+      r.status = GJK_S_INTERSECTION;
+      return r;
+    }
+    bool meets = false;
+    if (niter < 0) {
+      sx_reset(s, cso);
+      proj = sx_project_reduce(s);
+      f3 pd;
+      float nl;
+      if (try_normalize(proj, 0.f, &pd, &nl)) old_dir = -pd;
+      else meets = true;
+    } else {
+      r.iters += 1;
+      const float min_bound = -dot(dir, cso.pt());
+      if (!(min_bound == min_bound)) { r.status = GJK_S_NAN; return r; }
+      if (min_bound > max_dist) { r.dir = dir; r.status = GJK_S_NOINTER; return r; }
+      if (max_bound - min_bound <= eps_rel * max_bound || !sx_add(s, cso)) {
+        gjk_result(s, false, r.p1, r.p2);
+        r.dir = dir;
+        r.status = GJK_S_CLOSEST;
+        return r;
+      }
+      old_dir = dir;
+      proj = sx_project_reduce(s);
+      if (s.dim == 3) {
+        if (min_bound >= eps_tol) {
+          gjk_result(s, true, r.p1, r.p2);
+          r.dir = old_dir;
+          r.status = GJK_S_CLOSEST;
+          return r;
+        }
+        r.status = GJK_S_INTERSECTION;
+        return r;
+      }
+    }
+    niter += 1;
+    if (niter > 0 && niter == max_iter) { r.dir = f3{1.f, 0.f, 0.f}; r.status = GJK_S_CAP; return r; }
+    const float old_max_bound = max_bound;
+    f3 nd;
+    float dist;
+    if (!meets && try_normalize(-proj, eps_tol, &nd, &dist)) {
+      dir = nd;
+      max_bound = dist;
+    } else {
+      if (FOR_EPA && s.dim == 1) {
+        const f3 dpt = s.v1.pt() - s.v0.pt();
+        // nalgebra orthonormal_subspace_basis for one vector; epa3.rs:299-305 keeps a x dpt.
+        f3 a = fabsf(dpt.x) > fabsf(dpt.y) ? f3{dpt.z, 0.f, -dpt.x} : f3{0.f, -dpt.z, dpt.y};
+        a = normalize(a);
+        dir = cross(a, dpt);
+        niter = -2;
+        continue;
+      }
+      r.status = GJK_S_INTERSECTION;
+      return r;
     }
     if (max_bound >= old_max_bound) {
       gjk_result(s, true, r.p1, r.p2);
@@ -498,37 +581,6 @@ __device__ __forceinline__ GJKOut gjk(const Ctx2& c, float max_dist, Simplex& s,
       r.status = GJK_S_CLOSEST;
       return r;
     }
-    CSO cso = cso_from<G>(c, dir, P, gl);
-    r.iters += 1;
-    float min_bound = -dot(dir, cso.p);
-    if (!(min_bound == min_bound)) { r.status = GJK_S_NAN; return r; }
-    if (min_bound > max_dist) { r.dir = dir; r.status = GJK_S_NOINTER; return r; }
-    else if (max_bound - min_bound <= eps_rel * max_bound) {
-      gjk_result(s, false, r.p1, r.p2);
-      r.dir = dir;
-      r.status = GJK_S_CLOSEST;
-      return r;
-    }
-    if (!sx_add(s, cso)) {
-      gjk_result(s, false, r.p1, r.p2);
-      r.dir = dir;
-      r.status = GJK_S_CLOSEST;
-      return r;
-    }
-    old_dir = dir;
-    proj = sx_project_reduce(s);
-    if (s.dim == 3) {
-      if (min_bound >= eps_tol) {
-        gjk_result(s, true, r.p1, r.p2);
-        r.dir = old_dir;
-        r.status = GJK_S_CLOSEST;
-        return r;
-      }
-      r.status = GJK_S_INTERSECTION;
-      return r;
-    }
-    niter += 1;
-    if (niter == max_iter) { r.dir = f3{1.f, 0.f, 0.f}; r.status = GJK_S_CAP; return r; }
   }
 }
 
@@ -561,8 +613,8 @@ struct RCtx {
 };
 
 template <int G>
-__device__ __forceinline__ CSO cso_from_r(const RCtx& c, f3 dir, const Pool& P, int gl) {
-  CSO r;
+__device__ __forceinline__ CSOR cso_from_r(const RCtx& c, f3 dir, const Pool& P, int gl) {
+  CSOR r;
   if (c.dilated) {
     f3 u = normalize(dir);
     r.o1 = support_toward<G>(c.g1, c.m1, u, P, gl) + u * c.dil;
@@ -587,7 +639,7 @@ __device__ __forceinline__ bool same_bits3(f3 a, f3 b) {
 // small to change the origin (its f32 sums absorb it) with a support point the simplex rejects
 // as affinely dependent is such a fixed point.
 template <int G>
-__device__ __forceinline__ bool minkowski_ray_cast(const RCtx& c, f3 ro, f3 rd, float max_toi, Simplex& s,
+__device__ __forceinline__ bool minkowski_ray_cast(const RCtx& c, f3 ro, f3 rd, float max_toi, SimplexR& s,
                                                    const Pool& P, int gl, float& toi_out, f3& normal_out) {
   const float eps_tol = NCX_FLT_EPS * 10.f;
   const float eps_rel = __builtin_sqrtf(eps_tol);
@@ -597,9 +649,9 @@ __device__ __forceinline__ bool minkowski_ray_cast(const RCtx& c, f3 ro, f3 rd, 
   f3 co = ro, cd = rd / ray_length;
   f3 dir = -cd;
   f3 ldir = dir;
-  CSO sp = cso_from_r<G>(c, dir, P, gl);
+  CSOR sp = cso_from_r<G>(c, dir, P, gl);
   {
-    CSO t0 = sp;
+    CSOR t0 = sp;
     t0.p = sp.p + (-co);
     sx_reset(s, t0);
   }
@@ -665,7 +717,7 @@ __device__ __forceinline__ bool minkowski_ray_cast(const RCtx& c, f3 ro, f3 rd, 
     if (max_bound - min_bound <= eps_rel * max_bound) return false;
     bool added;
     {
-      CSO tp = sp;
+      CSOR tp = sp;
       tp.p = sp.p + (-co);
       added = sx_add(s, tp);
     }
@@ -698,7 +750,7 @@ __device__ __forceinline__ bool ray_support_map(const ShapeD& g, f3 ro, f3 rd, f
   c.g2.type = SHAPE_ORIGIN;
   c.dil = 0.f;
   c.dilated = false;
-  Simplex s;
+  SimplexR s;
   sx_init(s);
   float t;
   f3 n;
@@ -709,7 +761,7 @@ __device__ __forceinline__ bool ray_support_map(const ShapeD& g, f3 ro, f3 rd, f
   const f3 supp = support<G>(g, c.m1, ndir, P, gl);
   const float eps = 0.001f;
   const float shift = dot(supp - ro, ndir) + eps;
-  Simplex s2;
+  SimplexR s2;
   sx_init(s2);
   if (!minkowski_ray_cast<G>(c, ro + ndir * shift, -rd, shift + eps, s2, P, gl, t, n)) return false;
   const float tt = shift - t;

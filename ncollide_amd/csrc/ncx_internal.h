@@ -69,33 +69,38 @@ struct DevBuf {
   template <class T> T* as() const { return (T*)p; }
 };
 
-// Layout of ContactTiers::ovf (uint32 words): a header, then the pair indices whose EPA outgrew
+// Layout of ContactTiers::ovf (uint32 words): a header, then the EPA records whose run outgrew
 // the first-tier arena, those that outgrew the second tier, the third, and the fourth (cap
 // entries each).
-// Header words [0, NCX_OVF_TIER_WORDS) are the tiers' counts (cleared between tuning samples),
+// Header words [0, NCX_OVF_TIER_WORDS) are the tiers' counts and the launches' numbers of EPA
+// records (cleared between tuning samples),
 // [NCX_OVF_TIER_WORDS, NCX_OVF_COUNTS) the partition's (which the samples read): each vertex-count
 // bucket's range in the partitioned list, and each sort key's count and scatter cursor.  From
-// NCX_WORK_BASE on come the work counters of the launches (the tuning samples' first tier, the
-// second, third and fourth tiers, one per bucket), each on its own cache line.
+// NCX_WORK_BASE on come the work counters of the launches (the tuning samples' GJK, the
+// second, third and fourth tiers, the samples' EPA, one GJK and one EPA per bucket), each on its
+// own cache line.
 constexpr uint32_t NCX_OVERLAP_BINS = 8;  // 4 and 16 bins ordered the scene's pairs no better
 constexpr uint32_t NCX_NKEYS = 64 * NCX_OVERLAP_BINS;  // sort keys: vertex-count bucket x 16 shape-type pairs x overlap bins
 constexpr uint32_t NCX_OVF_T1_COUNT = 0, NCX_OVF_BAD = 1, NCX_OVF_T2_COUNT = 2, NCX_OVF_T3_COUNT = 3,
-                   NCX_OVF_T4_COUNT = 4, NCX_OVF_TIER_WORDS = 8, NCX_BKT_RANGE = 8, NCX_KEY_CNT = 16,
+                   NCX_OVF_T4_COUNT = 4, NCX_REC_COUNT = 5, NCX_REC_COUNT_TUNE = 9, NCX_OVF_TIER_WORDS = 16,
+                   NCX_BKT_RANGE = 16, NCX_KEY_CNT = 24,
                    NCX_KEY_FILL = NCX_KEY_CNT + NCX_NKEYS, NCX_OVF_COUNTS = NCX_KEY_FILL + NCX_NKEYS;
 constexpr uint32_t NCX_WORK_SET = 64, NCX_WORK_BASE = NCX_OVF_COUNTS, NCX_WORK_TUNE = 0, NCX_WORK_T2 = 1, NCX_WORK_T3 = 2,
-                   NCX_WORK_T4 = 3, NCX_WORK_BKT = 4, NCX_WORK_SETS = 8,
+                   NCX_WORK_T4 = 3, NCX_WORK_TUNE_EPA = 4, NCX_WORK_BKT = 5, NCX_WORK_EPA = 9, NCX_WORK_SETS = 13,
                    NCX_OVF_HEADER = NCX_WORK_BASE + NCX_WORK_SETS * NCX_WORK_SET;
 // Pairs are partitioned by their larger hull vertex count into NCX_NBUCKETS buckets, each run by
 // the kernel variant the autotuner picked for it.
 constexpr int NCX_NBUCKETS = 4;
 static_assert(NCX_OVF_T4_COUNT < NCX_OVF_TIER_WORDS && NCX_OVF_TIER_WORDS <= NCX_BKT_RANGE &&
                   NCX_BKT_RANGE + 2 * NCX_NBUCKETS <= NCX_KEY_CNT && NCX_NKEYS == 16 * NCX_OVERLAP_BINS * NCX_NBUCKETS &&
-                  NCX_WORK_BKT + NCX_NBUCKETS <= NCX_WORK_SETS,
+                  NCX_REC_COUNT + NCX_NBUCKETS <= NCX_REC_COUNT_TUNE && NCX_REC_COUNT_TUNE < NCX_OVF_TIER_WORDS &&
+                  NCX_WORK_BKT + NCX_NBUCKETS <= NCX_WORK_EPA && NCX_WORK_EPA + NCX_NBUCKETS <= NCX_WORK_SETS,
               "overflow header layout");
 // The work counter of launch k.
 inline uint32_t* ncx_work_set(uint32_t* ovf, uint32_t k) { return ovf + NCX_WORK_BASE + k * NCX_WORK_SET; }
 
-struct KArgs;  // contact kernel arguments (ncx_narrow.hip)
+struct KArgs;   // contact kernel arguments (ncx_narrow.hip)
+struct EpaRec;  // an intersecting pair's simplex (ncx_epa.h)
 
 // Overflow lists (NCX_OVF_* layout) and the arguments of the last tiered contact launch, one per
 // launch site (a shape set's batch calls, each scene), so launches on different streams never
@@ -106,8 +111,14 @@ struct ContactTiers {
   DevBuf bkey;       // each pair's sort key (count pass -> scatter pass)
   size_t bcap = 0;   // entries of blist and bkey
   uint32_t cap = 0;  // entries per overflow list
+  uint32_t sus0_cap = 0;  // slots of sus0
   KArgs* last = nullptr;
-  DevBuf sus[4];     // saved EPA runs handed on: T1 -> T2, T2 -> T3, T3 -> T4, T4 -> device-memory tier
+  DevBuf epa;        // the EPA kernels' memory:
+  float* sup = nullptr;     //   support points of the polytopes in flight
+  EpaRec* rec = nullptr;    //   records, one per pair at most
+  uint8_t* sus0 = nullptr;  //   saved runs handed from T1 to T2
+  size_t nrec = 0;
+  DevBuf sus[4];     // saved EPA runs handed on: (unused), T2 -> T3, T3 -> T4, T4 -> device-memory tier
   uint32_t* t1_list() const { return ovf.as<uint32_t>() + NCX_OVF_HEADER; }
   uint32_t* t2_list() const { return ovf.as<uint32_t>() + NCX_OVF_HEADER + cap; }
   uint32_t* t3_list() const { return ovf.as<uint32_t>() + NCX_OVF_HEADER + 2 * (size_t)cap; }
@@ -118,6 +129,7 @@ struct ContactTiers {
 struct ncx_shapes {
   ncx_ctx* ctx;
   size_t n = 0, npts = 0;
+  uint32_t buckets = 0xFu;  // bit b: a pair of vertex-count bucket b can occur
   DevBuf shapes;      // ncx_shape[n]
   DevBuf hx, hy, hz;  // hull pool
   ContactTiers tiers; // for ncx_contact_batch / ncx_distance_batch
@@ -288,7 +300,7 @@ struct ncx_mesh {
 
 // Tiered contact launch over pairs counted on the device (ncx_narrow.hip); no host
 // synchronisation unless may_tune (the autotuner's first run, never inside graph capture).
-int contact_tiers_reserve(ContactTiers& t, size_t cap);
+int contact_tiers_reserve(ContactTiers& t, ncx_ctx* ctx, size_t cap, size_t nrec);
 void contact_tiers_release(ContactTiers& t);
 int contact_tiers_reserve_list(ContactTiers& t, size_t npairs);
 int contacts_launch_device_count(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, const ncx_pose* poses,

@@ -893,7 +893,7 @@ extern "C" int ncx_contact_manifolds(ncx_manifolds* m, ncx_shapes* s, const ncx_
   if ((rc = build_hull_features(s))) return rc;
   if ((rc = m->idir.reserve(npairs * 12)) || (rc = m->has.reserve(npairs)) || (rc = m->w1.reserve(npairs * 12)) ||
       (rc = m->w2.reserve(npairs * 12)) || (rc = m->nrm.reserve(npairs * 12)) || (rc = m->depth.reserve(npairs * 4)) ||
-      (rc = m->fdir.reserve(npairs * 12)) || (rc = contact_tiers_reserve(m->tiers, npairs)))
+      (rc = m->fdir.reserve(npairs * 12)) || (rc = contact_tiers_reserve(m->tiers, ctx, npairs, npairs)))
     return rc;
   if ((rc = fill_u32(ctx, m->err.as<uint32_t>(), 1, 0u))) return rc;
   const unsigned nb = ceil_div(npairs, 256);

@@ -1,14 +1,12 @@
 // ncx_narrow.hip -- batched convex contact / distance (GJK + EPA) on the GPU.
 //
-// One group of G lanes (G = 4..64, a power of two inside a 64-wide wavefront)
-// handles one pair at a time; the grid loops over pairs.  Every lane of a group
-// runs the same GJK / EPA control flow on the same values (results are
-// identical across the group), and the lanes split the vertex scans of
-// ConvexHull support functions -- the dominant cost -- with an argmax reduction
-// that reproduces point_cloud_support_point_id's first-maximum rule
-// (src/utils/point_cloud_support_point.rs:6-24).  EPA's growing polytope lives
-// in a per-group arena in device memory; a pair whose polytope outgrows the
-// arena is re-run by the host in a second launch with a larger arena.
+// Contacts take two kernels.  k_contact_gjk runs GJK and the closed forms, one group of G lanes per
+// pair, finishes every pair that needs no EPA and writes an EPA record (the pair and its simplex)
+// for the others; k_epa (ncx_epa.h) runs the records on LDS arenas, in tiers of growing capacity.
+// Distances need GJK alone (k_distance).  Every lane of a group runs the same control flow on the
+// same values, and the lanes split the vertex scans of ConvexHull support functions with an argmax
+// reduction that reproduces point_cloud_support_point_id's first-maximum rule
+// (src/utils/point_cloud_support_point.rs:6-24).
 //
 // All arithmetic restates the reference in f32 with its operation order:
 //   GJK      src/query/algorithms/gjk.rs:76-177
@@ -17,7 +15,7 @@
 //   dispatch src/query/contact/contact_shape_shape.rs:10-48,
 //            src/query/distance/distance.rs:9-33
 #include <algorithm>
-#include "ncx_contact.h"
+#include "ncx_epa.h"
 
 struct KArgs {
   const ncx_shape* shapes;
@@ -41,16 +39,20 @@ struct KArgs {
   float* fdir;  // optional: the support-map result direction per pair (PairOut::fdir; the init_dir
                 // when that path returned nothing), for a per-pair direction cache
   float* dist;
-  uint8_t* arena;
+  uint8_t* arena;       // device-memory tier: EPA arenas of vcap vertices and fcap faces
   uint32_t vcap, fcap;
-  uint32_t* ovf_count;  // pairs whose EPA outgrew the arena
-  uint32_t* ovf_list;   // their pair indices (first ovf_cap of them)
+  EpaRec* rec;               // EPA records: GJK writes them, the EPA kernels read them
+  const uint32_t* rec_base;  // optional device offset into rec of this launch's records
+  uint32_t* rec_count;       // their number
+  float* sup;                // per EPA group: its polytope's support points, 6 floats a vertex
+  uint32_t* ovf_count;  // EPA runs that outgrew the arena
+  uint32_t* ovf_list;   // their records (first ovf_cap of them)
   uint32_t ovf_cap;
   int distance_mode;
   uint32_t nshapes;
   uint32_t* bad_index;  // set to 1 when a pair names a shape >= nshapes
-  const uint32_t* n_dev;  // optional device-side pair count (capped by npairs)
-  uint32_t* work;         // optional work counter (zero at launch): pairs are taken from it
+  const uint32_t* n_dev;  // optional device-side count of pairs or listed records (capped by npairs)
+  uint32_t* work;         // work counter (zero at launch): pairs and records are taken from it
   const uint32_t* range_b;  // optional device begin and end into list: a run of buckets
   const uint32_t* range_e;
   const uint8_t* sus_load;  // saved EPA runs of the list's ENTRY_SAVED entries, slot = list position
@@ -60,56 +62,82 @@ struct KArgs {
   uint32_t sus_save_cap;
 };
 
-// Contact/distance kernel, BS threads per block in groups of G lanes (one pair per group).
-// VC > 0: every group's EPA arena (VC vertices, FC faces, SC silhouette edges, STC search-stack
-// entries) lives in LDS; a pair whose polytope outgrows it is listed in ovf for a launch with
-// larger arenas.  VC == 0: the arena is the group's slice of a.arena (a.vcap, a.fcap) in device
-// memory.
-// Arena tiers (capacities; see the launch code below).
-#define T1_G 16
-#define T1_BS 128
-#define T1_VC 44u
-#define T1_FC 144u
-#define T1_SC 32u
-#define T1_STC 32u
-// A smaller first-tier arena (24 vertices, 80 faces, 2.7 KiB): nearly twice the arenas per CU
-// for pairs whose EPA ends within 20 iterations (most polytope pairs); the rest overflow to T2.
-#define T1S_VC 24u
-#define T1S_FC 80u
-#define T1S_SC 32u
-#define T1S_STC 32u
-#define T2_G 32
+// EPA arenas (ncx_epa.h): the first tier's two (40 and 20 iterations, of which 6 or 11 blocks of 8
+// runs fit a CU), then the tiers for the runs that outgrow them.
+typedef EpaArena<44, 86, 104, 32, 0, 10> ArenaT1;
+typedef EpaArena<24, 46, 54, 24, 0, 10> ArenaT1S;
+typedef EpaArena<64, 126, 150, 48, 0, 10> ArenaT2;
+typedef EpaArena<256, 510, 600, 96, 0, 10> ArenaT3;
+typedef EpaArena<2000, 4000, 4400, 256, 256, 16> ArenaT4;
+#define T1_BLOCKS 6u
+#define T1S_BLOCKS 11u
+#define T2_G 16
 #define T2_BS 64
-#define T2_BLOCKS_PER_CU (160u * 1024u / ((T2_BS / T2_G) * (uint32_t)arena_bytes(T2_VC, T2_FC, T2_SC, T2_STC)))
-#define T2_VC 128u
-#define T2_FC 384u
-#define T2_SC 64u
-#define T2_STC 64u
-#define T3_VC 512u
-#define T3_FC 1600u
-#define T3_SC 128u
-#define T3_STC 128u
-#define T4_VC 1536u
-#define T4_FC 4800u
-#define T4_SC 256u
-#define T4_STC 256u
+#define T2_BLOCKS_PER_CU 8u
+#define T3_BLOCKS_PER_CU 8u
+static_assert(ArenaT1::BYTES * 8 * T1_BLOCKS <= 163840 && ArenaT1S::BYTES * 8 * T1S_BLOCKS <= 163840, "blocks per CU");
+static_assert(ArenaT2::BYTES * (T2_BS / T2_G) * T2_BLOCKS_PER_CU <= 163840 && ArenaT4::BYTES <= 163840 &&
+                  ArenaT3::BYTES * T3_BLOCKS_PER_CU <= 163840, "blocks per CU");
+// Support points of the polytopes in flight, the most of any tier (per CU).
+constexpr size_t EPA_SUP_FLOATS_PER_CU = 6 * (size_t)std::max({T1_BLOCKS * 8 * ArenaT1::VC, T1S_BLOCKS * 8 * ArenaT1S::VC,
+                                                              T2_BLOCKS_PER_CU * (T2_BS / T2_G) * ArenaT2::VC,
+                                                              T3_BLOCKS_PER_CU * ArenaT3::VC, ArenaT4::VC});
 
 constexpr uint32_t ilog2_floor(uint32_t x) { return x <= 1 ? 0u : 1u + ilog2_floor(x >> 1); }
 
-template <int G, int BS, uint32_t VC, uint32_t FC, uint32_t SC, uint32_t STC, int MODE>
-__global__ __launch_bounds__(BS, MODE == 1 ? 3 : 2) void k_pairs(KArgs a) {
-  const int gl = threadIdx.x & (G - 1);
-  const size_t group = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) / G;
-  const size_t ngroups = ((size_t)gridDim.x * blockDim.x) / G;
-  constexpr bool LDS = VC > 0;
-  constexpr size_t LDS_BYTES = LDS ? (BS / G) * arena_bytes(VC, FC, SC, STC) : 16;
-  static_assert(LDS_BYTES <= 163840, "LDS arena exceeds the 160 KiB a gfx950 workgroup may hold");
-  static_assert(!LDS || (VC < 65536 && FC < 65536 && SC >= 3 && STC >= 3), "arena capacities");
-  static_assert(!LDS || ilog2_floor(FC) <= (uint32_t)G, "the parallel heap climb needs a lane per heap level");
-  __shared__ __align__(16) uint8_t lds_arena[LDS_BYTES];
-  Arena A;
-  if constexpr (LDS) A = arena_at(lds_arena, threadIdx.x / G, VC, FC, SC, STC);
-  else A = arena_at(a.arena, group, a.vcap, a.fcap, a.fcap, 2 * a.fcap);
+// The pair's shapes and poses, with the contact-manifold mode's capsules as their core segments
+// (capsule_shape_manifold_generator.rs:34-37, capsule_capsule_manifold_generator.rs:36-40), and
+// the pair's prediction.
+__device__ __forceinline__ Ctx2 contact_ctx(const KArgs& a, uint32_t i1, uint32_t i2, float& pred) {
+  Ctx2 c;
+  c.g1 = load_shape(a.shapes, i1);
+  c.g2 = load_shape(a.shapes, i2);
+  c.m1 = load_pose(a.poses, i1);
+  c.m2 = load_pose(a.poses, i2);
+  pred = a.prediction;
+  if (a.cap_seg) {
+    if (c.g1.type == NCX_CAPSULE) { pred = pred + c.g1.b; c.g1.type = SHAPE_SEGMENT; }
+    if (c.g2.type == NCX_CAPSULE) { pred = pred + c.g2.b; c.g2.type = SHAPE_SEGMENT; }
+  }
+  return c;
+}
+
+__device__ __forceinline__ void write_contact(const KArgs& a, size_t k, const PairOut& o, f3 idir) {
+  a.has[k] = (uint8_t)o.has;
+  const bool h = o.has == 1;
+  const f3 z = f3{0.f, 0.f, 0.f}, w1 = sel3(h, o.w1, z), w2 = sel3(h, o.w2, z), n = sel3(h, o.n, z);
+  a.w1[3 * k] = w1.x; a.w1[3 * k + 1] = w1.y; a.w1[3 * k + 2] = w1.z;
+  a.w2[3 * k] = w2.x; a.w2[3 * k + 1] = w2.y; a.w2[3 * k + 2] = w2.z;
+  a.nrm[3 * k] = n.x; a.nrm[3 * k + 1] = n.y; a.nrm[3 * k + 2] = n.z;
+  a.depth[k] = h ? o.depth : 0.f;
+  if (a.fdir) {
+    // ConvexPolyhedronConvexPolyhedronManifoldGenerator keeps its last_gjk_dir when the
+    // result carries no direction (manifold_generator.rs:115-146)
+    const bool z = o.fdir.x == 0.f && o.fdir.y == 0.f && o.fdir.z == 0.f;
+    const f3 fd = z ? idir : o.fdir;
+    a.fdir[3 * k] = fd.x; a.fdir[3 * k + 1] = fd.y; a.fdir[3 * k + 2] = fd.z;
+  }
+}
+
+__device__ __forceinline__ f3 load_init_dir(const KArgs& a, size_t k) {
+  if (!a.init_dir) return f3{0.f, 0.f, 0.f};
+  return f3{a.init_dir[3 * k], a.init_dir[3 * k + 1], a.init_dir[3 * k + 2]};
+}
+
+#define GJK_BS 256
+
+// The pairs of a wavefront's next pass: 64 / G of them, with one atomic.
+template <int G>
+__device__ __forceinline__ size_t next_pairs(uint32_t* work, int lane) {
+  uint32_t t = 0;
+  if (lane == 0) t = atomicAdd(work, 64u / G);
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)t) + (uint32_t)lane / G;
+}
+
+// GJK and closed forms of contact pairs; the pairs that need EPA leave a record.
+template <int G>
+__global__ __launch_bounds__(GJK_BS, 2) void k_contact_gjk(KArgs a) {
+  const int lane = threadIdx.x & 63, gl = lane & (G - 1);
   size_t npairs = a.npairs;
   if (a.n_dev) npairs = min(npairs, (size_t)*a.n_dev);
   size_t lbase = 0;
@@ -117,33 +145,237 @@ __global__ __launch_bounds__(BS, MODE == 1 ? 3 : 2) void k_pairs(KArgs a) {
     lbase = *a.range_b;
     npairs = *a.range_e - lbase;
   }
-  for (size_t it = 0;; ++it) {
-    size_t q;
-    if (a.work) {  // next pair from the work counter (lane 0 of the group takes it)
-      uint32_t t = 0;
-      if (gl == 0) t = atomicAdd(a.work, 1u);
-      q = (uint32_t)__shfl((int)t, 0, G);
-    } else {
-      q = group + it * ngroups;
+  const size_t rbase = a.rec_base ? *a.rec_base : 0;
+  for (;;) {
+    const size_t q = next_pairs<G>(a.work, lane);
+    if (__ballot(q < npairs) == 0) break;
+    bool epa_pair = false;
+    uint32_t k = 0, kind = 0;
+    Simplex s;
+    if (q < npairs) {
+      k = a.list ? a.list[lbase + q] : (uint32_t)q;
+      const uint32_t i1 = a.ia[k], i2 = a.ib[k];
+      if (i1 >= a.nshapes || i2 >= a.nshapes) {
+        if (gl == 0) atomicOr(a.bad_index, 1u);
+      } else {
+        float pred;
+        const Ctx2 c = contact_ctx(a, i1, i2, pred);
+        // An all-zero init_dir means None for this pair (the reference's default direction).
+        const f3 idir = load_init_dir(a, k);
+        bool has_init = idir.x != 0.f || idir.y != 0.f || idir.z != 0.f;
+        PairOut o;
+        int extra_iters = 0;
+        for (;;) {
+          o = contact_pair<G>(c, pred, has_init, idir, a.P, gl, has_init ? a.max_iter : 10000, s, kind);
+          if (o.has != 3) break;
+          // a warm start that hit its iteration cap: plain GJK (init_dir = None) judges the pair
+          extra_iters = o.gjk_iters;
+          has_init = false;
+        }
+        epa_pair = o.has == 5;
+        if (gl == 0) {
+          if (a.iters) a.iters[k] = o.gjk_iters + extra_iters;
+          if (!epa_pair) write_contact(a, k, o, idir);
+        }
+      }
     }
+    const uint64_t em = __ballot(epa_pair && gl == 0);
+    if (em) {
+      uint32_t t = 0;
+      const int first = __builtin_ctzll(em);
+      if (lane == first) t = atomicAdd(a.rec_count, (uint32_t)__popcll(em));
+      t = (uint32_t)__builtin_amdgcn_readlane((int)t, first);
+      if (epa_pair && gl == 0) {
+        float4* r = (float4*)(a.rec + rbase + t + (uint32_t)__popcll(em & ((1ull << lane) - 1ull)));
+        r[0] = float4{__uint_as_float(k), __uint_as_float((uint32_t)s.dim | (kind << 2)), 0.f, 0.f};
+        r[1] = float4{s.v0.o1.x, s.v0.o1.y, s.v0.o1.z, s.v0.o2.x};
+        r[2] = float4{s.v0.o2.y, s.v0.o2.z, s.v1.o1.x, s.v1.o1.y};
+        r[3] = float4{s.v1.o1.z, s.v1.o2.x, s.v1.o2.y, s.v1.o2.z};
+        r[4] = float4{s.v2.o1.x, s.v2.o1.y, s.v2.o1.z, s.v2.o2.x};
+        r[5] = float4{s.v2.o2.y, s.v2.o2.z, s.v3.o1.x, s.v3.o1.y};
+        r[6] = float4{s.v3.o1.z, s.v3.o2.x, s.v3.o2.y, s.v3.o2.z};
+      }
+    }
+  }
+}
+
+// The two support maps of a record's pair.
+__device__ __forceinline__ Ctx2 epa_ctx(const KArgs& a, uint32_t k, uint32_t kind) {
+  float pred;
+  const Ctx2 c = contact_ctx(a, a.ia[k], a.ib[k], pred);
+  if (kind == EPA_KIND_SM) return c;
+  if (kind == EPA_KIND_BALL_FIRST) return ball_projection_ctx(c.m1.t, c.m2, c.g2);
+  return ball_projection_ctx(c.m2.t, c.m1, c.g1);
+}
+
+// Completes pair k from its EPA run's points and normal (ok) or failure, as the path that started
+// it does (contact_sm, contact_ball_convex), and writes it.
+__device__ __forceinline__ void epa_write(const KArgs& a, uint32_t k, uint32_t kind, bool ok, f3 p1, f3 p2, f3 n) {
+  PairOut o;
+  pair_none(o);
+  if (kind == EPA_KIND_SM) {
+    if (ok) contact_sm_finish(o, p1, p2, n);
+    else o.fdir = f3{1.f, 0.f, 0.f};  // NoIntersection(x_axis)
+  } else {
+    float pred;
+    const Ctx2 c = contact_ctx(a, a.ia[k], a.ib[k], pred);
+    const bool first = kind == EPA_KIND_BALL_FIRST;
+    const f3 c1 = first ? c.m1.t : c.m2.t;
+    ball_convex_finish(o, c1, first ? c.g1.a : c.g2.a, ok ? p1 + c1 : c1, true, true, f3{0.f, 0.f, 0.f}, pred);
+    contact_flip(o, !first);
+  }
+  write_contact(a, k, o, load_init_dir(a, k));
+}
+
+// EPA records on LDS arenas (ncx_epa.h says what bounds them), BS threads per block in groups of G
+// lanes, one record per group at a time.  Every pass of the loop runs one iteration of each group's record; groups without one take
+// the next records together, with one atomic per wavefront, once REFILL of them wait or none runs.
+// SAVES: a run about to outgrow the arena is saved for the next tier.  LISTED: the records come
+// from the overflow list of the tier before (entries may be saved runs), otherwise from rec_base on.
+template <int G, int BS, class L, int REFILL, bool SAVES, bool LISTED>
+__global__ __launch_bounds__(BS, 1) void k_epa(KArgs a) {
+  static_assert(ilog2_floor(L::HC) <= (uint32_t)G, "the heap steps need a lane per heap level");
+  __shared__ __align__(16) uint8_t lds[(BS / G) * L::BYTES];
+  const int lane = threadIdx.x & 63, gl = lane & (G - 1), gbase = lane & ~(G - 1);
+  const uint64_t gmask = G == 64 ? ~0ull : ((1ull << (G & 63)) - 1ull);
+  L A;
+  A.p = lds + (threadIdx.x / G) * L::BYTES;
+  float* const sup = a.sup + ((size_t)blockIdx.x * (BS / G) + threadIdx.x / G) * (6 * (size_t)L::VC);
+  uint32_t n = LISTED ? min(*a.n_dev, a.ovf_cap) : *a.rec_count;
+  const uint32_t rbase = !LISTED && a.rec_base ? *a.rec_base : 0u;
+  bool live = false, done = false;
+  Ctx2 c;
+  EpaState<L> s;
+  uint32_t rec = 0, k = 0, kind = 0;
+  int st = EPA_RUNNING;
+  for (;;) {
+    const uint64_t wm = __ballot(!live && !done && gl == 0), lm = __ballot(live);
+    if ((wm | lm) == 0) break;
+    if (wm && (lm == 0 || __popcll(wm) >= REFILL)) {
+      uint32_t t = 0;
+      const int first = __builtin_ctzll(wm);
+      if (lane == first) t = atomicAdd(a.work, (uint32_t)__popcll(wm));
+      t = (uint32_t)__builtin_amdgcn_readlane((int)t, first);
+      if (!live && !done) {
+        const uint32_t q = t + (uint32_t)__popcll(wm & ((1ull << gbase) - 1ull));
+        if (q >= n) {
+          done = true;
+        } else {
+          live = true;
+          const uint32_t entry = LISTED ? a.list[q] : rbase + q;
+          rec = entry & ~ENTRY_SAVED;
+          const EpaRec* r = a.rec + rec;
+          k = r->k;
+          kind = r->dim_kind >> 2;
+          c = epa_ctx(a, k, kind);
+          if (LISTED && (entry & ENTRY_SAVED)) {
+            epa_read_saved<G>(a.sus_load + (size_t)q * a.sus_load_bytes, A, sup, s, gl);
+            st = EPA_RUNNING;
+          } else {
+            st = epa_begin<G>(A, r, sup, s, gl, gbase, gmask);
+          }
+        }
+      }
+    }
+    if (live) {
+      if (st == EPA_RUNNING) st = epa_step<G, L, SAVES>(A, c, a.P, sup, s, gl, gbase, gmask);
+      if (st != EPA_RUNNING) {
+        live = false;
+        if (st == EPA_TOO_LARGE || st == EPA_SUSPEND) {
+          uint32_t slot = 0;
+          if (gl == 0) slot = atomicAdd(a.ovf_count, 1u);
+          slot = (uint32_t)__shfl((int)slot, gbase, 64);
+          bool saved = false;
+          if constexpr (SAVES) {
+            saved = st == EPA_SUSPEND && slot < a.sus_save_cap;
+            if (saved) {
+              __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+              epa_write_saved<G>(a.sus_save + (size_t)slot * a.sus_save_bytes, A, sup, s, gl);
+            }
+          }
+          if (gl == 0 && slot < a.ovf_cap) a.ovf_list[slot] = rec | (saved ? ENTRY_SAVED : 0u);
+        } else if (gl == 0) {
+          f3 p1 = f3{0.f, 0.f, 0.f}, p2 = p1, nn = f3{0.f, 1.f, 0.f};
+          if (st == EPA_FACE) {
+            // Face::closest_points with the barycentric coordinates new_with_proj stored (zero
+            // unless the projection was inside the face)
+            const typename L::W w = s.end;
+            const float* q0 = sup + 6 * fld<L::BITS>(w, 0);
+            const float* q1 = sup + 6 * fld<L::BITS>(w, 1);
+            const float* q2 = sup + 6 * fld<L::BITS>(w, 2);
+            const f3 a1 = f3{q0[0], q0[1], q0[2]}, a2 = f3{q0[3], q0[4], q0[5]};
+            const f3 b1 = f3{q1[0], q1[1], q1[2]}, b2 = f3{q1[3], q1[4], q1[5]};
+            const f3 c1 = f3{q2[0], q2[1], q2[2]}, c2 = f3{q2[3], q2[4], q2[5]};
+            const f3 va = a1 - a2, vb = b1 - b2, vc = c1 - c2;
+            Loc loc;
+            proj_triangle(va, vb, vc, loc);
+            float b0 = 0.f, b1c = 0.f, b2c = 0.f;
+            if (loc.kind == LOC_FACE) { b0 = loc.bc0; b1c = loc.bc1; b2c = loc.bc2; }
+            p1 = a1 * b0 + b1 * b1c + c1 * b2c;
+            p2 = a2 * b0 + b2 * b1c + c2 * b2c;
+            nn = tri_normal(va, vb, vc);
+          }
+          epa_write(a, k, kind, st != EPA_NOTHING, p1, p2, nn);
+        }
+      }
+    }
+  }
+}
+
+// EPA records on device-memory arenas (a.vcap, a.fcap), a wavefront per listed record.
+__global__ __launch_bounds__(64, 1) void k_epa_global(KArgs a) {
+  const int gl = threadIdx.x & 63;
+  const size_t q = blockIdx.x;
+  if (q >= a.npairs) return;
+  const Arena A = arena_at(a.arena, q, a.vcap, a.fcap, a.fcap, 2 * a.fcap);
+  const uint32_t entry = a.list[q], rec = entry & ~ENTRY_SAVED;
+  const EpaRec* r = a.rec + rec;
+  const uint32_t k = r->k, kind = r->dim_kind >> 2;
+  const Ctx2 c = epa_ctx(a, k, kind);
+  Simplex s;
+  sx_init(s);
+  s.dim = (int)(r->dim_kind & 3u);
+  auto vertex = [&](int i) {
+    CSO v;
+    v.o1 = f3{r->v[i][0], r->v[i][1], r->v[i][2]};
+    v.o2 = f3{r->v[i][3], r->v[i][4], r->v[i][5]};
+    return v;
+  };
+  s.v0 = vertex(0);
+  s.v1 = vertex(1);
+  s.v2 = vertex(2);
+  s.v3 = vertex(3);
+  const uint8_t* load = (entry & ENTRY_SAVED) && a.sus_load ? a.sus_load + q * a.sus_load_bytes : nullptr;
+  f3 p1, p2, n;
+  int it;
+  const int e = epa<64>(c, s, a.P, gl, A, p1, p2, n, it, load);
+  if (gl != 0) return;
+  if (e == EPA_OVERFLOW) {
+    const uint32_t slot = atomicAdd(a.ovf_count, 1u);
+    if (slot < a.ovf_cap) a.ovf_list[slot] = rec;
+  } else {
+    epa_write(a, k, kind, e == EPA_OK, p1, p2, n);
+  }
+}
+
+// Distances (query::distance, distance.rs:9-33), BS threads per block in groups of G lanes, one
+// pair per group at a time from the work counter.
+template <int G, int BS>
+__global__ __launch_bounds__(BS, 3) void k_distance(KArgs a) {
+  const int gl = threadIdx.x & (G - 1);
+  size_t npairs = a.npairs;
+  size_t lbase = 0;
+  if (a.range_b) {
+    lbase = *a.range_b;
+    npairs = *a.range_e - lbase;
+  }
+  for (;;) {
+    uint32_t t = 0;
+    if (gl == 0) t = atomicAdd(a.work, 1u);
+    const size_t q = (uint32_t)__shfl((int)t, 0, G);
     if (q >= npairs) break;
-    const uint32_t entry = a.list ? a.list[lbase + q] : (uint32_t)q;
-    size_t k = entry & ~ENTRY_SAVED;
-    EpaIO io;
-    // Runs are saved by the second to fourth LDS tiers and continued by the third, fourth and
-    // device-memory tiers; the first tier, where nearly all pairs finish, has neither path.
-    constexpr bool SAVES = LDS && VC > T1_VC;
-    constexpr bool LOADS = !LDS || VC > T2_VC;
-    io.load = (LOADS && a.list && (entry & ENTRY_SAVED) && a.sus_load) ? a.sus_load + (size_t)q * a.sus_load_bytes
-                                                                       : nullptr;
-    io.save = SAVES ? a.sus_save : nullptr;
-    io.save_bytes = a.sus_save_bytes;
-    io.save_cap = a.sus_save_cap;
-    io.count = a.ovf_count;
-    io.list = a.ovf_list;
-    io.list_cap = a.ovf_cap;
-    io.k = (uint32_t)k;
-    uint32_t i1 = a.ia[k], i2 = a.ib[k];
+    const size_t k = a.list ? a.list[lbase + q] : (uint32_t)q;
+    const uint32_t i1 = a.ia[k], i2 = a.ib[k];
     if (i1 >= a.nshapes || i2 >= a.nshapes) {
       if (gl == 0) atomicOr(a.bad_index, 1u);
       continue;
@@ -153,109 +385,50 @@ __global__ __launch_bounds__(BS, MODE == 1 ? 3 : 2) void k_pairs(KArgs a) {
     c.g2 = load_shape(a.shapes, i2);
     c.m1 = load_pose(a.poses, i1);
     c.m2 = load_pose(a.poses, i2);
-    float pred = a.prediction;
-    if (MODE == 0 && a.cap_seg) {
-      // CapsuleShapeManifoldGenerator / CapsuleCapsuleManifoldGenerator
-      // (capsule_shape_manifold_generator.rs:34-37, capsule_capsule_manifold_generator.rs:36-40)
-      if (c.g1.type == NCX_CAPSULE) { pred = pred + c.g1.b; c.g1.type = SHAPE_SEGMENT; }
-      if (c.g2.type == NCX_CAPSULE) { pred = pred + c.g2.b; c.g2.type = SHAPE_SEGMENT; }
-    }
-    if (MODE == 1) {  // distance (a compile-time branch: each kernel holds one query's code)
-      float d = 0.f;
-      int it = 0;
-      bool ovf = false;
-      if (c.g1.type == NCX_BALL && c.g2.type == NCX_BALL) {
-        // distance_ball_ball (distance_ball_ball.rs:7-24)
-        f3 delta = c.m2.t - c.m1.t;
-        float d2 = norm_sq(delta);
-        float sr = c.g1.a + c.g2.a;
-        d = d2 <= sr * sr ? 0.f : __builtin_sqrtf(d2) - sr;
-      } else {
-        // distance_support_map_support_map_with_params (distance_support_map_support_map.rs:25-53)
-        // init_dir (an all-zero entry means None) with GJK capped at max_iter; on the cap,
-        // plain GJK from the default direction judges the pair.
-        f3 d0 = c.m1.t - c.m2.t;
-        bool warm = false;
-        if (a.init_dir) {
-          f3 idir = f3{a.init_dir[3 * k], a.init_dir[3 * k + 1], a.init_dir[3 * k + 2]};
-          if (idir.x != 0.f || idir.y != 0.f || idir.z != 0.f) {
-            d0 = idir;
-            warm = true;
-          }
+    float d = 0.f;
+    int it = 0;
+    if (c.g1.type == NCX_BALL && c.g2.type == NCX_BALL) {
+      // distance_ball_ball (distance_ball_ball.rs:7-24)
+      f3 delta = c.m2.t - c.m1.t;
+      float d2 = norm_sq(delta);
+      float sr = c.g1.a + c.g2.a;
+      d = d2 <= sr * sr ? 0.f : __builtin_sqrtf(d2) - sr;
+    } else {
+      // distance_support_map_support_map_with_params (distance_support_map_support_map.rs:25-53)
+      // init_dir (an all-zero entry means None) with GJK capped at max_iter; on the cap,
+      // plain GJK from the default direction judges the pair.
+      f3 d0 = c.m1.t - c.m2.t;
+      const f3 idir = load_init_dir(a, k);
+      bool warm = idir.x != 0.f || idir.y != 0.f || idir.z != 0.f;
+      if (warm) d0 = idir;
+      for (int pass = 0; pass < 2; ++pass) {
+        f3 dir;
+        float nl;
+        if (!try_normalize(d0, NCX_FLT_EPS, &dir, &nl)) dir = f3{1.f, 0.f, 0.f};
+        Simplex s;
+        GJKOut r = gjk<G>(c, dir, NCX_FLT_MAX, s, a.P, gl, warm ? a.max_iter : 10000);
+        it += r.iters;
+        if (warm && r.status == GJK_S_CAP && a.max_iter < 10000) {
+          warm = false;
+          d0 = c.m1.t - c.m2.t;
+          continue;
         }
-        for (int pass = 0; pass < 2; ++pass) {
-          f3 dir;
-          float nl;
-          if (!try_normalize(d0, NCX_FLT_EPS, &dir, &nl)) dir = f3{1.f, 0.f, 0.f};
-          Simplex s;
-          sx_init(s);
-          sx_reset(s, cso_from<G>(c, dir, a.P, gl));
-          GJKOut r = gjk<G>(c, NCX_FLT_MAX, s, a.P, gl, warm ? a.max_iter : 10000);
-          it += r.iters;
-          if (warm && r.status == GJK_S_CAP && a.max_iter < 10000) {
-            warm = false;
-            d0 = c.m1.t - c.m2.t;
-            continue;
-          }
-          d = r.status == GJK_S_CLOSEST ? norm(r.p1 - r.p2) : 0.f;
-          break;
-        }
+        d = r.status == GJK_S_CLOSEST ? norm(r.p1 - r.p2) : 0.f;
+        break;
       }
-      (void)ovf;
-      if (gl == 0) {
-        a.dist[k] = d;
-        if (a.iters) a.iters[k] = it;
-      }
-      continue;
-    }
-    f3 idir = f3{0.f, 0.f, 0.f};
-    bool has_init = false;
-    if (a.init_dir) {
-      idir = f3{a.init_dir[3 * k], a.init_dir[3 * k + 1], a.init_dir[3 * k + 2]};
-      // An all-zero entry means None for this pair (the reference's default direction).
-      has_init = idir.x != 0.f || idir.y != 0.f || idir.z != 0.f;
-    }
-    PairOut o = contact_pair<G, LDS ? 1 : 2>(c, pred, has_init, idir, a.P, gl, A, has_init ? a.max_iter : 10000, io);
-    int extra_iters = 0;
-    if (o.has == 3) {
-      // Warm start hit its iteration cap: plain GJK (init_dir = None) judges the pair.
-      extra_iters = o.gjk_iters;
-      o = contact_pair<G, LDS ? 1 : 2>(c, pred, false, idir, a.P, gl, A, 10000, io);
-    }
-    if (o.has == 4) continue;  // suspended: listed (and saved) for the next tier
-    if (o.has == 2) {
-      if (gl == 0) {
-        uint32_t slot = atomicAdd(a.ovf_count, 1u);
-        if (slot < a.ovf_cap) a.ovf_list[slot] = (uint32_t)k;
-      }
-      continue;
     }
     if (gl == 0) {
-      a.has[k] = (uint8_t)o.has;
-      if (o.has == 1) {
-        a.w1[3 * k] = o.w1.x; a.w1[3 * k + 1] = o.w1.y; a.w1[3 * k + 2] = o.w1.z;
-        a.w2[3 * k] = o.w2.x; a.w2[3 * k + 1] = o.w2.y; a.w2[3 * k + 2] = o.w2.z;
-        a.nrm[3 * k] = o.n.x; a.nrm[3 * k + 1] = o.n.y; a.nrm[3 * k + 2] = o.n.z;
-        a.depth[k] = o.depth;
-      } else {
-        a.w1[3 * k] = 0.f; a.w1[3 * k + 1] = 0.f; a.w1[3 * k + 2] = 0.f;
-        a.w2[3 * k] = 0.f; a.w2[3 * k + 1] = 0.f; a.w2[3 * k + 2] = 0.f;
-        a.nrm[3 * k] = 0.f; a.nrm[3 * k + 1] = 0.f; a.nrm[3 * k + 2] = 0.f;
-        a.depth[k] = 0.f;
-      }
-      if (a.iters) a.iters[k] = o.gjk_iters + extra_iters;
-      if (a.fdir) {
-        // ConvexPolyhedronConvexPolyhedronManifoldGenerator keeps its last_gjk_dir when the
-        // result carries no direction (manifold_generator.rs:115-146)
-        const bool z = o.fdir.x == 0.f && o.fdir.y == 0.f && o.fdir.z == 0.f;
-        const f3 fd = z ? idir : o.fdir;
-        a.fdir[3 * k] = fd.x; a.fdir[3 * k + 1] = fd.y; a.fdir[3 * k + 2] = fd.z;
-      }
+      a.dist[k] = d;
+      if (a.iters) a.iters[k] = it;
     }
   }
 }
 
 // ------------------------------------------------------------------ host side
+// Vertex-count bucket of the larger hull vertex count m of a pair (0: no hull).
+__host__ __device__ __forceinline__ uint32_t count_bucket(uint32_t m) {
+  return m == 0 ? 0u : (m <= 32 ? 1u : (m <= 96 ? 2u : 3u));
+}
 __global__ void k_shape_radius(ncx_shape* __restrict__ shapes, size_t n, Pool P);
 
 extern "C" int ncx_shapes_create(ncx_ctx* ctx, const ncx_shape* shapes, size_t n, const float* hx, const float* hy,
@@ -269,12 +442,15 @@ extern "C" int ncx_shapes_create(ncx_ctx* ctx, const ncx_shape* shapes, size_t n
                   "ncx_shapes_create: hull range outside the point pool");
   }
   ncx_shapes* S = new ncx_shapes;
+  S->buckets = 0;
+  for (size_t i = 0; i < n; ++i)
+    S->buckets |= 1u << (shapes[i].type == NCX_CONVEX_HULL ? count_bucket(shapes[i].hull_count) : 0u);
   S->ctx = ctx;
   S->n = n;
   S->npts = npts;
   int rc;
   if ((rc = S->shapes.reserve(n * sizeof(ncx_shape) + 64)) || (rc = S->hx.reserve(npts * 4 + 4)) ||
-      (rc = S->hy.reserve(npts * 4 + 4)) || (rc = S->hz.reserve(npts * 4 + 4)) || (rc = contact_tiers_reserve(S->tiers, 4096))) {
+      (rc = S->hy.reserve(npts * 4 + 4)) || (rc = S->hz.reserve(npts * 4 + 4)) || (rc = contact_tiers_reserve(S->tiers, ctx, 4096, 4096))) {
     delete S;
     return rc;
   }
@@ -339,7 +515,7 @@ __device__ __forceinline__ uint32_t pair_key(const ncx_shape* __restrict__ shape
   uint32_t c1 = s1.type == NCX_CONVEX_HULL ? s1.hull_count : 0;
   uint32_t c2 = s2.type == NCX_CONVEX_HULL ? s2.hull_count : 0;
   uint32_t m = c1 > c2 ? c1 : c2;
-  uint32_t b = m == 0 ? 0u : (m <= 32 ? 1u : (m <= 96 ? 2u : 3u));
+  const uint32_t b = count_bucket(m);
   uint32_t t1 = s1.type < 3u ? s1.type : 3u, t2 = s2.type < 3u ? s2.type : 3u;
   const float dx = poses[i1].tx - poses[i2].tx, dy = poses[i1].ty - poses[i2].ty, dz = poses[i1].tz - poses[i2].tz;
   const float rs = __uint_as_float(s1.pad[0]) + __uint_as_float(s2.pad[0]);
@@ -398,17 +574,24 @@ __global__ __launch_bounds__(BKT_BLOCK) void k_bucket_count(const uint32_t* __re
     if (h[k]) atomicAdd(&hdr[NCX_KEY_CNT + k], h[k]);
 }
 
-// Key offsets (the scatter cursors) and each bucket's range [begin, end) in the partitioned list.
-__global__ void k_bucket_offsets(uint32_t* __restrict__ hdr) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  uint32_t off = 0;
-  for (uint32_t key = 0; key < NCX_NKEYS; ++key) {
-    constexpr uint32_t per_bucket = NCX_NKEYS / NCX_NBUCKETS;
-    if (key % per_bucket == 0) hdr[NCX_BKT_RANGE + 2 * (key / per_bucket)] = off;
-    hdr[NCX_KEY_FILL + key] = off;
-    off += hdr[NCX_KEY_CNT + key];
-    if (key % per_bucket == per_bucket - 1) hdr[NCX_BKT_RANGE + 2 * (key / per_bucket) + 1] = off;
+// Key offsets (the scatter cursors) and each bucket's range [begin, end) in the partitioned list:
+// one thread per key, an inclusive scan in LDS (one thread over all keys took 20 us).
+__global__ __launch_bounds__(NCX_NKEYS) void k_bucket_offsets(uint32_t* __restrict__ hdr) {
+  constexpr uint32_t per_bucket = NCX_NKEYS / NCX_NBUCKETS;
+  __shared__ uint32_t sum[NCX_NKEYS];
+  const uint32_t key = threadIdx.x, c = hdr[NCX_KEY_CNT + key];
+  uint32_t x = c;
+  sum[key] = x;
+  for (uint32_t o = 1; o < NCX_NKEYS; o *= 2) {
+    __syncthreads();
+    const uint32_t y = key >= o ? sum[key - o] : 0u;
+    __syncthreads();
+    x += y;
+    sum[key] = x;
   }
+  hdr[NCX_KEY_FILL + key] = x - c;
+  if (key % per_bucket == 0) hdr[NCX_BKT_RANGE + 2 * (key / per_bucket)] = x - c;
+  if (key % per_bucket == per_bucket - 1) hdr[NCX_BKT_RANGE + 2 * (key / per_bucket) + 1] = x;
 }
 
 // Pass 2: scatter pair indices to their key's range (one atomic per key per block for the
@@ -444,28 +627,45 @@ __global__ __launch_bounds__(BKT_BLOCK) void k_bucket_scatter(const uint32_t* __
 }
 
 // Arena tiers, all but the last in LDS and in the graph:
-//   T1: 8 pairs per block (8, 16 or 32 lanes per pair, the autotuner's choice), arenas of 44
-//       vertices and 144 faces (4.7 KiB per pair; 4 blocks fit a CU);
-//   T2: 32 lanes per pair, 2 pairs per 64-thread block, 128 vertices and 384 faces (12.5 KiB;
-//       with 16 lanes and 4 pairs per block only 3 blocks fit a CU's LDS, one SIMD idle);
-//   T3: 64 lanes, one pair per 64-thread block, 512 vertices and 1600 faces (51 KiB);
-//   T4: 64 lanes, one pair per 64-thread block, T4_VC vertices and T4_FC faces (up to the
-//       160 KiB a gfx950 workgroup may hold; one block per CU);
-//   then device-memory arenas 8x larger than T4's, 64 lanes per pair, host-driven.
+//   T1: 8 records per block (8, 16 or 32 lanes each, the autotuner's choice), arenas of 44 or 24
+//       vertices (3.3 and 1.9 KB; 6 or 11 blocks fit a CU);
+//   T2: 16 lanes, 4 records per 64-thread block, 64 vertices (5.0 KB);
+//   T3: 64 lanes, one record per block, 256 vertices (20 KB);
+//   T4: 64 lanes, one record per block, 2000 vertices (132 KB, one block per CU);
+//   then device-memory arenas 8x larger than T4's, 64 lanes per record, host-driven.
 
 // Saved-run slots handed from each LDS tier to the next (the first SUS_CAP[t] suspended runs of
-// a launch are saved; later ones start again in the next tier) and their sizes.  The first tier
-// saves nothing (slot count 0): replaying its short runs costs less than carrying the save path
-// in its kernel.
-static const uint32_t SUS_CAP[4] = {0, 4096, 1024, 256};
-static const size_t SUS_BYTES[4] = {epa_save_bytes(T1_VC, T1_FC), epa_save_bytes(T2_VC, T2_FC),
-                                    epa_save_bytes(T3_VC, T3_FC), epa_save_bytes(T4_VC, T4_FC)};
+// a launch are saved; later ones start again in the next tier) and their sizes.  The first tier's
+// are at most one for 32 pairs.  About one run in ten takes more than 20 iterations (12 on average)
+// on a scene of mixed shapes, so runs started again would cost the second tier three times the
+// iterations that continued ones do.
+static const uint32_t SUS_CAP[4] = {1u << 19, 4096, 1024, 256};
+static const size_t SUS_BYTES[4] = {epa_save_bytes(ArenaT1::VC, ArenaT1::HC), epa_save_bytes(ArenaT2::VC, ArenaT2::HC),
+                                    epa_save_bytes(ArenaT3::VC, ArenaT3::HC), epa_save_bytes(ArenaT4::VC, ArenaT4::HC)};
+static_assert(ArenaT1::FC + 2 <= ArenaT1::HC && ArenaT1S::HC <= ArenaT1::HC, "a saved run's faces");
+static_assert(ArenaT2::FC + 2 <= ArenaT2::HC && ArenaT3::FC + 2 <= ArenaT3::HC && ArenaT4::FC + 2 <= ArenaT4::HC,
+              "a saved run's faces");
 
 // Overflow lists of at least cap entries each (at most 2^24: a call with more overflowing pairs
-// fails with NCX_E_CAPACITY), and the saved-run slots.
-int contact_tiers_reserve(ContactTiers& t, size_t cap) {
-  for (int i = 0; i < 4; ++i) {
-    if (t.sus[i].p || SUS_CAP[i] == 0) continue;
+// fails with NCX_E_CAPACITY), the saved-run slots, and EPA records of nrec pairs (0: none, for
+// distances).
+int contact_tiers_reserve(ContactTiers& t, ncx_ctx* ctx, size_t cap, size_t nrec) {
+  if (nrec > t.nrec) {
+    // one allocation: support points, records, the first tier's saved runs
+    const size_t sup = (size_t)ctx->num_cus * EPA_SUP_FLOATS_PER_CU * 4;
+    const size_t slots = std::min<size_t>(SUS_CAP[0], nrec / 32);
+    t.epa.release();
+    t.nrec = 0;
+    int rc = t.epa.reserve(sup + nrec * sizeof(EpaRec) + slots * SUS_BYTES[0]);
+    if (rc) return rc;
+    t.nrec = nrec;
+    t.sus0_cap = (uint32_t)slots;
+    t.sup = t.epa.as<float>();
+    t.rec = (EpaRec*)(t.epa.as<uint8_t>() + sup);
+    t.sus0 = (uint8_t*)(t.rec + nrec);
+  }
+  for (int i = 1; i < 4; ++i) {
+    if (t.sus[i].p) continue;
     int rc = t.sus[i].reserve((size_t)SUS_CAP[i] * SUS_BYTES[i]);
     if (rc) return rc;
   }
@@ -483,23 +683,17 @@ void contact_tiers_release(ContactTiers& t) {
   t.ovf.release();
   t.blist.release();
   t.bkey.release();
+  t.epa.release();
+  t.nrec = 0;
   t.bcap = 0;
   t.cap = 0;
+  t.sus0_cap = 0;
   for (int i = 0; i < 4; ++i) t.sus[i].release();
   delete t.last;
   t.last = nullptr;
 }
 
-// Device-memory tiers (VC = 0): static grid-stride over the listed pairs.
-static int launch_global_tier(hipStream_t stream, KArgs a, size_t npairs) {
-  a.npairs = npairs;
-  a.work = nullptr;
-  hipLaunchKernelGGL((k_pairs<64, 128, 0u, 0u, 0u, 0u, 0>), dim3(ceil_div(npairs * 64, 128)), dim3(128), 0, stream, a);
-  NCX_HIP_CHECK(hipGetLastError());
-  return NCX_OK;
-}
-
-// Re-runs the n pairs listed at list_src (device) with device-memory arenas 8x larger per round
+// Re-runs the n records listed at list_src (device) with device-memory arenas 8x larger per round
 // (starting from 8 x the last tier's vcap/fcap) until none overflows; host-driven (synchronises
 // the stream).  Chunks keep each round's arenas <= 2 GiB.  The first round continues the runs
 // the last LDS tier saved (sus_src, slot = list position); device-memory rounds do not suspend.
@@ -534,10 +728,9 @@ static int rerun_overflows(ContactTiers& T, ncx_ctx* ctx, KArgs a, uint32_t n, c
       b.ovf_cap = T.cap;
       b.sus_load = sus_src ? sus_src + off * sus_bytes : nullptr;
       b.sus_load_bytes = sus_bytes;
-      b.sus_save = nullptr;
-      b.sus_save_bytes = 0;
-      b.sus_save_cap = 0;
-      if ((rc = launch_global_tier(ctx->stream, b, m))) return rc;
+      b.npairs = m;
+      hipLaunchKernelGGL(k_epa_global, dim3((unsigned)m), dim3(64), 0, ctx->stream, b);
+      NCX_HIP_CHECK(hipGetLastError());
     }
     sus_src = nullptr;  // later rounds list this tier's own overflows, with nothing saved
     uint32_t left = 0;
@@ -555,21 +748,22 @@ static int rerun_overflows(ContactTiers& T, ncx_ctx* ctx, KArgs a, uint32_t n, c
   return NCX_OK;
 }
 
-// First-tier kernel variants, the autotuner's choices.  Contact: group width G = 8, 16, 32 lanes
-// per pair with the 44-vertex, 144-face LDS arena (variants 0-2), and G = 8, 16 with the
-// 24-vertex, 80-face arena (variants 3-4); every variant holds 8 pairs per block.  The wide
-// arena's variants differ in occupancy and lanes per pair only; the small arena's hold more pairs
-// per CU and send more pairs to the second tier, which the tuner times with them.  Distance
-// queries need no EPA arena and use 128-thread variants without LDS with 8, 16, 32, 4 or 2 lanes.
+// First-tier kernel variants, the autotuner's choices.  Contact: EPA with G = 8, 16, 32 lanes per
+// record on the 44-vertex arena (variants 0-2), and G = 8, 16 on the 24-vertex arena (variants
+// 3-4); every variant holds 8 records per block.  The small arena's hold more records per CU and
+// send more of them to the second tier, which the tuner times with them.  Distance queries have no
+// arena: 128-thread variants with 8, 16, 32, 4 or 2 lanes per pair.
 static const int T1_NVARIANTS[2] = {NCX_T1_VARIANTS, NCX_T1_VARIANTS};
-// lanes per pair: contact variants 3, 4 are the small-arena ones; distance variants 3, 4 (no
-// arena) take 4 and 2 lanes, for pairs whose supports are closed forms or small hulls
 static const int T1_VARIANT_G[2][NCX_T1_VARIANTS] = {{8, 16, 32, 8, 16}, {8, 16, 32, 4, 2}};
 static const int T1_VARIANT_BS[2][NCX_T1_VARIANTS] = {{64, 128, 256, 64, 128}, {128, 128, 128, 128, 128}};
-// twice the resident blocks (LDS: 4 wide-arena or 7 small-arena blocks per CU; VGPRs: 8 waves).
-// A middle arena (32 vertices, 112 faces, 8 lanes) was never the tuner's choice on the scene's
-// buckets (5.17 / 2.51 / 3.31 ms against 5.04 / 2.13 / 2.81 for the best) and is left out.
-static const unsigned T1_BLOCKS_PER_CU[2][NCX_T1_VARIANTS] = {{8, 8, 4, 14, 8}, {8, 8, 8, 8, 8}};
+// contact: the resident blocks (LDS); distance: twice the resident blocks (VGPRs: 8 waves)
+static const unsigned T1_BLOCKS_PER_CU[2][NCX_T1_VARIANTS] = {{T1_BLOCKS, T1_BLOCKS, T1_BLOCKS, T1S_BLOCKS, T1S_BLOCKS},
+                                                               {8, 8, 8, 8, 8}};
+// Lanes per pair of the GJK kernel by vertex-count bucket: without hulls the supports are closed
+// forms and a group's lanes would only repeat each other.
+static const int GJK_BUCKET_G[NCX_NBUCKETS] = {1, 4, 4, 8};
+#define GJK_BLOCKS_PER_CU 4u
+#define GJK_SMALL_G 8  // batches too small to partition
 
 extern "C" int ncx_shapes_set_tuning(ncx_shapes* s, int query, const int32_t* choice) {
   NCX_REQUIRE(s && choice && (query == 0 || query == 1), "ncx_shapes_set_tuning: bad argument");
@@ -579,34 +773,48 @@ extern "C" int ncx_shapes_set_tuning(ncx_shapes* s, int query, const int32_t* ch
   return NCX_OK;
 }
 
-static int launch_t1(int variant, bool distance, hipStream_t stream, const KArgs& a, unsigned blocks) {
-  if (distance) {
-    switch (variant) {
-      case 0: hipLaunchKernelGGL((k_pairs<8, 128, 0u, 0u, 0u, 0u, 1>), dim3(blocks), dim3(128), 0, stream, a); break;
-      case 2: hipLaunchKernelGGL((k_pairs<32, 128, 0u, 0u, 0u, 0u, 1>), dim3(blocks), dim3(128), 0, stream, a); break;
-      case 3: hipLaunchKernelGGL((k_pairs<4, 128, 0u, 0u, 0u, 0u, 1>), dim3(blocks), dim3(128), 0, stream, a); break;
-      case 4: hipLaunchKernelGGL((k_pairs<2, 128, 0u, 0u, 0u, 0u, 1>), dim3(blocks), dim3(128), 0, stream, a); break;
-      default: hipLaunchKernelGGL((k_pairs<16, 128, 0u, 0u, 0u, 0u, 1>), dim3(blocks), dim3(128), 0, stream, a); break;
-    }
-  } else {
-    switch (variant) {
-      case 0:
-        hipLaunchKernelGGL((k_pairs<8, 64, T1_VC, T1_FC, T1_SC, T1_STC, 0>), dim3(blocks), dim3(64), 0, stream, a);
-        break;
-      case 2:
-        hipLaunchKernelGGL((k_pairs<32, 256, T1_VC, T1_FC, T1_SC, T1_STC, 0>), dim3(blocks), dim3(256), 0, stream, a);
-        break;
-      case 3:
-        hipLaunchKernelGGL((k_pairs<8, 64, T1S_VC, T1S_FC, T1S_SC, T1S_STC, 0>), dim3(blocks), dim3(64), 0, stream, a);
-        break;
-      case 4:
-        hipLaunchKernelGGL((k_pairs<16, 128, T1S_VC, T1S_FC, T1S_SC, T1S_STC, 0>), dim3(blocks), dim3(128), 0, stream,
-                           a);
-        break;
-      default:
-        hipLaunchKernelGGL((k_pairs<16, 128, T1_VC, T1_FC, T1_SC, T1_STC, 0>), dim3(blocks), dim3(128), 0, stream, a);
-        break;
-    }
+static unsigned capped_blocks(ncx_ctx* ctx, unsigned per_cu, size_t n, size_t per_block) {
+  return (unsigned)std::max<size_t>(1, std::min<size_t>((size_t)ctx->num_cus * per_cu, (n + per_block - 1) / per_block));
+}
+
+static int launch_distance(int variant, ncx_ctx* ctx, const KArgs& a, size_t n) {
+  const unsigned blocks = capped_blocks(ctx, T1_BLOCKS_PER_CU[1][variant], n,
+                                        (size_t)T1_VARIANT_BS[1][variant] / T1_VARIANT_G[1][variant]);
+  switch (variant) {
+    case 0: hipLaunchKernelGGL((k_distance<8, 128>), dim3(blocks), dim3(128), 0, ctx->stream, a); break;
+    case 2: hipLaunchKernelGGL((k_distance<32, 128>), dim3(blocks), dim3(128), 0, ctx->stream, a); break;
+    case 3: hipLaunchKernelGGL((k_distance<4, 128>), dim3(blocks), dim3(128), 0, ctx->stream, a); break;
+    case 4: hipLaunchKernelGGL((k_distance<2, 128>), dim3(blocks), dim3(128), 0, ctx->stream, a); break;
+    default: hipLaunchKernelGGL((k_distance<16, 128>), dim3(blocks), dim3(128), 0, ctx->stream, a); break;
+  }
+  NCX_HIP_CHECK(hipGetLastError());
+  return NCX_OK;
+}
+
+// GJK over at most n pairs with G lanes each, then the first-tier EPA variant over its records
+// (work counters `work` and `epa_work`).
+static int launch_contact_t1(int variant, int G, ncx_ctx* ctx, const KArgs& a, size_t n, uint32_t* work,
+                             uint32_t* epa_work) {
+  KArgs g = a;
+  g.work = work;
+  const unsigned gb = capped_blocks(ctx, GJK_BLOCKS_PER_CU, n, GJK_BS / G);
+  switch (G) {
+    case 1: hipLaunchKernelGGL(k_contact_gjk<1>, dim3(gb), dim3(GJK_BS), 0, ctx->stream, g); break;
+    case 4: hipLaunchKernelGGL(k_contact_gjk<4>, dim3(gb), dim3(GJK_BS), 0, ctx->stream, g); break;
+    case 8: hipLaunchKernelGGL(k_contact_gjk<8>, dim3(gb), dim3(GJK_BS), 0, ctx->stream, g); break;
+    default: hipLaunchKernelGGL(k_contact_gjk<16>, dim3(gb), dim3(GJK_BS), 0, ctx->stream, g); break;
+  }
+  NCX_HIP_CHECK(hipGetLastError());
+  KArgs e = a;
+  e.work = epa_work;
+  const unsigned eb = capped_blocks(ctx, T1_BLOCKS_PER_CU[0][variant], n, 8);
+  const dim3 bs(T1_VARIANT_BS[0][variant]);
+  switch (variant) {
+    case 0: hipLaunchKernelGGL((k_epa<8, 64, ArenaT1, 2, true, false>), dim3(eb), bs, 0, ctx->stream, e); break;
+    case 2: hipLaunchKernelGGL((k_epa<32, 256, ArenaT1, 1, true, false>), dim3(eb), bs, 0, ctx->stream, e); break;
+    case 3: hipLaunchKernelGGL((k_epa<8, 64, ArenaT1S, 2, true, false>), dim3(eb), bs, 0, ctx->stream, e); break;
+    case 4: hipLaunchKernelGGL((k_epa<16, 128, ArenaT1S, 2, true, false>), dim3(eb), bs, 0, ctx->stream, e); break;
+    default: hipLaunchKernelGGL((k_epa<16, 128, ArenaT1, 2, true, false>), dim3(eb), bs, 0, ctx->stream, e); break;
   }
   NCX_HIP_CHECK(hipGetLastError());
   return NCX_OK;
@@ -614,76 +822,49 @@ static int launch_t1(int variant, bool distance, hipStream_t stream, const KArgs
 
 // Saved-run buffers of LDS tier `tier` (0 = T1): it continues the runs T(tier) saved and saves
 // its own suspended runs for the next tier.
+static uint8_t* sus_slots(const ContactTiers& T, int tier) { return tier == 0 ? T.sus0 : T.sus[tier].as<uint8_t>(); }
+
 static void set_sus(ContactTiers& T, KArgs& b, int tier) {
-  b.sus_load = tier > 0 ? T.sus[tier - 1].as<uint8_t>() : nullptr;
+  b.sus_load = tier > 0 ? sus_slots(T, tier - 1) : nullptr;
   b.sus_load_bytes = tier > 0 ? SUS_BYTES[tier - 1] : 0;
-  b.sus_save = T.sus[tier].as<uint8_t>();
+  b.sus_save = sus_slots(T, tier);
   b.sus_save_bytes = SUS_BYTES[tier];
-  b.sus_save_cap = T.sus[tier].p ? SUS_CAP[tier] : 0u;
+  b.sus_save_cap = tier == 0 ? T.sus0_cap : SUS_CAP[tier];
 }
 
-// T2 over the device-counted T1 overflow list.
-static KArgs t2_args(ContactTiers& T, const KArgs& a) {
+// Tier t (1 = T2, ...) over the device-counted overflow list of the tier before it.
+static KArgs tier_args(ContactTiers& T, const KArgs& a, int t) {
   uint32_t* ovf = T.ovf.as<uint32_t>();
+  uint32_t* const counts[4] = {ovf + NCX_OVF_T1_COUNT, ovf + NCX_OVF_T2_COUNT, ovf + NCX_OVF_T3_COUNT,
+                               ovf + NCX_OVF_T4_COUNT};
+  uint32_t* const lists[4] = {T.t1_list(), T.t2_list(), T.t3_list(), T.t4_list()};
+  const uint32_t works[4] = {0, NCX_WORK_T2, NCX_WORK_T3, NCX_WORK_T4};
   KArgs b = a;
   b.range_b = nullptr;
   b.range_e = nullptr;
-  b.list = T.t1_list();
-  b.n_dev = ovf + NCX_OVF_T1_COUNT;
-  b.npairs = T.cap;
-  b.vcap = T2_VC;
-  b.fcap = T2_FC;
-  b.ovf_count = ovf + NCX_OVF_T2_COUNT;
-  b.ovf_list = T.t2_list();
-  b.work = ncx_work_set(ovf, NCX_WORK_T2);
-  set_sus(T, b, 1);
+  b.rec_base = nullptr;
+  b.list = lists[t - 1];
+  b.n_dev = counts[t - 1];
+  b.ovf_count = counts[t];
+  b.ovf_list = lists[t];
+  b.work = ncx_work_set(ovf, works[t]);
+  set_sus(T, b, t);
   return b;
 }
 
-// T3 over the device-counted T2 overflow list: 64 lanes and one pair per block, with a
-// 512-vertex, 1600-face LDS arena (51 KiB).
-static KArgs t3_args(ContactTiers& T, const KArgs& a) {
-  uint32_t* ovf = T.ovf.as<uint32_t>();
-  KArgs b = t2_args(T, a);
-  b.list = T.t2_list();
-  b.n_dev = ovf + NCX_OVF_T2_COUNT;
-  b.vcap = T3_VC;
-  b.fcap = T3_FC;
-  b.ovf_count = ovf + NCX_OVF_T3_COUNT;
-  b.ovf_list = T.t3_list();
-  b.work = ncx_work_set(ovf, NCX_WORK_T3);
-  set_sus(T, b, 2);
-  return b;
-}
-
-// T4 over the device-counted T3 overflow list: one pair per 64-thread block with the largest
-// LDS arena a workgroup may hold.
-static KArgs t4_args(ContactTiers& T, const KArgs& a) {
-  uint32_t* ovf = T.ovf.as<uint32_t>();
-  KArgs b = t3_args(T, a);
-  b.list = T.t3_list();
-  b.n_dev = ovf + NCX_OVF_T3_COUNT;
-  b.vcap = T4_VC;
-  b.fcap = T4_FC;
-  b.ovf_count = ovf + NCX_OVF_T4_COUNT;
-  b.ovf_list = T.t4_list();
-  b.work = ncx_work_set(ovf, NCX_WORK_T4);
-  set_sus(T, b, 3);
-  return b;
-}
-
-static int launch_t2(ncx_ctx* ctx, ContactTiers& T, const KArgs& a) {
-  KArgs b = t2_args(T, a);
-  hipLaunchKernelGGL((k_pairs<T2_G, T2_BS, T2_VC, T2_FC, T2_SC, T2_STC, 0>), dim3(ctx->num_cus * T2_BLOCKS_PER_CU), dim3(T2_BS), 0,
-                     ctx->stream, b);
+// T2 to T4 after the first tier of about n pairs.  The grids are persistent, so any size is right:
+// about one pair in twenty is taken to reach T2, one in 400 T3 and one in 4,000 T4, because the
+// blocks of an empty launch cost time too (16 us for 1,280 blocks of 30 KB).
+static int launch_upper_tiers(ncx_ctx* ctx, ContactTiers& T, const KArgs& a, size_t n) {
+  hipLaunchKernelGGL((k_epa<T2_G, T2_BS, ArenaT2, 2, true, true>),
+                     dim3(capped_blocks(ctx, T2_BLOCKS_PER_CU, n, 20 * (T2_BS / T2_G))), dim3(T2_BS), 0, ctx->stream,
+                     tier_args(T, a, 1));
   NCX_HIP_CHECK(hipGetLastError());
-  KArgs c = t3_args(T, a);
-  hipLaunchKernelGGL((k_pairs<64, 64, T3_VC, T3_FC, T3_SC, T3_STC, 0>), dim3(ctx->num_cus * 3), dim3(64), 0,
-                     ctx->stream, c);
+  hipLaunchKernelGGL((k_epa<64, 64, ArenaT3, 1, true, true>), dim3(capped_blocks(ctx, T3_BLOCKS_PER_CU, n, 400)), dim3(64),
+                     0, ctx->stream, tier_args(T, a, 2));
   NCX_HIP_CHECK(hipGetLastError());
-  KArgs d = t4_args(T, a);
-  hipLaunchKernelGGL((k_pairs<64, 64, T4_VC, T4_FC, T4_SC, T4_STC, 0>), dim3(ctx->num_cus), dim3(64), 0,
-                     ctx->stream, d);
+  hipLaunchKernelGGL((k_epa<64, 64, ArenaT4, 1, true, true>), dim3(capped_blocks(ctx, 1u, n, 4000)), dim3(64), 0,
+                     ctx->stream, tier_args(T, a, 3));
   NCX_HIP_CHECK(hipGetLastError());
   return NCX_OK;
 }
@@ -709,8 +890,9 @@ int contact_tiers_reserve_list(ContactTiers& t, size_t npairs) {
 static int clear_tier_counters(ncx_ctx* ctx, uint32_t* hdr) {
   int rc = fill_u32(ctx, hdr, NCX_OVF_TIER_WORDS, 0u);
   if (rc) return rc;
-  static_assert(NCX_WORK_TUNE == 0 && NCX_WORK_T2 == 1 && NCX_WORK_T3 == 2 && NCX_WORK_T4 == 3, "work sets");
-  return fill_u32(ctx, ncx_work_set(hdr, 0), 4 * NCX_WORK_SET, 0u);
+  static_assert(NCX_WORK_TUNE == 0 && NCX_WORK_T2 == 1 && NCX_WORK_T3 == 2 && NCX_WORK_T4 == 3 && NCX_WORK_TUNE_EPA == 4,
+                "work sets");
+  return fill_u32(ctx, ncx_work_set(hdr, 0), 5 * NCX_WORK_SET, 0u);
 }
 
 #define TUNE_MIN_PAIRS 4096u
@@ -738,7 +920,7 @@ static int autotune(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, const KArgs& b
   NCX_HIP_CHECK(hipEventCreate(&e1));
   for (int b = 0; b < NCX_NBUCKETS; ++b) {
     const uint32_t cnt = rng[2 * b + 1] - rng[2 * b];
-    if (S->tune[mode][b] >= 0 || cnt < TUNE_MIN_PAIRS) continue;
+    if (S->tune[mode][b] >= 0 || cnt < (size_t)TUNE_MIN_PAIRS) continue;
     const uint32_t ns = std::min(cnt, TUNE_SAMPLE);
     hipLaunchKernelGGL(k_tune_sample, dim3(ceil_div(ns, 256)), dim3(256), 0, ctx->stream, base.list, rng[2 * b],
                        cnt / ns, ns, smp.as<uint32_t>());
@@ -756,11 +938,14 @@ static int autotune(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, const KArgs& b
         a.range_b = dr.as<uint32_t>();
         a.range_e = dr.as<uint32_t>() + 1;
         a.work = ncx_work_set(hdr, NCX_WORK_TUNE);
+        a.rec_count = hdr + NCX_REC_COUNT_TUNE;
         if ((rc = clear_tier_counters(ctx, hdr))) break;
         NCX_HIP_CHECK(hipEventRecord(e0, ctx->stream));
-        if ((rc = launch_t1(v, mode == 1, ctx->stream, a, (unsigned)ctx->num_cus * T1_BLOCKS_PER_CU[mode][v]))) break;
+        if (mode == 1) rc = launch_distance(v, ctx, a, ns);
+        else rc = launch_contact_t1(v, GJK_BUCKET_G[b], ctx, a, ns, a.work, ncx_work_set(hdr, NCX_WORK_TUNE_EPA));
+        if (rc) break;
         // the variant's first-tier overflows cost a second-tier run: time it too
-        if (mode == 0 && (rc = launch_t2(ctx, T, a))) break;
+        if (mode == 0 && (rc = launch_upper_tiers(ctx, T, a, ns))) break;
         NCX_HIP_CHECK(hipEventRecord(e1, ctx->stream));
         NCX_HIP_CHECK(hipEventSynchronize(e1));
         float ms = 0.f;
@@ -803,21 +988,25 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
   a.nshapes = (uint32_t)S->n;
   a.bad_index = ovf + NCX_OVF_BAD;
   a.arena = nullptr;
-  a.vcap = T1_VC;
-  a.fcap = T1_FC;
+  a.vcap = ArenaT4::VC;
+  a.fcap = ArenaT4::FC;
+  a.rec = T.rec;
+  a.rec_base = nullptr;
+  a.sup = T.sup;
   a.ovf_count = ovf + NCX_OVF_T1_COUNT;
   a.ovf_list = T.t1_list();
   a.ovf_cap = T.cap;
   set_sus(T, a, 0);
   a.range_b = nullptr;
   a.range_e = nullptr;
+  // a device-counted call's likely number of pairs, for grid sizes
+  const size_t likely = n_dev ? std::min(npairs, 16 * S->n) : npairs;
   bool untuned = false;
   for (int b = 0; b < NCX_NBUCKETS; ++b) untuned = untuned || S->tune[mode][b] < 0;
-  const bool tune_now = may_tune && untuned;
-  bool same = true;  // one variant for every bucket
-  for (int b = 1; b < NCX_NBUCKETS; ++b) same = same && S->tune[mode][b] == S->tune[mode][0];
-  // Partition (sort by key) unless the batch is small and needs no per-bucket variants.
-  const bool partition = tune_now || !same || npairs >= PARTITION_MIN_PAIRS;
+  const bool tune_now = may_tune && untuned && npairs >= TUNE_MIN_PAIRS;
+  // Partition (sort by key) unless the batch is small: below 16,384 pairs the three partition
+  // kernels and the launches per bucket cost more (about 60 us) than the order saves.
+  const bool partition = tune_now || npairs >= PARTITION_MIN_PAIRS;
   if (partition) {
     // partition the pair indices by sort key (vertex-count bucket, then type pair)
     if ((rc = contact_tiers_reserve_list(T, npairs))) return rc;
@@ -825,7 +1014,7 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
     hipLaunchKernelGGL(k_bucket_count, dim3(bblocks), dim3(BKT_BLOCK), 0, ctx->stream, a.ia, a.ib, a.shapes,
                        a.nshapes, a.poses, npairs, n_dev, ovf, T.bkey.as<uint32_t>());
     NCX_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_bucket_offsets, dim3(1), dim3(1), 0, ctx->stream, ovf);
+    hipLaunchKernelGGL(k_bucket_offsets, dim3(1), dim3(NCX_NKEYS), 0, ctx->stream, ovf);
     NCX_HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(k_bucket_scatter, dim3(bblocks), dim3(BKT_BLOCK), 0, ctx->stream, T.bkey.as<uint32_t>(),
                        npairs, n_dev, ovf, T.blist.as<uint32_t>());
@@ -838,22 +1027,28 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
   }
   if (!partition) {
     // one launch over all pairs, in their own order
-    const int v = S->tune[mode][0] >= 0 ? S->tune[mode][0] : 1;
+    const int big = 31 - __builtin_clz(S->buckets | 1u);  // the variant of the set's largest hulls
+    const int v = S->tune[mode][big] >= 0 ? S->tune[mode][big] : 1;
     KArgs ab = a;
     ab.list = nullptr;
     ab.n_dev = n_dev;
     ab.npairs = npairs;
     ab.work = ncx_work_set(ovf, NCX_WORK_BKT);
-    unsigned blocks = (unsigned)ctx->num_cus * T1_BLOCKS_PER_CU[mode][v];
-    if (!n_dev)
-      blocks = std::max(1u, std::min<unsigned>(blocks, ceil_div(npairs * T1_VARIANT_G[mode][v], T1_VARIANT_BS[mode][v])));
-    if ((rc = launch_t1(v, mode == 1, ctx->stream, ab, blocks))) return rc;
+    ab.rec_count = ovf + NCX_REC_COUNT;
+    if (mode == 1) rc = launch_distance(v, ctx, ab, npairs);
+    else rc = launch_contact_t1(v, GJK_SMALL_G, ctx, ab, likely, ab.work, ncx_work_set(ovf, NCX_WORK_EPA));
+    if (rc) return rc;
   } else {
-    // one launch per run of consecutive buckets sharing a variant, over the partitioned list
+    // distance: one launch per run of consecutive buckets sharing a variant, over the partitioned
+    // list; contact: one GJK and one EPA launch per bucket, its records from its own range on
     for (int b0 = 0; b0 < NCX_NBUCKETS;) {
+      if (mode == 0 && !(S->buckets >> b0 & 1u)) {  // no shape of the set makes such a pair
+        ++b0;
+        continue;
+      }
       const int v = S->tune[mode][b0] >= 0 ? S->tune[mode][b0] : 1;
       int b1 = b0;
-      while (b1 + 1 < NCX_NBUCKETS && (S->tune[mode][b1 + 1] >= 0 ? S->tune[mode][b1 + 1] : 1) == v) ++b1;
+      while (mode == 1 && b1 + 1 < NCX_NBUCKETS && (S->tune[mode][b1 + 1] >= 0 ? S->tune[mode][b1 + 1] : 1) == v) ++b1;
       KArgs ab = a;
       ab.list = T.blist.as<uint32_t>();
       ab.n_dev = nullptr;
@@ -861,16 +1056,17 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
       ab.range_b = ovf + NCX_BKT_RANGE + 2 * b0;
       ab.range_e = ovf + NCX_BKT_RANGE + 2 * b1 + 1;
       ab.work = ncx_work_set(ovf, NCX_WORK_BKT + b0);
-      unsigned blocks = (unsigned)ctx->num_cus * T1_BLOCKS_PER_CU[mode][v];
-      if (!n_dev)
-        blocks = std::max(1u, std::min<unsigned>(blocks, ceil_div(npairs * T1_VARIANT_G[mode][v], T1_VARIANT_BS[mode][v])));
-      if ((rc = launch_t1(v, mode == 1, ctx->stream, ab, blocks))) return rc;
+      ab.rec_base = ab.range_b;
+      ab.rec_count = ovf + NCX_REC_COUNT + b0;
+      if (mode == 1) rc = launch_distance(v, ctx, ab, npairs);
+      else rc = launch_contact_t1(v, GJK_BUCKET_G[b0], ctx, ab, likely, ab.work, ncx_work_set(ovf, NCX_WORK_EPA + b0));
+      if (rc) return rc;
       b0 = b1 + 1;
     }
   }
-  if (mode == 0 && (rc = launch_t2(ctx, T, a))) return rc;
+  if (mode == 0 && (rc = launch_upper_tiers(ctx, T, a, likely))) return rc;
   if (!T.last) T.last = new KArgs;
-  *T.last = t4_args(T, a);
+  *T.last = tier_args(T, a, 3);
   return NCX_OK;
 }
 
@@ -912,14 +1108,14 @@ int contacts_resolve_overflow(ContactTiers& T, ncx_ctx* ctx, size_t* n_large) {
     return NCX_E_CAPACITY;
   }
   if (n_large) *n_large = hdr[NCX_OVF_T1_COUNT];
-  return rerun_overflows(T, ctx, *T.last, hdr[NCX_OVF_T4_COUNT], T.t4_list(), T4_VC, T4_FC, T.sus[3].as<uint8_t>(),
+  return rerun_overflows(T, ctx, *T.last, hdr[NCX_OVF_T4_COUNT], T.t4_list(), ArenaT4::VC, ArenaT4::FC, T.sus[3].as<uint8_t>(),
                          SUS_BYTES[3]);
 }
 
 static int run_pairs(ncx_shapes* S, KArgs a, size_t npairs) {
   if (npairs == 0) return NCX_OK;
   int rc;
-  if ((rc = contact_tiers_reserve(S->tiers, npairs))) return rc;
+  if ((rc = contact_tiers_reserve(S->tiers, S->ctx, npairs, a.distance_mode ? 0 : npairs))) return rc;
   if ((rc = launch_tiers(S, S->tiers, S->ctx, a, npairs, nullptr, true))) return rc;
   return contacts_resolve_overflow(S->tiers, S->ctx, nullptr);
 }

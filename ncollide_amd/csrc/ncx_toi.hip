@@ -69,7 +69,7 @@ __device__ __forceinline__ TOIOut toi_pair(const iso& m1, f3 v1, const ShapeD& g
   c.m1 = m1; c.m2 = m2; c.g1 = g1; c.g2 = g2;
   c.dil = target;
   c.dilated = target != 0.f;
-  Simplex s;
+  SimplexR s;
   sx_init(s);
   float t;
   f3 normal;
@@ -97,9 +97,7 @@ __device__ __forceinline__ TOIOut toi_pair(const iso& m1, f3 v1, const ShapeD& g
     float nl;
     if (!try_normalize(normal, NCX_FLT_EPS, &d, &nl)) d = f3{1.f, 0.f, 0.f};
     Simplex s2;
-    sx_init(s2);
-    sx_reset(s2, cso_from<G>(c2, d, P, gl));
-    GJKOut r = gjk<G>(c2, target, s2, P, gl, 10000);
+    GJKOut r = gjk<G>(c2, d, target, s2, P, gl, 10000);
     if (r.status == GJK_S_CLOSEST) {
       const f3 nn = normalize(r.p2 - r.p1);
       o.n1 = inv_xform_vec(m1, nn);
