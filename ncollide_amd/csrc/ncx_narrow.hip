@@ -524,16 +524,16 @@ __device__ __forceinline__ uint32_t pair_key(const ncx_shape* __restrict__ shape
   return 16u * NCX_OVERLAP_BINS * b + NCX_OVERLAP_BINS * (4u * (t1 < t2 ? t1 : t2) + (t1 < t2 ? t2 : t1)) + o;
 }
 
-// Bounding radius of each shape about its local origin, into pad[0] of its device record (a
-// sort heuristic only: nothing else reads it).
+// Bounding radius of each shape about its local origin, into pad[0] of its device record, for the
+// sort key and the mesh distance search's bounds.
 __global__ __launch_bounds__(256) void k_shape_radius(ncx_shape* __restrict__ shapes, size_t n, Pool P) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const ncx_shape s = shapes[i];
   float r = 0.f;
-  if (s.type == NCX_BALL) r = s.p0;
+  if (s.type == NCX_BALL) r = fabsf(s.p0);
   else if (s.type == NCX_CUBOID) r = __builtin_sqrtf(s.p0 * s.p0 + s.p1 * s.p1 + s.p2 * s.p2);
-  else if (s.type == NCX_CAPSULE) r = s.p0 + s.p1;
+  else if (s.type == NCX_CAPSULE) r = fabsf(s.p0) + fabsf(s.p1);
   else {
     for (uint32_t k = 0; k < s.hull_count; ++k) {
       const uint32_t j = s.hull_offset + k;
