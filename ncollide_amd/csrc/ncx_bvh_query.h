@@ -92,6 +92,8 @@ template <int K, bool WRITE>
 __global__ __launch_bounds__(BQ_BLOCK) void k_bq_collect(BQArgs a) {
   const uint32_t qi = blockIdx.x * BQ_BLOCK + threadIdx.x;
   if (qi >= a.nq) return;
+  __shared__ float snaps[K == BQ_RAY ? BQ_BLOCK : 1][RC_SNAP];
+  float* const snap = snaps[K == BQ_RAY ? threadIdx.x : 0];
   const int nq = K == BQ_POINT ? 3 : 6;
   float qv[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   for (int d = 0; d < nq; ++d) qv[d] = a.q[d][qi];
@@ -105,7 +107,7 @@ __global__ __launch_bounds__(BQ_BLOCK) void k_bq_collect(BQArgs a) {
     if (K == BQ_RAY && a.cast_shapes) {
       uint32_t feat;
       if (!shape_ray_cast<1>(load_shape(a.shapes, h), load_pose(a.poses, h), f3{qv[0], qv[1], qv[2]},
-                             f3{qv[3], qv[4], qv[5]}, a.max_toi, true, a.P, 0, t, n, feat))
+                             f3{qv[3], qv[4], qv[5]}, a.max_toi, true, a.P, 0, snap, t, n, feat))
         return;
     }
     if (WRITE) {
@@ -162,6 +164,8 @@ template <int G>
 static __global__ __launch_bounds__(BQ_BLOCK) void k_bq_first_ray(BQArgs a) {
   const uint32_t gi = (blockIdx.x * BQ_BLOCK + threadIdx.x) / G;
   const int gl = threadIdx.x % G;
+  __shared__ float snaps[BQ_BLOCK / G][RC_SNAP];
+  float* const snap = snaps[threadIdx.x / G];
   if (gi >= a.nq) return;  // whole groups: BQ_BLOCK is a multiple of G
   const uint32_t qi = a.perm ? a.perm[gi] : gi;
   float qv[6];
@@ -175,8 +179,8 @@ static __global__ __launch_bounds__(BQ_BLOCK) void k_bq_first_ray(BQArgs a) {
     float t;
     f3 n;
     uint32_t feat;
-    if (shape_ray_cast<G>(load_shape(a.shapes, h), load_pose(a.poses, h), o, dir, a.max_toi, true, a.P, gl, t, n,
-                          feat)) {
+    if (shape_ray_cast<G>(load_shape(a.shapes, h), load_pose(a.poses, h), o, dir, a.max_toi, true, a.P, gl, snap, t,
+                          n, feat)) {
       if (t < best_t || (t == best_t && h < best_h)) {
         best_t = t;
         best_h = h;

@@ -209,17 +209,24 @@ struct Loc {
   float bc0, bc1, bc2;
 };
 
+// xform_pt(iso_identity(), v), bit for bit, without its products by zero: they add +0 to finite
+// components (which turns -0 into +0) and make all three NaN when one is infinite or NaN.
+__device__ __forceinline__ f3 ident_pt(f3 v) {
+  const float z = ((0.f * v.x + 0.f * v.y) + 0.f * v.z) + 0.f;
+  return f3{v.x + z, v.y + z, v.z + z};
+}
+
 // point_segment.rs:52-91 (identity isometry, point = origin)
 __device__ __forceinline__ f3 proj_segment(f3 a, f3 b, Loc& loc) {
   iso m = iso_identity();
   f3 ls = inv_xform_pt(m, f3{0.f, 0.f, 0.f});
   f3 ab = b - a, ap = ls - a;
   float ab_ap = dot(ab, ap), sqnab = norm_sq(ab);
-  if (ab_ap <= 0.f) { loc.kind = LOC_VERTEX; loc.id = 0; return xform_pt(m, a); }
-  if (ab_ap >= sqnab) { loc.kind = LOC_VERTEX; loc.id = 1; return xform_pt(m, b); }
+  if (ab_ap <= 0.f) { loc.kind = LOC_VERTEX; loc.id = 0; return ident_pt(a); }
+  if (ab_ap >= sqnab) { loc.kind = LOC_VERTEX; loc.id = 1; return ident_pt(b); }
   float u = ab_ap / sqnab;
   loc.kind = LOC_EDGE; loc.id = 0; loc.bc0 = 1.f - u; loc.bc1 = u;
-  return xform_pt(m, a + ab * u);
+  return ident_pt(a + ab * u);
 }
 
 // point_triangle.rs:61-309, dim3, solid = true
@@ -229,46 +236,46 @@ __device__ __forceinline__ f3 proj_triangle(f3 a, f3 b, f3 c, Loc& loc) {
   f3 p = inv_xform_pt(m, o);
   f3 ab = b - a, ac = c - a, ap = p - a;
   float ab_ap = dot(ab, ap), ac_ap = dot(ac, ap);
-  if (ab_ap <= 0.f && ac_ap <= 0.f) { loc.kind = LOC_VERTEX; loc.id = 0; return xform_pt(m, a); }
+  if (ab_ap <= 0.f && ac_ap <= 0.f) { loc.kind = LOC_VERTEX; loc.id = 0; return ident_pt(a); }
   f3 bp = p - b;
   float ab_bp = dot(ab, bp), ac_bp = dot(ac, bp);
-  if (ab_bp >= 0.f && ac_bp <= ab_bp) { loc.kind = LOC_VERTEX; loc.id = 1; return xform_pt(m, b); }
+  if (ab_bp >= 0.f && ac_bp <= ab_bp) { loc.kind = LOC_VERTEX; loc.id = 1; return ident_pt(b); }
   f3 cp = p - c;
   float ab_cp = dot(ab, cp), ac_cp = dot(ac, cp);
-  if (ac_cp >= 0.f && ab_cp <= ac_cp) { loc.kind = LOC_VERTEX; loc.id = 2; return xform_pt(m, c); }
+  if (ac_cp >= 0.f && ab_cp <= ac_cp) { loc.kind = LOC_VERTEX; loc.id = 2; return ident_pt(c); }
   f3 bc = c - b;
   f3 n = cross(ab, ac);
   float vc = dot(n, cross(ab, ap));
   if (vc < 0.f && ab_ap >= 0.f && ab_bp <= 0.f) {
     float v = ab_ap / norm_sq(ab);
     loc.kind = LOC_EDGE; loc.id = 0; loc.bc0 = 1.f - v; loc.bc1 = v;
-    return xform_pt(m, a + ab * v);
+    return ident_pt(a + ab * v);
   }
   float vb = -dot(n, cross(ac, cp));
   if (vb < 0.f && ac_ap >= 0.f && ac_cp <= 0.f) {
     float w = ac_ap / norm_sq(ac);
     loc.kind = LOC_EDGE; loc.id = 2; loc.bc0 = 1.f - w; loc.bc1 = w;
-    return xform_pt(m, a + ac * w);
+    return ident_pt(a + ac * w);
   }
   float va = dot(n, cross(bc, bp));
   if (va < 0.f && ac_bp - ab_bp >= 0.f && ab_cp - ac_cp >= 0.f) {
     float w = dot(bc, bp) / norm_sq(bc);
     loc.kind = LOC_EDGE; loc.id = 1; loc.bc0 = 1.f - w; loc.bc1 = w;
-    return xform_pt(m, b + bc * w);
+    return ident_pt(b + bc * w);
   }
   int clockwise = dot(n, ap) >= 0.f ? 0 : 1;
   if (va + vb + vc != 0.f) {
     float denom = 1.f / (va + vb + vc);
     float v = vb * denom, w = vc * denom;
     loc.kind = LOC_FACE; loc.id = clockwise; loc.bc0 = 1.f - v - w; loc.bc1 = v; loc.bc2 = w;
-    return xform_pt(m, a + ab * v + ac * w);
+    return ident_pt(a + ab * v + ac * w);
   }
   loc.kind = LOC_SOLID; loc.id = 0;
   return o;
 }
 
 // check_edge of point_tetrahedron.rs:106-152
-__device__ __forceinline__ bool tet_edge(int i, const iso& m, f3 a, f3 nabc, f3 nabd, f3 ap, f3 ab, float ap_ab,
+__device__ __forceinline__ bool tet_edge(int i, f3 a, f3 nabc, f3 nabd, f3 ap, f3 ab, float ap_ab,
                                          float bp_ab, float& dabc, float& dabd, Loc& loc, f3& out) {
   float ab_ab = ap_ab - bp_ab;
   f3 ap_x_ab = cross(ap, ab);
@@ -277,14 +284,14 @@ __device__ __forceinline__ bool tet_edge(int i, const iso& m, f3 a, f3 nabc, f3 
   if (ab_ab != 0.f && dabc >= 0.f && dabd >= 0.f && ap_ab >= 0.f && ap_ab <= ab_ab) {
     float u = ap_ab / ab_ab;
     loc.kind = LOC_EDGE; loc.id = i; loc.bc0 = 1.f - u; loc.bc1 = u;
-    out = xform_pt(m, a + ab * u);
+    out = ident_pt(a + ab * u);
     return true;
   }
   return false;
 }
 
 // check_face of point_tetrahedron.rs:251-306
-__device__ __forceinline__ bool tet_face(int i, const iso& m, f3 a, f3 b, f3 c, f3 ap, f3 bp, f3 cp, f3 ab, f3 ac,
+__device__ __forceinline__ bool tet_face(int i, f3 a, f3 b, f3 c, f3 ap, f3 bp, f3 cp, f3 ab, f3 ac,
                                          f3 ad, float d1, float d2, float d3, Loc& loc, f3& out) {
   if (d1 < 0.f && d2 < 0.f && d3 < 0.f) {
     f3 n = cross(ab, ac);
@@ -299,7 +306,7 @@ __device__ __forceinline__ bool tet_face(int i, const iso& m, f3 a, f3 b, f3 c, 
       float inv_denom = 1.f / denom;
       float b0 = va * inv_denom, b1 = vb * inv_denom, b2 = vc * inv_denom;
       loc.kind = LOC_FACE; loc.id = i; loc.bc0 = b0; loc.bc1 = b1; loc.bc2 = b2;
-      out = xform_pt(m, a * b0 + b * b1 + c * b2);
+      out = ident_pt(a * b0 + b * b1 + c * b2);
       return true;
     }
   }
@@ -312,31 +319,31 @@ __device__ __forceinline__ f3 proj_tetrahedron(f3 A, f3 B, f3 C, f3 D, Loc& loc)
   f3 p = inv_xform_pt(m, f3{0.f, 0.f, 0.f});
   f3 ab = B - A, ac = C - A, ad = D - A, ap = p - A;
   float ap_ab = dot(ap, ab), ap_ac = dot(ap, ac), ap_ad = dot(ap, ad);
-  if (ap_ab <= 0.f && ap_ac <= 0.f && ap_ad <= 0.f) { loc.kind = LOC_VERTEX; loc.id = 0; return xform_pt(m, A); }
+  if (ap_ab <= 0.f && ap_ac <= 0.f && ap_ad <= 0.f) { loc.kind = LOC_VERTEX; loc.id = 0; return ident_pt(A); }
   f3 bc = C - B, bd = D - B, bp = p - B;
   float bp_bc = dot(bp, bc), bp_bd = dot(bp, bd), bp_ab = dot(bp, ab);
-  if (bp_bc <= 0.f && bp_bd <= 0.f && bp_ab >= 0.f) { loc.kind = LOC_VERTEX; loc.id = 1; return xform_pt(m, B); }
+  if (bp_bc <= 0.f && bp_bd <= 0.f && bp_ab >= 0.f) { loc.kind = LOC_VERTEX; loc.id = 1; return ident_pt(B); }
   f3 cd = D - C, cp = p - C;
   float cp_ac = dot(cp, ac), cp_bc = dot(cp, bc), cp_cd = dot(cp, cd);
-  if (cp_cd <= 0.f && cp_bc >= 0.f && cp_ac >= 0.f) { loc.kind = LOC_VERTEX; loc.id = 2; return xform_pt(m, C); }
+  if (cp_cd <= 0.f && cp_bc >= 0.f && cp_ac >= 0.f) { loc.kind = LOC_VERTEX; loc.id = 2; return ident_pt(C); }
   f3 dp = p - D;
   float dp_cd = dot(dp, cd), dp_bd = dot(dp, bd), dp_ad = dot(dp, ad);
-  if (dp_ad >= 0.f && dp_bd >= 0.f && dp_cd >= 0.f) { loc.kind = LOC_VERTEX; loc.id = 3; return xform_pt(m, D); }
+  if (dp_ad >= 0.f && dp_bd >= 0.f && dp_cd >= 0.f) { loc.kind = LOC_VERTEX; loc.id = 3; return ident_pt(D); }
   f3 out;
   float dabc, dabd, dacd, dacb, dadb, dadc, dbca, dbcd, dbdc, dbda, dcda, dcdb;
   f3 nabc = cross(ab, ac), nabd = cross(ab, ad);
-  if (tet_edge(0, m, A, nabc, nabd, ap, ab, ap_ab, bp_ab, dabc, dabd, loc, out)) return out;
+  if (tet_edge(0, A, nabc, nabd, ap, ab, ap_ab, bp_ab, dabc, dabd, loc, out)) return out;
   f3 nacd = cross(ac, ad);
-  if (tet_edge(1, m, A, nacd, -nabc, ap, ac, ap_ac, cp_ac, dacd, dacb, loc, out)) return out;
-  if (tet_edge(2, m, A, -nabd, -nacd, ap, ad, ap_ad, dp_ad, dadb, dadc, loc, out)) return out;
+  if (tet_edge(1, A, nacd, -nabc, ap, ac, ap_ac, cp_ac, dacd, dacb, loc, out)) return out;
+  if (tet_edge(2, A, -nabd, -nacd, ap, ad, ap_ad, dp_ad, dadb, dadc, loc, out)) return out;
   f3 nbcd = cross(bc, bd);
-  if (tet_edge(3, m, B, nabc, nbcd, bp, bc, bp_bc, cp_bc, dbca, dbcd, loc, out)) return out;
-  if (tet_edge(4, m, B, -nbcd, nabd, bp, bd, bp_bd, dp_bd, dbdc, dbda, loc, out)) return out;
-  if (tet_edge(5, m, C, nacd, nbcd, cp, cd, cp_cd, dp_cd, dcda, dcdb, loc, out)) return out;
-  if (tet_face(0, m, A, B, C, ap, bp, cp, ab, ac, ad, dabc, dbca, dacb, loc, out)) return out;
-  if (tet_face(1, m, A, B, D, ap, bp, dp, ab, ad, ac, dadb, dabd, dbda, loc, out)) return out;
-  if (tet_face(2, m, A, C, D, ap, cp, dp, ac, ad, ab, dacd, dcda, dadc, loc, out)) return out;
-  if (tet_face(3, m, B, C, D, bp, cp, dp, bc, bd, -ab, dbcd, dcdb, dbdc, loc, out)) return out;
+  if (tet_edge(3, B, nabc, nbcd, bp, bc, bp_bc, cp_bc, dbca, dbcd, loc, out)) return out;
+  if (tet_edge(4, B, -nbcd, nabd, bp, bd, bp_bd, dp_bd, dbdc, dbda, loc, out)) return out;
+  if (tet_edge(5, C, nacd, nbcd, cp, cd, cp_cd, dp_cd, dcda, dcdb, loc, out)) return out;
+  if (tet_face(0, A, B, C, ap, bp, cp, ab, ac, ad, dabc, dbca, dacb, loc, out)) return out;
+  if (tet_face(1, A, B, D, ap, bp, dp, ab, ad, ac, dadb, dabd, dbda, loc, out)) return out;
+  if (tet_face(2, A, C, D, ap, cp, dp, ac, ad, ab, dacd, dcda, dadc, loc, out)) return out;
+  if (tet_face(3, B, C, D, bp, cp, dp, bc, bd, -ab, dbcd, dcdb, dbdc, loc, out)) return out;
   loc.kind = LOC_SOLID; loc.id = 0;
   return xform_pt(m, p);
 }
@@ -610,11 +617,44 @@ struct RCtx {
   ShapeD g1, g2;
   float dil;
   bool dilated;
+  bool local;  // the first map at the identity against ConstantOrigin (m1, m2 and g2 unused)
 };
 
-template <int G>
+// inv_xform_vec(iso_identity(), v), bit for bit: v itself unless a component is zero (whose sign the
+// products by zero may change), infinite or NaN.
+__device__ __forceinline__ f3 ident_inv_vec(f3 v) {
+  const float p = (v.x * v.y) * v.z;
+  if (p != 0.f && p - p == 0.f) return v;
+  return inv_xform_vec(iso_identity(), v);
+}
+
+// support() of a shape at the identity.
+template <int G, int KIND>
+__device__ __forceinline__ f3 support_local(const ShapeD& g, f3 dir, const Pool& P, int gl) {
+  const f3 ld = ident_inv_vec(dir);
+  if (KIND == NCX_CAPSULE || (KIND < 0 && g.type == NCX_CAPSULE)) {
+    const f3 u = normalize(ld);
+    return ident_pt(f3{0.f, copysignf(g.a, u.y), 0.f} + u * g.b);
+  }
+  if (KIND == NCX_CONVEX_HULL || (KIND < 0 && g.type == NCX_CONVEX_HULL)) {
+    const uint32_t id = g.off + hull_support_id<G>(P, g.off, g.cnt, ld, gl);
+    return ident_pt(f3{P.x[id], P.y[id], P.z[id]});
+  }
+  return support<G>(g, iso_identity(), dir, P, gl);
+}
+
+// KIND: the first map's shape type where the caller knows it (any: RC_ANY), which leaves the other
+// types' code out.
+#define RC_ANY -1
+template <int G, int KIND = RC_ANY>
 __device__ __forceinline__ CSOR cso_from_r(const RCtx& c, f3 dir, const Pool& P, int gl) {
   CSOR r;
+  if (KIND != RC_ANY || c.local) {  // ConstantOrigin (special_support_maps.rs:9-13) is the second map
+    r.o1 = support_local<G, KIND>(c.g1, dir, P, gl);
+    r.o2 = f3{0.f, 0.f, 0.f};
+    r.p = r.o1 - r.o2;
+    return r;
+  }
   if (c.dilated) {
     f3 u = normalize(dir);
     r.o1 = support_toward<G>(c.g1, c.m1, u, P, gl) + u * c.dil;
@@ -627,122 +667,143 @@ __device__ __forceinline__ CSOR cso_from_r(const RCtx& c, f3 dir, const Pool& P,
 }
 
 __device__ __forceinline__ bool same_bits(float a, float b) { return __float_as_uint(a) == __float_as_uint(b); }
-__device__ __forceinline__ bool same_bits3(f3 a, f3 b) {
-  return same_bits(a.x, b.x) && same_bits(a.y, b.y) && same_bits(a.z, b.z);
+
+// gjk::minkowski_ray_cast (src/query/algorithms/gjk.rs:245-365) on m1*g1 - m2*g2, ray (o, d), as a
+// state that rc_step advances by one iteration.  The improved_fixed_point_support feature is off
+// (the crate's default).
+#define RC_RUNNING 0
+#define RC_HIT 1
+#define RC_MISS 2
+struct RCState {
+  f3 co, cd, ldir, proj;
+  float ray_length, ltoi, max_bound;
+  bool last_chance;
+  int niter;
+  int still;  // iterations since ltoi last changed
+  SimplexR s;
+};
+
+// The loop is a deterministic function of the simplex's points and dimension, the ray origin and
+// toi, the projection, max_bound and last_chance, and it ends in None after 10000 iterations.  So a
+// cast whose values repeat, bit for bit, those of an earlier iteration is in a cycle that nothing
+// but that cap ends: it returns None at once.  (A shift too small to change the origin with a
+// support point the simplex rejects repeats at once.  About one time of impact in 10,000 of
+// ball-capsule and capsule-capsule pairs does, and one such cast made a batch of 262,144 last 20 ms.)
+// The toi never falls, so it is constant in a cycle: once it has been for RC_STILL iterations, the
+// values of every 2^k-th such iteration are kept in RC_SNAP floats of LDS and those of the ones
+// after it compared with them (Brent's cycle search).
+#define RC_SNAP 21  // odd: the lanes' areas start in different banks
+#define RC_STILL 8
+__device__ __forceinline__ bool rc_repeats(const RCState& r, float* snap) {
+  if (r.still < RC_STILL) return false;
+  const bool keep = (r.still & (r.still - 1)) == 0;
+  if (!keep) {  // the projection alone tells most iterations apart
+    const uint32_t d = (__float_as_uint(snap[0]) ^ __float_as_uint(r.proj.x)) |
+                       (__float_as_uint(snap[1]) ^ __float_as_uint(r.proj.y)) |
+                       (__float_as_uint(snap[2]) ^ __float_as_uint(r.proj.z));
+    if (d != 0) return false;
+  }
+  const int dim = r.s.dim;
+  const f3 z = f3{0.f, 0.f, 0.f};
+  const f3 v[6] = {r.proj, r.co, r.s.v0.p, sel3(dim >= 1, r.s.v1.p, z), sel3(dim >= 2, r.s.v2.p, z),
+                   sel3(dim >= 3, r.s.v3.p, z)};
+  const float w[3] = {r.max_bound, (float)dim, r.last_chance ? 1.f : 0.f};
+  uint32_t diff = keep ? 1u : 0u;
+#pragma unroll
+  for (int i = 0; i < 21; ++i) {
+    const f3 q = v[i < 18 ? i / 3 : 0];
+    const float x = i < 18 ? (i % 3 == 0 ? q.x : (i % 3 == 1 ? q.y : q.z)) : w[i < 18 ? 0 : i - 18];
+    diff |= __float_as_uint(snap[i]) ^ __float_as_uint(x);
+    if (keep) snap[i] = x;
+  }
+  return diff == 0;
 }
 
-// gjk::minkowski_ray_cast (src/query/algorithms/gjk.rs:245-365) on m1*g1 - m2*g2, ray (o, d).
-// Returns false for None.  The improved_fixed_point_support feature is off (the crate's default).
-// An iteration that leaves every value the loop reads bit-identical (the simplex's points and
-// dimension, the ray origin and toi, the projection, max_bound, last_chance and the last normal)
-// is repeated identically until the 10000-iteration cap, so it returns None at once: a shift too
-// small to change the origin (its f32 sums absorb it) with a support point the simplex rejects
-// as affinely dependent is such a fixed point.
-template <int G>
-__device__ __forceinline__ bool minkowski_ray_cast(const RCtx& c, f3 ro, f3 rd, float max_toi, SimplexR& s,
-                                                   const Pool& P, int gl, float& toi_out, f3& normal_out) {
+// The start of a cast, with its first support point.  Returns RC_MISS for a ray without a direction.
+template <int G, int KIND = RC_ANY>
+__device__ __forceinline__ int rc_begin(const RCtx& c, RCState& r, f3 ro, f3 rd, const Pool& P, int gl) {
+  r.ray_length = norm(rd);
+  if (relative_eq_zero(r.ray_length)) return RC_MISS;
+  r.co = ro;
+  r.cd = rd / r.ray_length;
+  r.ldir = -r.cd;
+  r.ltoi = 0.f;
+  r.max_bound = NCX_FLT_MAX;
+  r.last_chance = false;
+  r.niter = 0;
+  r.still = 0;
+  sx_init(r.s);
+  CSOR sp = cso_from_r<G, KIND>(c, r.ldir, P, gl);
+  sp.p = sp.p + (-r.co);
+  sx_reset(r.s, sp);
+  r.proj = sx_project_reduce(r.s);
+  return RC_RUNNING;
+}
+
+// One iteration.  RC_HIT: the toi is ltoi / ray_length and the normal ldir.  Casts that run for
+// hundreds of iterations do so alone in their wavefront, so the step has few branches: updates that
+// an iteration does not make are selects, or additions of -0, which change no value.
+template <int G, int KIND = RC_ANY>
+__device__ __forceinline__ int rc_step(const RCtx& c, float max_toi, RCState& r, const Pool& P, int gl, float* snap) {
   const float eps_tol = NCX_FLT_EPS * 10.f;
   const float eps_rel = __builtin_sqrtf(eps_tol);
-  const float ray_length = norm(rd);
-  if (relative_eq_zero(ray_length)) return false;
-  float ltoi = 0.f;
-  f3 co = ro, cd = rd / ray_length;
-  f3 dir = -cd;
-  f3 ldir = dir;
-  CSOR sp = cso_from_r<G>(c, dir, P, gl);
-  {
-    CSOR t0 = sp;
-    t0.p = sp.p + (-co);
-    sx_reset(s, t0);
+  // try_normalize(-proj, eps_tol)
+  const float dist = norm(-r.proj);
+  const f3 dir = -r.proj / dist;
+  const bool single = dist >= r.max_bound;  // CSOPoint::single_point (cso_point.rs:42-44)
+  const bool lc = r.last_chance || single;
+  if (dist <= eps_tol || (lc && r.ltoi > 0.f)) return RC_HIT;
+  CSOR sp = cso_from_r<G, KIND>(c, dir, P, gl);
+  const f3 pc = r.proj + r.co;
+  sp.p = sel3(single, pc, sp.p);
+  sp.o1 = sel3(single, pc, sp.o1);
+  sp.o2 = sel3(single, f3{0.f, 0.f, 0.f}, sp.o2);
+  // query::ray_toi_with_plane(support point, dir, curr_ray) (src/query/ray/ray_plane.rs:8-37)
+  const float denom = dot(dir, r.cd);
+  const float t = dot(dir, sp.p - r.co) / denom;
+  const bool has_t = !relative_eq_zero(denom) && t >= 0.f;
+  const bool moves = has_t && denom < 0.f && t > 0.f;
+  const float ltoi = r.ltoi + t;
+  const f3 shift = r.cd * t;
+  r.still = moves && !same_bits(ltoi, r.ltoi) ? 0 : r.still + 1;
+  r.ldir = sel3(moves, dir, r.ldir);
+  r.ltoi = moves ? ltoi : r.ltoi;
+  r.co = sel3(moves, r.co + shift, r.co);
+  r.max_bound = moves ? NCX_FLT_MAX : dist;
+  r.last_chance = lc && !moves;
+  {  // VoronoiSimplex::modify_pnts over vertices 0..=dim (voronoi_simplex3.rs:347-351)
+    const f3 z = f3{-0.f, -0.f, -0.f}, ns = -shift;
+    r.s.v0.p = r.s.v0.p + sel3(moves, ns, z);
+    r.s.v1.p = r.s.v1.p + sel3(moves && r.s.dim >= 1, ns, z);
+    r.s.v2.p = r.s.v2.p + sel3(moves && r.s.dim >= 2, ns, z);
+    r.s.v3.p = r.s.v3.p + sel3(moves && r.s.dim >= 3, ns, z);
   }
-  f3 proj = sx_project_reduce(s);
-  float max_bound = NCX_FLT_MAX;
-  int niter = 0;
-  bool last_chance = false;
-  for (;;) {
-    const float old_max_bound = max_bound;
-    const f3 proj_in = proj;
-    const bool lc_in = last_chance;
-    const int dim_in = s.dim;
-    bool same = true;  // nothing changed so far in this iteration
-    {
-      f3 nd;
-      float dist;
-      if (try_normalize(-proj, eps_tol, &nd, &dist)) { dir = nd; max_bound = dist; }
-      else { toi_out = ltoi / ray_length; normal_out = ldir; return true; }
-    }
-    if (max_bound >= old_max_bound) {
-      last_chance = true;  // CSOPoint::single_point (cso_point.rs:42-44)
-      f3 p = proj + co;
-      sp.p = p; sp.o1 = p; sp.o2 = f3{0.f, 0.f, 0.f};
-    } else {
-      sp = cso_from_r<G>(c, dir, P, gl);
-    }
-    if (last_chance && ltoi > 0.f) { toi_out = ltoi / ray_length; normal_out = ldir; return true; }
-    // query::ray_toi_with_plane(support point, dir, curr_ray) (src/query/ray/ray_plane.rs:8-37)
-    const float denom = dot(dir, cd);
-    bool has_t = false;
-    float t = 0.f;
-    if (!relative_eq_zero(denom)) {
-      t = dot(dir, sp.p - co) / denom;
-      has_t = t >= 0.f;
-    }
-    if (has_t) {
-      if (denom < 0.f && t > 0.f) {
-        same = same_bits3(ldir, dir);
-        ldir = dir;
-        const float ltoi_in = ltoi;
-        ltoi += t;
-        if (ltoi / ray_length > max_toi) return false;
-        const f3 shift = cd * t;
-        const f3 co_in = co;
-        co = co + shift;
-        max_bound = NCX_FLT_MAX;
-        const f3 ns = -shift;  // VoronoiSimplex::modify_pnts over vertices 0..=dim (voronoi_simplex3.rs:347-351)
-        const f3 v0 = s.v0.p + ns, v1 = s.v1.p + ns, v2 = s.v2.p + ns, v3 = s.v3.p + ns;
-        same = same && same_bits(ltoi, ltoi_in) && same_bits3(co, co_in) && same_bits3(v0, s.v0.p) &&
-               (s.dim < 1 || same_bits3(v1, s.v1.p)) && (s.dim < 2 || same_bits3(v2, s.v2.p)) &&
-               (s.dim < 3 || same_bits3(v3, s.v3.p));
-        s.v0.p = v0;
-        s.v1.p = sel3(s.dim >= 1, v1, s.v1.p);
-        s.v2.p = sel3(s.dim >= 2, v2, s.v2.p);
-        s.v3.p = sel3(s.dim >= 3, v3, s.v3.p);
-        last_chance = false;
-      }
-    } else if (denom > eps_tol) {
-      return false;
-    }
-    if (last_chance) return false;
-    const float min_bound = -dot(dir, sp.p - co);
-    if (max_bound - min_bound <= eps_rel * max_bound) return false;
-    bool added;
-    {
-      CSOR tp = sp;
-      tp.p = sp.p + (-co);
-      added = sx_add(s, tp);
-    }
-    proj = sx_project_reduce(s);
-    if (s.dim == 3) {
-      if (min_bound >= eps_tol) return false;
-      toi_out = ltoi / ray_length;
-      normal_out = ldir;
-      return true;
-    }
-    // a rejected point leaves the points in place, and a reduction that keeps the dimension of
-    // a point, segment or triangle keeps them in order
-    if (same && !added && s.dim == dim_in && last_chance == lc_in && same_bits(max_bound, old_max_bound) &&
-        same_bits3(proj, proj_in))
-      return false;
-    niter += 1;
-    if (niter == 10000) return false;
-  }
+  const float min_bound = -dot(dir, sp.p - r.co);
+  if ((moves && r.ltoi / r.ray_length > max_toi) || (!has_t && denom > eps_tol) || r.last_chance ||
+      r.max_bound - min_bound <= eps_rel * r.max_bound)
+    return RC_MISS;
+  sp.p = sp.p + (-r.co);
+  sx_add(r.s, sp);
+  r.proj = sx_project_reduce(r.s);
+  if (r.s.dim == 3) return min_bound >= eps_tol ? RC_MISS : RC_HIT;
+  r.niter += 1;
+  return r.niter == 10000 || rc_repeats(r, snap) ? RC_MISS : RC_RUNNING;
+}
+
+// The whole cast.  Returns false for None.  snap: RC_SNAP floats of LDS of this group's own.
+template <int G>
+__device__ __forceinline__ bool minkowski_ray_cast(const RCtx& c, f3 ro, f3 rd, float max_toi, RCState& r,
+                                                   const Pool& P, int gl, float* snap, float& toi_out, f3& normal_out) {
+  int st = rc_begin<G>(c, r, ro, rd, P, gl);
+  while (st == RC_RUNNING) st = rc_step<G>(c, max_toi, r, P, gl, snap);
+  toi_out = r.ltoi / r.ray_length;
+  normal_out = r.ldir;
+  return st == RC_HIT;
 }
 
 // ray_intersection_with_support_map_with_params (src/query/ray/ray_support_map.rs:15-62), shape
-// at the identity (the callers pass a local-frame ray).
-template <int G>
-__device__ __forceinline__ bool ray_support_map(const ShapeD& g, f3 ro, f3 rd, float max_toi, bool solid,
-                                                const Pool& P, int gl, float& toi, f3& normal) {
+// at the identity (the callers pass a local-frame ray): the shape against ConstantOrigin.
+__device__ __forceinline__ RCtx ray_ctx(const ShapeD& g) {
   RCtx c;
   c.m1 = iso_identity();
   c.m2 = iso_identity();
@@ -750,25 +811,45 @@ __device__ __forceinline__ bool ray_support_map(const ShapeD& g, f3 ro, f3 rd, f
   c.g2.type = SHAPE_ORIGIN;
   c.dil = 0.f;
   c.dilated = false;
-  SimplexR s;
-  sx_init(s);
-  float t;
-  f3 n;
-  if (!minkowski_ray_cast<G>(c, ro, rd, max_toi, s, P, gl, t, n)) return false;
-  if (solid || t != 0.f) { toi = t; normal = n; return true; }
-  // the ray starts inside the shape: cast back from a point past its far side
+  c.local = true;
+  return c;
+}
+
+// A ray that starts inside a shape that is not solid is cast back from a point past its far side:
+// the second ray, and how far along the first its origin lies.
+template <int G>
+__device__ __forceinline__ float ray_from_behind(const RCtx& c, f3 ro, f3 rd, const Pool& P, int gl, f3& back) {
   const f3 ndir = normalize(rd);
-  const f3 supp = support<G>(g, c.m1, ndir, P, gl);
-  const float eps = 0.001f;
-  const float shift = dot(supp - ro, ndir) + eps;
-  SimplexR s2;
-  sx_init(s2);
-  if (!minkowski_ray_cast<G>(c, ro + ndir * shift, -rd, shift + eps, s2, P, gl, t, n)) return false;
-  const float tt = shift - t;
-  if (!(tt <= max_toi)) return false;
-  toi = tt;
-  normal = n;
-  return true;
+  const f3 supp = support<G>(c.g1, c.m1, ndir, P, gl);
+  const float shift = dot(supp - ro, ndir) + 0.001f;
+  back = ro + ndir * shift;
+  return shift;
+}
+
+template <int G>
+__device__ __forceinline__ bool ray_support_map(const ShapeD& g, f3 ro, f3 rd, float max_toi, bool solid,
+                                                const Pool& P, int gl, float* snap, float& toi, f3& normal) {
+  const RCtx c = ray_ctx(g);
+  RCState r;
+  f3 o = ro, d = rd;
+  float limit = max_toi, shift = 0.f;
+  bool behind = false;
+  for (;;) {  // one copy of the cast's code
+    float t;
+    f3 n;
+    if (!minkowski_ray_cast<G>(c, o, d, limit, r, P, gl, snap, t, n)) return false;
+    if (behind) t = shift - t;
+    if (behind && !(t <= max_toi)) return false;
+    if (behind || solid || t != 0.f) {
+      toi = t;
+      normal = n;
+      return true;
+    }
+    behind = true;
+    shift = ray_from_behind<G>(c, ro, rd, P, gl, o);
+    d = -rd;
+    limit = shift + 0.001f;
+  }
 }
 
 // ray_toi_with_ball (src/query/ray/ray_ball.rs:83-124).
@@ -877,14 +958,15 @@ __device__ __forceinline__ bool shape_ray_cast_closed(const ShapeD& g, const iso
 
 template <int G>
 __device__ __forceinline__ bool shape_ray_cast(const ShapeD& g, const iso& m, f3 ro, f3 rd, float max_toi, bool solid,
-                                               const Pool& P, int gl, float& toi, f3& normal, uint32_t& feature) {
+                                               const Pool& P, int gl, float* snap, float& toi, f3& normal,
+                                               uint32_t& feature) {
   if (g.type == NCX_BALL || g.type == NCX_CUBOID)
     return shape_ray_cast_closed(g, m, ro, rd, max_toi, solid, toi, normal, feature);
   if (g.type == NCX_CAPSULE || g.type == NCX_CONVEX_HULL) {
     const f3 lo = inv_xform_pt(m, ro), ld = inv_xform_vec(m, rd);
     float t;
     f3 n;
-    if (!ray_support_map<G>(g, lo, ld, max_toi, solid, P, gl, t, n)) return false;
+    if (!ray_support_map<G>(g, lo, ld, max_toi, solid, P, gl, snap, t, n)) return false;
     toi = t;
     normal = xform_vec(m, n);
     feature = NCX_FEAT_UNKNOWN;

@@ -129,6 +129,7 @@ struct ContactTiers {
 struct ncx_shapes {
   ncx_ctx* ctx;
   size_t n = 0, npts = 0;
+  uint32_t types = 0;  // bit t: the set has a shape of type t
   uint32_t buckets = 0xFu;  // bit b: a pair of vertex-count bucket b can occur
   DevBuf shapes;      // ncx_shape[n]
   DevBuf hx, hy, hz;  // hull pool
@@ -308,6 +309,12 @@ int contacts_launch_device_count(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, c
                                  float prediction, const float* init_dir, int max_iter, uint8_t* has, float* w1,
                                  float* w2, float* nrm, float* depth, int32_t* iters, bool may_tune,
                                  float* fdir = nullptr, bool cap_seg = false);
+// Partitions pairs by vertex-count bucket, shape types and overlap into T.blist, each bucket's range
+// at NCX_BKT_RANGE of the header, whose other words it clears; for batches of at least
+// NCX_PARTITION_MIN_PAIRS.
+#define NCX_PARTITION_MIN_PAIRS 16384u
+int pairs_partition(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, const ncx_pose* poses, const uint32_t* ia,
+                    const uint32_t* ib, size_t npairs, const uint32_t* n_dev);
 // Host side after that launch completed: checks, re-runs what both LDS tiers could not hold,
 // and reports the number of pairs that needed more than the first-tier arena.
 int contacts_resolve_overflow(ContactTiers& T, ncx_ctx* ctx, size_t* n_large);

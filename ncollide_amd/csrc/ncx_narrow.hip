@@ -443,6 +443,7 @@ extern "C" int ncx_shapes_create(ncx_ctx* ctx, const ncx_shape* shapes, size_t n
   }
   ncx_shapes* S = new ncx_shapes;
   S->buckets = 0;
+  for (size_t i = 0; i < n; ++i) S->types |= 1u << shapes[i].type;
   for (size_t i = 0; i < n; ++i)
     S->buckets |= 1u << (shapes[i].type == NCX_CONVEX_HULL ? count_bucket(shapes[i].hull_count) : 0u);
   S->ctx = ctx;
@@ -509,8 +510,9 @@ extern "C" int ncx_shapes_count(ncx_shapes* s, size_t* n) {
 // their own order, 133 ms sorted by type pair, 121 ms by type pair and bin.  The radius of shape i
 // is kept in its record's pad[0] (ncx_shapes_create).
 __device__ __forceinline__ uint32_t pair_key(const ncx_shape* __restrict__ shapes, uint32_t nshapes,
-                                             const ncx_pose* __restrict__ poses, uint32_t i1, uint32_t i2) {
-  if (i1 >= nshapes || i2 >= nshapes) return 0;  // the pair kernel reports the bad index
+                                             const ncx_pose* __restrict__ poses, uint32_t i1, uint32_t i2,
+                                             uint32_t bad_key) {
+  if (i1 >= nshapes || i2 >= nshapes) return bad_key;  // the pair kernel reports the bad index
   const ncx_shape s1 = shapes[i1], s2 = shapes[i2];
   uint32_t c1 = s1.type == NCX_CONVEX_HULL ? s1.hull_count : 0;
   uint32_t c2 = s2.type == NCX_CONVEX_HULL ? s2.hull_count : 0;
@@ -554,7 +556,8 @@ __global__ __launch_bounds__(BKT_BLOCK) void k_bucket_count(const uint32_t* __re
                                                             const ncx_shape* __restrict__ shapes, uint32_t nshapes,
                                                             const ncx_pose* __restrict__ poses, size_t npairs,
                                                             const uint32_t* __restrict__ n_dev,
-                                                            uint32_t* __restrict__ hdr, uint32_t* __restrict__ keys) {
+                                                            uint32_t* __restrict__ hdr, uint32_t* __restrict__ keys,
+                                                            uint32_t bad_key) {
   __shared__ uint32_t h[NCX_NKEYS];
   for (uint32_t k = threadIdx.x; k < NCX_NKEYS; k += BKT_BLOCK) h[k] = 0;
   __syncthreads();
@@ -564,7 +567,7 @@ __global__ __launch_bounds__(BKT_BLOCK) void k_bucket_count(const uint32_t* __re
   for (int r = 0; r < BKT_ITEMS; ++r) {
     size_t q = base + (size_t)r * BKT_BLOCK + threadIdx.x;
     if (q < n) {
-      const uint32_t key = pair_key(shapes, nshapes, poses, ia[q], ib[q]);
+      const uint32_t key = pair_key(shapes, nshapes, poses, ia[q], ib[q], bad_key);
       keys[q] = key;
       atomicAdd(&h[key], 1u);
     }
@@ -896,7 +899,6 @@ static int clear_tier_counters(ncx_ctx* ctx, uint32_t* hdr) {
 }
 
 #define TUNE_MIN_PAIRS 4096u
-#define PARTITION_MIN_PAIRS 16384u
 #define TUNE_SAMPLE 131072u
 #define TUNE_ROUNDS 4
 // Every stride-th entry of a bucket's run of the partitioned list, so the sample holds each of
@@ -970,6 +972,34 @@ static int autotune(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, const KArgs& b
   return clear_tier_counters(ctx, hdr);
 }
 
+// Partitions the pair indices by sort key (vertex-count bucket, then type pair and overlap bin)
+// into T.blist, each bucket's range in the header (which is clear).
+static int partition_launch(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, const ncx_pose* poses, const uint32_t* ia,
+                            const uint32_t* ib, size_t npairs, const uint32_t* n_dev) {
+  int rc;
+  if ((rc = contact_tiers_reserve_list(T, npairs))) return rc;
+  uint32_t* ovf = T.ovf.as<uint32_t>();
+  // a pair with a bad index goes to a bucket that is launched
+  const uint32_t bad_key = (NCX_NKEYS / NCX_NBUCKETS) * (uint32_t)__builtin_ctz(S->buckets | 1u << NCX_NBUCKETS);
+  const unsigned bblocks = std::max(1u, ceil_div(npairs, (size_t)BKT_BLOCK * BKT_ITEMS));
+  hipLaunchKernelGGL(k_bucket_count, dim3(bblocks), dim3(BKT_BLOCK), 0, ctx->stream, ia, ib, S->shapes.as<ncx_shape>(),
+                     (uint32_t)S->n, poses, npairs, n_dev, ovf, T.bkey.as<uint32_t>(),
+                     bad_key < NCX_NKEYS ? bad_key : 0u);
+  NCX_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(k_bucket_offsets, dim3(1), dim3(NCX_NKEYS), 0, ctx->stream, ovf);
+  NCX_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(k_bucket_scatter, dim3(bblocks), dim3(BKT_BLOCK), 0, ctx->stream, T.bkey.as<uint32_t>(), npairs,
+                     n_dev, ovf, T.blist.as<uint32_t>());
+  NCX_HIP_CHECK(hipGetLastError());
+  return NCX_OK;
+}
+
+int pairs_partition(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, const ncx_pose* poses, const uint32_t* ia,
+                    const uint32_t* ib, size_t npairs, const uint32_t* n_dev) {
+  int rc = fill_u32(ctx, T.ovf.as<uint32_t>(), NCX_OVF_HEADER, 0u);
+  return rc ? rc : partition_launch(S, T, ctx, poses, ia, ib, npairs, n_dev);
+}
+
 // The launch: partition the pairs into vertex-count buckets (device-side counts, so it is
 // graph-safe), run each bucket with its variant (T1, LDS arenas), then T2, T3 and T4
 // rerun the device-counted overflow list of the tier before with larger LDS arenas, the last
@@ -1006,19 +1036,9 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
   const bool tune_now = may_tune && untuned && npairs >= TUNE_MIN_PAIRS;
   // Partition (sort by key) unless the batch is small: below 16,384 pairs the three partition
   // kernels and the launches per bucket cost more (about 60 us) than the order saves.
-  const bool partition = tune_now || npairs >= PARTITION_MIN_PAIRS;
+  const bool partition = tune_now || npairs >= NCX_PARTITION_MIN_PAIRS;
   if (partition) {
-    // partition the pair indices by sort key (vertex-count bucket, then type pair)
-    if ((rc = contact_tiers_reserve_list(T, npairs))) return rc;
-    unsigned bblocks = std::max(1u, ceil_div(npairs, (size_t)BKT_BLOCK * BKT_ITEMS));
-    hipLaunchKernelGGL(k_bucket_count, dim3(bblocks), dim3(BKT_BLOCK), 0, ctx->stream, a.ia, a.ib, a.shapes,
-                       a.nshapes, a.poses, npairs, n_dev, ovf, T.bkey.as<uint32_t>());
-    NCX_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_bucket_offsets, dim3(1), dim3(NCX_NKEYS), 0, ctx->stream, ovf);
-    NCX_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_bucket_scatter, dim3(bblocks), dim3(BKT_BLOCK), 0, ctx->stream, T.bkey.as<uint32_t>(),
-                       npairs, n_dev, ovf, T.blist.as<uint32_t>());
-    NCX_HIP_CHECK(hipGetLastError());
+    if ((rc = partition_launch(S, T, ctx, a.poses, a.ia, a.ib, npairs, n_dev))) return rc;
     KArgs t = a;
     t.list = T.blist.as<uint32_t>();
     t.n_dev = nullptr;

@@ -84,3 +84,21 @@ def test_runs_past_the_first_arena(variant):
     r = _check(ncx, rec, pool, poses, ia, ib, variant=variant)
     it = r["epa_iters"]
     assert (it > 20).any() and (it > 40).any() and (it > 62).any() and ((it > 0) & (it < 20)).any()
+
+
+@pytest.mark.parametrize("types,npairs", [([3], 20000), ([0, 1], 20000), ([3], 300)])
+def test_bad_index_is_refused(types, npairs):
+    """Whatever buckets the set's pairs fall in, and in batches that are partitioned or not."""
+    import torch
+    import ncollide_amd as ncx
+    from ncollide_amd import query
+    rec, pool, poses, rng = _scene(3, types, 200, 250)
+    ss = ncx.ShapeSet(records=rec, pool=pool)
+    p = torch.as_tensor(poses, device="cuda")
+    ia, ib = rng.integers(0, 200, (2, npairs)).astype(np.int32)
+    ib[npairs // 2] = 200
+    v = torch.zeros((200, 3), device="cuda")
+    for call in (lambda: query.contact(ss, p, ia, ib, 0.0), lambda: query.distance(ss, p, ia, ib),
+                 lambda: query.time_of_impact(ss, p, v, ia, ib, 1.0)):
+        with pytest.raises(ncx.NcxError):
+            call()
