@@ -40,7 +40,8 @@ struct BQArgs {
   float* toi;
   float* nrm;
   uint32_t* err;          // set when a traversal stack would overflow (a tree deeper than the bound)
-  const uint32_t* perm;   // first-hit rays: group k takes ray perm[k] (null: ray k)
+  const uint32_t* perm;   // first-hit rays: the k-th ray taken is perm[k] (null: ray k)
+  uint32_t* work;         // first-hit rays: ray counter (zero at launch)
 };
 
 #define BQ_STACK (LBVH_MAX_DEPTH + 2)
@@ -157,87 +158,176 @@ __global__ __launch_bounds__(BQ_BLOCK) void k_bq_collect(BQArgs a) {
 
 // First hit of each ray among the proxies' shapes (solid = true, toi <= max_toi): the least
 // (toi, handle) over the leaves whose box the ray enters no later than the best hit so far.
-// G lanes per ray: they run the same search, and split the support scans of hull shapes at the
-// leaves (shape_ray_cast<G>).
-#define BQ_RAY_G 4
-template <int G>
-static __global__ __launch_bounds__(BQ_BLOCK) void k_bq_first_ray(BQArgs a) {
-  const uint32_t gi = (blockIdx.x * BQ_BLOCK + threadIdx.x) / G;
-  const int gl = threadIdx.x % G;
-  __shared__ float snaps[BQ_BLOCK / G][RC_SNAP];
-  float* const snap = snaps[threadIdx.x / G];
-  if (gi >= a.nq) return;  // whole groups: BQ_BLOCK is a multiple of G
-  const uint32_t qi = a.perm ? a.perm[gi] : gi;
-  float qv[6];
-  for (int d = 0; d < 6; ++d) qv[d] = a.q[d][qi];
-  const f3 o = f3{qv[0], qv[1], qv[2]}, dir = f3{qv[3], qv[4], qv[5]};
-  float best_t = a.max_toi;
-  uint32_t best_h = BQ_NONE;
-  f3 best_n = f3{0.f, 0.f, 0.f};
-  auto leaf = [&](uint32_t leaf_pos) {
-    const uint32_t h = bq_handle(a, leaf_pos);
-    float t;
-    f3 n;
-    uint32_t feat;
-    if (shape_ray_cast<G>(load_shape(a.shapes, h), load_pose(a.poses, h), o, dir, a.max_toi, true, a.P, gl, snap, t,
-                          n, feat)) {
-      if (t < best_t || (t == best_t && h < best_h)) {
-        best_t = t;
-        best_h = h;
-        best_n = n;
-      }
+// What bounds it: the ray casts on capsules and hulls (GJK, 7 to 20 iterations), and divergence --
+// the rays of a wavefront reach them at different times, and a cast that one lane does alone takes
+// as long as one that all do.  So one lane walks the tree for one ray; balls and cuboids (closed
+// forms) are cast as they are reached; capsules and hulls are kept, up to BQ_KEEP of them, while the
+// lane goes on; and when BQ_WAITING lanes have kept all they can, or have nothing left to walk, each
+// casts its nearest kept one.  A lane whose ray has ended takes the next at the wavefront's next
+// refill.  524,288 rays over 262,144 mixed shapes: 6.45 ms with one ray a lane and casts in place,
+// 1.7 ms now (3.5 ms where one ray's cast runs to thousands of iterations).  Casting at 16, 32, 48,
+// 56, 60 and 64 waiting lanes (whole call): 3.2, 2.6, 2.38, 2.3, 2.29, 2.32 ms with two wavefronts on
+// a SIMD; three of them 2.03; four, which spill, 2.34.  Every kept one is cast, without a test of its bounding ball or segment first: GJK's ray
+// cast reports rays that pass a shape by several hundredths of its size as hits.
+#define BQ_KEEP 2
+#define BQ_LDS_STACK 14
+#define BQ_WAITING 56  // lanes that wait before the kept shapes are cast
+#define BQ_REFILL 8    // idle lanes before the next rays are taken
+#define BQ_CU_BLOCKS 6
+static __global__ __launch_bounds__(BQ_BLOCK, 3) void k_bq_first_ray(BQArgs a) {
+  __shared__ float snaps[BQ_BLOCK][RC_SNAP];
+  __shared__ uint2 lstk[BQ_LDS_STACK][BQ_BLOCK];
+  float* const snap = snaps[threadIdx.x];
+  uint2 deep[BQ_STACK + 1 - BQ_LDS_STACK];  // entries past the LDS ones; one more for a leaf put back
+  const int lane = threadIdx.x & 63;
+  bool live = false, done = false, walk = false;
+  uint32_t qi = 0, node = 0, best_h = BQ_NONE, kh0 = 0, kh1 = 0;
+  int sp = 0, nk = 0;
+  float best_t = 0.f, kt0 = 0.f, kt1 = 0.f;
+  f3 o = f3{0.f, 0.f, 0.f}, dir = o, best_n = o;
+  auto hit = [&](uint32_t h, float t, f3 n) {
+    if (t < best_t || (t == best_t && h < best_h)) {
+      best_t = t;
+      best_h = h;
+      best_n = n;
     }
   };
-  if (a.nleaves == 1) {
-    const float* b = a.leaf_soa;
-    float c;
-    if (bq_ray_box(o, dir, a.max_toi, b[0], b[1], b[2], b[3], b[4], b[5], c)) leaf(0);
-  } else {
-    uint32_t stk[BQ_STACK];
-    float stc[BQ_STACK];
-    int sp = 0;
-    uint32_t node = 0;
-    for (;;) {
-      const LNode nd = a.nodes[node];
-      float cl, cr;
-      bool hl = bq_ray_box(o, dir, a.max_toi, nd.lminx, nd.lminy, nd.lminz, nd.lmaxx, nd.lmaxy, nd.lmaxz, cl) &&
-                cl <= best_t;
-      bool hr = bq_ray_box(o, dir, a.max_toi, nd.rminx, nd.rminy, nd.rminz, nd.rmaxx, nd.rmaxy, nd.rmaxz, cr) &&
-                cr <= best_t;
-      if (hl && (nd.child_l & NCX_LEAF_BIT)) { leaf(nd.child_l & ~NCX_LEAF_BIT); hl = false; }
-      if (hr && (nd.child_r & NCX_LEAF_BIT)) { leaf(nd.child_r & ~NCX_LEAF_BIT); hr = false; }
-      hl = hl && cl <= best_t;
-      hr = hr && cr <= best_t;
-      if (hl && hr) {
-        if (sp == BQ_STACK) { atomicOr(a.err, 1u); break; }
-        const bool lfirst = cl <= cr;
-        stk[sp] = lfirst ? nd.child_r : nd.child_l;
-        stc[sp] = lfirst ? cr : cl;
-        ++sp;
-        node = lfirst ? nd.child_l : nd.child_r;
-      } else if (hl) {
-        node = nd.child_l;
-      } else if (hr) {
-        node = nd.child_r;
-      } else {
-        // pop entries until one can still hold a better hit
-        bool found = false;
-        while (sp > 0) {
-          --sp;
-          if (stc[sp] <= best_t) { node = stk[sp]; found = true; break; }
+  auto leaf = [&](uint32_t leaf_pos, float entry) {
+    const uint32_t h = bq_handle(a, leaf_pos);
+    const ShapeD g = load_shape(a.shapes, h);
+    const iso m = load_pose(a.poses, h);
+    if (g.type == NCX_CAPSULE || g.type == NCX_CONVEX_HULL) {
+      // the nearest of the kept ones first
+      const bool front = nk == 0 || entry < kt0;
+      kh1 = front ? kh0 : h;
+      kt1 = front ? kt0 : entry;
+      kh0 = front ? h : kh0;
+      kt0 = front ? entry : kt0;
+      ++nk;
+    } else {
+      float t;
+      f3 n;
+      uint32_t feat;
+      if (shape_ray_cast_closed(g, m, o, dir, a.max_toi, true, t, n, feat)) hit(h, t, n);
+    }
+  };
+  auto push = [&](uint32_t child, float entry) {
+    if (sp == BQ_STACK + 1) {
+      atomicOr(a.err, 1u);
+      return;
+    }
+    const uint2 e = uint2{child, __float_as_uint(entry)};
+    if (sp < BQ_LDS_STACK) lstk[sp][threadIdx.x] = e;
+    else deep[sp - BQ_LDS_STACK] = e;
+    ++sp;
+  };
+  for (;;) {
+    const uint64_t wm = __ballot(!live && !done), lm = __ballot(live);
+    if ((wm | lm) == 0) break;
+    if (wm && (lm == 0 || __popcll(wm) >= BQ_REFILL)) {
+      uint32_t t = 0;
+      const int first = __builtin_ctzll(wm);
+      if (lane == first) t = atomicAdd(a.work, (uint32_t)__popcll(wm));
+      t = (uint32_t)__builtin_amdgcn_readlane((int)t, first);
+      if (!live && !done) {
+        const uint32_t gi = t + (uint32_t)__popcll(wm & ((1ull << lane) - 1ull));
+        if (gi >= a.nq) {
+          done = true;
+        } else {
+          live = true;
+          qi = a.perm ? a.perm[gi] : gi;
+          o = f3{a.q[0][qi], a.q[1][qi], a.q[2][qi]};
+          dir = f3{a.q[3][qi], a.q[4][qi], a.q[5][qi]};
+          best_t = a.max_toi;
+          best_h = BQ_NONE;
+          best_n = f3{0.f, 0.f, 0.f};
+          sp = nk = 0;
+          node = 0;
+          walk = a.nleaves > 1;
+          if (!walk) {
+            const float* b = a.leaf_soa;
+            float c;
+            if (bq_ray_box(o, dir, a.max_toi, b[0], b[1], b[2], b[3], b[4], b[5], c)) leaf(0, c);
+          }
         }
-        if (!found) break;
       }
     }
+    for (;;) {
+      const bool act = live && walk && nk < BQ_KEEP;
+      const uint64_t am = __ballot(act);
+      if (am == 0 || __popcll(__ballot(live && !act)) >= BQ_WAITING) break;
+      if (act) {
+        uint32_t next = BQ_NONE;
+        float next_t = 0.f;
+        if (node != BQ_NONE) {
+          const LNode nd = a.nodes[node];
+          float cl, cr;
+          const bool hl = bq_ray_box(o, dir, a.max_toi, nd.lminx, nd.lminy, nd.lminz, nd.lmaxx, nd.lmaxy, nd.lmaxz, cl);
+          const bool hr = bq_ray_box(o, dir, a.max_toi, nd.rminx, nd.rminy, nd.rminz, nd.rmaxx, nd.rmaxy, nd.rmaxz, cr);
+          const bool lfirst = hl && (!hr || cl <= cr);
+          const bool h0 = (lfirst ? hl : hr) && (lfirst ? cl : cr) <= best_t;
+          const bool h1 = (lfirst ? hr : hl) && (lfirst ? cr : cl) <= best_t;
+          const uint32_t c0 = lfirst ? nd.child_l : nd.child_r, c1 = lfirst ? nd.child_r : nd.child_l;
+          const float t1 = lfirst ? cr : cl;
+          if (h0) {
+            next = c0;
+            next_t = lfirst ? cl : cr;
+            if (h1) push(c1, t1);
+          } else if (h1) {
+            next = c1;
+            next_t = t1;
+          }
+        }
+        // the next node; leaves are taken on the way
+        for (;;) {
+          if (next == BQ_NONE) {
+            if (sp == 0) break;
+            --sp;
+            uint2 e;
+            if (sp < BQ_LDS_STACK) e = lstk[sp][threadIdx.x];
+            else e = deep[sp - BQ_LDS_STACK];
+            next_t = __uint_as_float(e.y);
+            if (!(next_t <= best_t)) continue;
+            next = e.x;
+          }
+          if (!(next & NCX_LEAF_BIT)) break;
+          if (nk == BQ_KEEP) {  // no room: back onto the stack
+            push(next, next_t);
+            next = BQ_NONE;
+            break;
+          }
+          leaf(next & ~NCX_LEAF_BIT, next_t);
+          next = BQ_NONE;
+        }
+        node = next;
+        walk = node != BQ_NONE || sp > 0;
+      }
+    }
+    if (live && nk > 0 && (nk == BQ_KEEP || !walk)) {
+      const uint32_t h = kh0;
+      const float entry = kt0;
+      kh0 = kh1;
+      kt0 = kt1;
+      --nk;
+      if (entry <= best_t) {
+        float t;
+        f3 n;
+        uint32_t feat;
+        if (shape_ray_cast<1>(load_shape(a.shapes, h), load_pose(a.poses, h), o, dir, a.max_toi, true, a.P, 0, snap, t,
+                              n, feat))
+          hit(h, t, n);
+      }
+    }
+    if (live && nk == 0 && !walk) {
+      a.handles[qi] = best_h;
+      a.toi[qi] = best_h == BQ_NONE ? -1.f : best_t;
+      a.nrm[3 * (size_t)qi] = best_n.x;
+      a.nrm[3 * (size_t)qi + 1] = best_n.y;
+      a.nrm[3 * (size_t)qi + 2] = best_n.z;
+      live = false;
+    }
   }
-  if (gl != 0) return;
-  a.handles[qi] = best_h;
-  a.toi[qi] = best_h == BQ_NONE ? -1.f : best_t;
-  a.nrm[3 * (size_t)qi] = best_n.x;
-  a.nrm[3 * (size_t)qi + 1] = best_n.y;
-  a.nrm[3 * (size_t)qi + 2] = best_n.z;
 }
-static_assert(BQ_BLOCK % BQ_RAY_G == 0, "a block holds whole groups");
 
 // Count pass, scan, write pass.  *total = hits over all queries; NCX_E_CAPACITY when above cap
 // (nothing written).  offs (nq + 1 entries) receives each query's first slot and the total.

@@ -968,8 +968,9 @@ extern "C" int ncx_world_first_interference_with_rays(ncx_world* w, const ncx_po
   a.toi = toi_dev;
   a.nrm = normal_dev;
   int rc;
-  if ((rc = w->qtot.reserve(16)) || (rc = fill_u32(w->ctx, w->qtot.as<uint32_t>() + 1, 1, 0u))) return rc;
+  if ((rc = w->qtot.reserve(16)) || (rc = fill_u32(w->ctx, w->qtot.as<uint32_t>() + 1, 2, 0u))) return rc;
   a.err = w->qtot.as<uint32_t>() + 1;
+  a.work = w->qtot.as<uint32_t>() + 2;
   a.perm = nullptr;
   if (n >= BQ_SORT_MIN && w->n > 1) {
     if ((rc = w->rkeys.reserve(n * 4)) || (rc = w->rvals.reserve(n * 4))) return rc;
@@ -984,8 +985,8 @@ extern "C" int ncx_world_first_interference_with_rays(ncx_world* w, const ncx_po
     if ((rc = radix_sort_u32(w->ctx, k.keys, k.vals, n, 0, 30, w->rtk, w->rtv, w->rhist, w->rscan))) return rc;
     a.perm = k.vals;  // a permutation of 0..n-1
   }
-  hipLaunchKernelGGL(k_bq_first_ray<BQ_RAY_G>, dim3(ceil_div(n * BQ_RAY_G, BQ_BLOCK)), dim3(BQ_BLOCK), 0,
-                     w->ctx->stream, a);
+  hipLaunchKernelGGL(k_bq_first_ray, dim3(std::min<unsigned>(ceil_div(n, BQ_BLOCK), (unsigned)w->ctx->num_cus * BQ_CU_BLOCKS)),
+                     dim3(BQ_BLOCK), 0, w->ctx->stream, a);
   NCX_HIP_CHECK(hipGetLastError());
   uint32_t err = 0;
   NCX_HIP_CHECK(hipMemcpyAsync(&err, w->qtot.as<uint32_t>() + 1, 4, hipMemcpyDeviceToHost, w->ctx->stream));
