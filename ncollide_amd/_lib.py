@@ -158,3 +158,17 @@ def soa_columns(rows, k, device):
     import torch
     t = torch.as_tensor(rows, device=device, dtype=torch.float32).reshape(-1, k)
     return [t[:, d].contiguous() for d in range(k)]
+
+
+def ray_columns(origins, dirs, device):
+    """(n, 3) host or device origins and directions -> the rays' six float32 device columns."""
+    import torch
+    o = torch.as_tensor(origins, device=device, dtype=torch.float32).reshape(-1, 3)
+    d = torch.as_tensor(dirs, device=device, dtype=torch.float32).reshape(-1, 3)
+    if o.shape != d.shape:
+        return [c.contiguous() for c in (*o.unbind(1), *d.unbind(1))]
+    # two transposing copies into one array; a copy per column takes six launches
+    cols = torch.empty((6, o.shape[0]), dtype=torch.float32, device=device)
+    cols[:3].copy_(o.t())
+    cols[3:].copy_(d.t())
+    return list(cols.unbind(0))

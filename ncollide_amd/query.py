@@ -120,13 +120,10 @@ def cast_rays(shapes, poses, shape_idx, origins, dirs, max_toi, solid=True):
     dev = ctx.device
     poses = torch.as_tensor(poses, device=dev, dtype=torch.float32).contiguous()
     idx = _u32(shape_idx, dev)
-    o = torch.as_tensor(origins, device=dev, dtype=torch.float32).reshape(-1, 3)
-    d = torch.as_tensor(dirs, device=dev, dtype=torch.float32).reshape(-1, 3)
+    soa = _lib.ray_columns(origins, dirs, dev)
     n = idx.numel()
-    if o.shape[0] != n or d.shape[0] != n:
+    if soa[0].numel() != n or soa[3].numel() != n:
         raise ValueError("one ray per shape index is required")
-    soa = [o[:, 0].contiguous(), o[:, 1].contiguous(), o[:, 2].contiguous(),
-           d[:, 0].contiguous(), d[:, 1].contiguous(), d[:, 2].contiguous()]
     toi = torch.empty(n, dtype=torch.float32, device=dev)
     nrm = torch.empty((n, 3), dtype=torch.float32, device=dev)
     feat = torch.empty(n, dtype=torch.int32, device=dev)

@@ -27,12 +27,7 @@ class TriMesh:
         self.nfaces = len(self.indices)
 
     def _rays(self, origins, dirs):
-        dev = self.ctx.device
-        o = torch.as_tensor(origins, device=dev, dtype=torch.float32).reshape(-1, 3)
-        d = torch.as_tensor(dirs, device=dev, dtype=torch.float32).reshape(-1, 3)
-        soa = [o[:, 0].contiguous(), o[:, 1].contiguous(), o[:, 2].contiguous(),
-               d[:, 0].contiguous(), d[:, 1].contiguous(), d[:, 2].contiguous()]
-        return soa
+        return _lib.ray_columns(origins, dirs, self.ctx.device)
 
     @staticmethod
     def _pose(pose):

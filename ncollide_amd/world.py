@@ -112,9 +112,10 @@ class World:
 
     # -- world-level queries through the broad phase (after a step; handles are shape indices)
     def _rays(self, origins, dirs):
-        return _lib.soa_columns(torch.cat([torch.as_tensor(origins, dtype=torch.float32).reshape(-1, 3).cpu(),
-                                           torch.as_tensor(dirs, dtype=torch.float32).reshape(-1, 3).cpu()], 1),
-                                6, self.ctx.device)
+        cols = _lib.ray_columns(origins, dirs, self.ctx.device)
+        if cols[0].numel() != cols[3].numel():
+            raise RuntimeError("origins and dirs differ in length")
+        return cols
 
     def first_interference_with_rays(self, poses, origins, dirs, max_toi):
         """CollisionWorld::first_interference_with_ray per ray (solid casts): (handle, toi, normal)
