@@ -153,3 +153,25 @@ def test_gpu_descriptors_and_features(ctx):
         ref = np.concatenate([(R1.T @ R2).ravel(), R1.T @ (P[ib[k], :3] - P[ia[k], :3]), desc[ia[k]], desc[ib[k]],
                               np.zeros(4)])
         assert np.allclose(f[k], ref, atol=2e-3 * np.maximum(1, np.abs(ref)).max()), k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 16, 17, 63, 64, 65, 1000, 64 * 512 + 1])
+def test_gpu_gradient_at_tile_edges(ctx, n):
+    """Batches around a sample tile, a block's 64 rows and the grid's end.  A gradient entry sums n
+    products of 16-bit operands in 32 bits, so up to a row whose rounding at a ReLU's zero differs,
+    it matches the emulation to sqrt(n) 2^-11 of the entries' size; 1e-2 of the norm covers both."""
+    import torch
+    from ncollide_amd.warmstart import WarmStartMLP
+    rng = np.random.default_rng(n)
+    mlp = WarmStartMLP(ctx, seed=5)
+    p = random_params(rng, 0.2).astype(np.float32)
+    mlp.set_params(p)
+    X = random_features(rng, n).astype(np.float16)
+    Y = rng.normal(0, 1, (n, 3)).astype(np.float32)
+    g, loss = mlp.grad(torch.as_tensor(X, device=ctx.device), torch.as_tensor(Y, device=ctx.device))
+    g = g.cpu().numpy()
+    rl, rg = mlp_ref.loss_and_grad(p, X.astype(np.float32), Y, emulated=True)
+    assert abs(loss.item() - rl) < 1e-3 * rl
+    assert np.linalg.norm(g - rg) < 1e-2 * np.linalg.norm(rg)
+    assert np.all(g[~mlp_ref.valid_mask()] == 0)
