@@ -696,7 +696,7 @@ __device__ __forceinline__ PairOut contact_pair(const Ctx2& c, float prediction,
     max_iter = 10000;
   }
   if (!found) dir = f3{1.f, 0.f, 0.f};
-  const GJKOut g = gjk<G, true>(cc, dir, max_dist, s, P, gl, max_iter);
+  const GJKOut g = gjk<G, true, 8>(cc, dir, max_dist, s, P, gl, max_iter);
   o.gjk_iters = g.iters;
   if (g.status == GJK_S_INTERSECTION) {
     o.has = 5;

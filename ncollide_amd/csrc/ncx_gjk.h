@@ -92,10 +92,13 @@ template <int G, int O = 1> __device__ __forceinline__ void hull_best(float& bes
 // the maximum over the non-NaN dots (NaN never compares greater).  Each lane scans vertices
 // gl, gl + G, ... in increasing order keeping its first maximum over non-NaN dots; the lane
 // reduction keeps the larger value and, on ties, the lower index (vertex 0 with a NaN dot enters
-// it as infinity).  U vertices' loads are issued together so their latencies overlap.
-template <int G>
+// it as infinity).  U vertices' loads are issued together so their latencies overlap:
+// the hulls in flight are far more than the first-level cache holds.  262,144 hull pairs of up to 256
+// vertices, U = 4 and 8: contacts 2.71 and 2.48 ms, distances 2.12 and 1.76 ms; 12 and 16 no better.
+// In the other kernels, whose scans are shorter or whose registers decide how many wavefronts run,
+// 4: 65,536 shapes over a terrain take 27.2 ms with 4 and 30.3 ms with 8.
+template <int G, int U = 4>
 __device__ __forceinline__ uint32_t hull_support_id(const Pool& P, uint32_t off, uint32_t cnt, f3 dir, int gl) {
-  constexpr int U = 4;
   float best = 0.f;
   uint32_t bi = HULL_NONE;
   bool nan0 = false;
@@ -133,7 +136,8 @@ __device__ __forceinline__ uint32_t hull_support_id(const Pool& P, uint32_t off,
 // SupportMap::support_point (src/shape/support_map.rs:26-29) and the overrides of
 // Ball (ball.rs:31-38), Cuboid (cuboid.rs:135-146), Capsule (capsule.rs:72-84),
 // ConvexHull (convex.rs:418-423), ConstantOrigin (special_support_maps.rs:9-13).
-template <int G>
+// HULLS false: for shapes other than hulls.
+template <int G, bool HULLS = true, int U = 4>
 __device__ __forceinline__ f3 support(const ShapeD& g, const iso& m, f3 dir, const Pool& P, int gl) {
   switch (g.type) {
     case NCX_BALL: {
@@ -152,8 +156,9 @@ __device__ __forceinline__ f3 support(const ShapeD& g, const iso& m, f3 dir, con
       return xform_pt(m, res + u * g.b);
     }
     case NCX_CONVEX_HULL: {
+      if constexpr (!HULLS) return f3{0.f, 0.f, 0.f};
       f3 ld = inv_xform_vec(m, dir);
-      uint32_t id = hull_support_id<G>(P, g.off, g.cnt, ld, gl);
+      uint32_t id = hull_support_id<G, U>(P, g.off, g.cnt, ld, gl);
       f3 p = f3{P.x[g.off + id], P.y[g.off + id], P.z[g.off + id]};
       return xform_pt(m, p);
     }
@@ -191,11 +196,47 @@ struct Ctx2 {
   ShapeD g1, g2;
 };
 
-template <int G>
+template <int G, int U = 4>
 __device__ __forceinline__ CSO cso_from(const Ctx2& c, f3 dir, const Pool& P, int gl) {
   CSO r;
-  r.o1 = support<G>(c.g1, c.m1, dir, P, gl);
-  r.o2 = support<G>(c.g2, c.m2, -dir, P, gl);
+  r.o1 = support<G, true, U>(c.g1, c.m1, dir, P, gl);
+  r.o2 = support<G, true, U>(c.g2, c.m2, -dir, P, gl);
+  return r;
+}
+
+// support() of a shape per lane, called by the whole wavefront (`on`: the lanes that want one).  The
+// hulls' scans are shared: group by group of GS lanes, the lanes of a group scan the hull of one of
+// them after the other.
+template <int GS>
+__device__ __forceinline__ f3 support_wave(const ShapeD& g, const iso& m, f3 dir, const Pool& P, bool on) {
+  const int lane = __lane_id(), gl = lane & (GS - 1);
+  const bool hull = on && g.type == NCX_CONVEX_HULL;
+  f3 r = f3{0.f, 0.f, 0.f};
+  const uint64_t need = __ballot(hull);
+  if (need) {
+    const f3 ld = inv_xform_vec(m, dir);
+    const uint32_t off = g.off, cnt = hull ? g.cnt : 0u;
+    uint32_t id = 0;
+#pragma unroll 1
+    for (int j = 0; j < GS; ++j) {
+      if (!(need & ((~0ull / ((1ull << GS) - 1ull)) << j))) continue;
+      const int src = 4 * ((lane & ~(GS - 1)) + j);
+      auto of = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)v); };
+      const f3 d = f3{__uint_as_float(of(__float_as_uint(ld.x))), __uint_as_float(of(__float_as_uint(ld.y))),
+                      __uint_as_float(of(__float_as_uint(ld.z)))};
+      const uint32_t best = hull_support_id<GS, 8>(P, of(off), of(cnt), d, gl);
+      id = gl == j ? best : id;
+    }
+    if (hull) r = xform_pt(m, f3{P.x[off + id], P.y[off + id], P.z[off + id]});
+  }
+  if (on && !hull) r = support<1, false>(g, m, dir, P, 0);
+  return r;
+}
+template <int GS>
+__device__ __forceinline__ CSO cso_wave(const Ctx2& c, f3 dir, const Pool& P, bool on) {
+  CSO r;
+  r.o1 = support_wave<GS>(c.g1, c.m1, dir, P, on);
+  r.o2 = support_wave<GS>(c.g2, c.m2, -dir, P, on);
   return r;
 }
 
@@ -509,86 +550,102 @@ struct GJKOut {
 // point (epa3.rs:294-305) are taken by one support call in the loop, so a kernel holds the support
 // functions of every shape once; with a call each, the contact kernel's GJK spilled 103 registers
 // more.
-template <int G, bool FOR_EPA = false>
+struct GJKRun {
+  f3 dir, old_dir;
+  float max_bound;
+  int niter;  // -1: the first point; -2: a segment's third point
+};
+__device__ __forceinline__ void gjk_begin(GJKRun& g, Simplex& s, GJKOut& r, f3 dir) {
+  r.iters = 0;
+  sx_init(s);
+  g.dir = dir;
+  g.old_dir = f3{0.f, 0.f, 0.f};
+  g.max_bound = NCX_FLT_MAX;
+  g.niter = -1;
+}
+// What follows the support point along g.dir; true when the run has ended, with its result in r.
+template <bool FOR_EPA>
+__device__ __forceinline__ bool gjk_step(GJKRun& g, Simplex& s, const CSO& cso, float max_dist, int max_iter,
+                                         GJKOut& r) {
+  const float eps_tol = NCX_FLT_EPS * 10.f;
+  const float eps_rel = __builtin_sqrtf(eps_tol);
+  f3 proj;
+  if (FOR_EPA && g.niter == -2) {
+    s.v2 = cso;
+    s.dim = 2;
+    r.status = GJK_S_INTERSECTION;
+    return true;
+  }
+  bool meets = false;
+  if (g.niter < 0) {
+    sx_reset(s, cso);
+    proj = sx_project_reduce(s);
+    f3 pd;
+    float nl;
+    if (try_normalize(proj, 0.f, &pd, &nl)) g.old_dir = -pd;
+    else meets = true;
+  } else {
+    r.iters += 1;
+    const float min_bound = -dot(g.dir, cso.pt());
+    if (!(min_bound == min_bound)) { r.status = GJK_S_NAN; return true; }
+    if (min_bound > max_dist) { r.dir = g.dir; r.status = GJK_S_NOINTER; return true; }
+    if (g.max_bound - min_bound <= eps_rel * g.max_bound || !sx_add(s, cso)) {
+      gjk_result(s, false, r.p1, r.p2);
+      r.dir = g.dir;
+      r.status = GJK_S_CLOSEST;
+      return true;
+    }
+    g.old_dir = g.dir;
+    proj = sx_project_reduce(s);
+    if (s.dim == 3) {
+      if (min_bound >= eps_tol) {
+        gjk_result(s, true, r.p1, r.p2);
+        r.dir = g.old_dir;
+        r.status = GJK_S_CLOSEST;
+        return true;
+      }
+      r.status = GJK_S_INTERSECTION;
+      return true;
+    }
+  }
+  g.niter += 1;
+  if (g.niter > 0 && g.niter == max_iter) { r.dir = f3{1.f, 0.f, 0.f}; r.status = GJK_S_CAP; return true; }
+  const float old_max_bound = g.max_bound;
+  f3 nd;
+  float dist;
+  if (!meets && try_normalize(-proj, eps_tol, &nd, &dist)) {
+    g.dir = nd;
+    g.max_bound = dist;
+  } else {
+    if (FOR_EPA && s.dim == 1) {
+      const f3 dpt = s.v1.pt() - s.v0.pt();
+      // nalgebra orthonormal_subspace_basis for one vector; epa3.rs:299-305 keeps a x dpt.
+      f3 a = fabsf(dpt.x) > fabsf(dpt.y) ? f3{dpt.z, 0.f, -dpt.x} : f3{0.f, -dpt.z, dpt.y};
+      a = normalize(a);
+      g.dir = cross(a, dpt);
+      g.niter = -2;
+      return false;
+    }
+    r.status = GJK_S_INTERSECTION;
+    return true;
+  }
+  if (g.max_bound >= old_max_bound) {
+    gjk_result(s, true, r.p1, r.p2);
+    r.dir = g.old_dir;
+    r.status = GJK_S_CLOSEST;
+    return true;
+  }
+  return false;
+}
+template <int G, bool FOR_EPA = false, int U = 4>
 __device__ __forceinline__ GJKOut gjk(const Ctx2& c, f3 dir, float max_dist, Simplex& s, const Pool& P, int gl,
                                       int max_iter) {
   GJKOut r;
-  r.iters = 0;
-  const float eps_tol = NCX_FLT_EPS * 10.f;
-  const float eps_rel = __builtin_sqrtf(eps_tol);
-  sx_init(s);
-  f3 old_dir = f3{0.f, 0.f, 0.f};
-  float max_bound = NCX_FLT_MAX;
-  int niter = -1;  // -1: the first point; -2: a segment's third point
-  for (;;) {
-    const CSO cso = cso_from<G>(c, dir, P, gl);
-    f3 proj;
-    if (FOR_EPA && niter == -2) {
-      s.v2 = cso;
-      s.dim = 2;
-      r.status = GJK_S_INTERSECTION;
-      return r;
-    }
-    bool meets = false;
-    if (niter < 0) {
-      sx_reset(s, cso);
-      proj = sx_project_reduce(s);
-      f3 pd;
-      float nl;
-      if (try_normalize(proj, 0.f, &pd, &nl)) old_dir = -pd;
-      else meets = true;
-    } else {
-      r.iters += 1;
-      const float min_bound = -dot(dir, cso.pt());
-      if (!(min_bound == min_bound)) { r.status = GJK_S_NAN; return r; }
-      if (min_bound > max_dist) { r.dir = dir; r.status = GJK_S_NOINTER; return r; }
-      if (max_bound - min_bound <= eps_rel * max_bound || !sx_add(s, cso)) {
-        gjk_result(s, false, r.p1, r.p2);
-        r.dir = dir;
-        r.status = GJK_S_CLOSEST;
-        return r;
-      }
-      old_dir = dir;
-      proj = sx_project_reduce(s);
-      if (s.dim == 3) {
-        if (min_bound >= eps_tol) {
-          gjk_result(s, true, r.p1, r.p2);
-          r.dir = old_dir;
-          r.status = GJK_S_CLOSEST;
-          return r;
-        }
-        r.status = GJK_S_INTERSECTION;
-        return r;
-      }
-    }
-    niter += 1;
-    if (niter > 0 && niter == max_iter) { r.dir = f3{1.f, 0.f, 0.f}; r.status = GJK_S_CAP; return r; }
-    const float old_max_bound = max_bound;
-    f3 nd;
-    float dist;
-    if (!meets && try_normalize(-proj, eps_tol, &nd, &dist)) {
-      dir = nd;
-      max_bound = dist;
-    } else {
-      if (FOR_EPA && s.dim == 1) {
-        const f3 dpt = s.v1.pt() - s.v0.pt();
-        // nalgebra orthonormal_subspace_basis for one vector; epa3.rs:299-305 keeps a x dpt.
-        f3 a = fabsf(dpt.x) > fabsf(dpt.y) ? f3{dpt.z, 0.f, -dpt.x} : f3{0.f, -dpt.z, dpt.y};
-        a = normalize(a);
-        dir = cross(a, dpt);
-        niter = -2;
-        continue;
-      }
-      r.status = GJK_S_INTERSECTION;
-      return r;
-    }
-    if (max_bound >= old_max_bound) {
-      gjk_result(s, true, r.p1, r.p2);
-      r.dir = old_dir;
-      r.status = GJK_S_CLOSEST;
-      return r;
-    }
+  GJKRun g;
+  gjk_begin(g, s, r, dir);
+  while (!gjk_step<FOR_EPA>(g, s, cso_from<G, U>(c, g.dir, P, gl), max_dist, max_iter, r)) {
   }
+  return r;
 }
 
 // ------------------------------------------------------------------ time of impact and ray casts on support maps

@@ -406,7 +406,7 @@ __global__ __launch_bounds__(BS, 3) void k_distance(KArgs a) {
         float nl;
         if (!try_normalize(d0, NCX_FLT_EPS, &dir, &nl)) dir = f3{1.f, 0.f, 0.f};
         Simplex s;
-        GJKOut r = gjk<G>(c, dir, NCX_FLT_MAX, s, a.P, gl, warm ? a.max_iter : 10000);
+        GJKOut r = gjk<G, false, 8>(c, dir, NCX_FLT_MAX, s, a.P, gl, warm ? a.max_iter : 10000);
         it += r.iters;
         if (warm && r.status == GJK_S_CAP && a.max_iter < 10000) {
           warm = false;
@@ -420,6 +420,97 @@ __global__ __launch_bounds__(BS, 3) void k_distance(KArgs a) {
     if (gl == 0) {
       a.dist[k] = d;
       if (a.iters) a.iters[k] = it;
+    }
+  }
+}
+
+// The same with one pair a lane, the lanes of a group of DW_G scanning each other's hulls in turn.
+// What bounds k_distance on hulls: two thirds of its VALU slots are taken, three quarters of them by
+// the simplex's projection and reduction, which every lane of a group repeats for the one pair; and
+// the scans' loads, which the second-level cache serves.  Here a lane projects its own pair's simplex
+// and only the scans are shared, so that both are done once a pair; the loads still come 8 lanes at a
+// time from one hull.  262,144 hull pairs of up to 256 vertices, whole batch: 2.37 ms in groups,
+// 1.76 ms so (groups of 4 and 16: 2.1 and 1.78 ms; a wavefront's lanes that wait for new pairs at 4
+// or 16 idle ones, the same).  It needs 64 pairs a wavefront to pay, so the autotuner chooses it or a
+// group's kernel for each vertex-count bucket by timing both on a sample.
+#define DW_G 8
+#define DW_REFILL 16  // idle lanes before the wavefront takes more pairs
+template <int BS>
+__global__ __launch_bounds__(BS, 2) void k_distance_wave(KArgs a) {
+  const int lane = __lane_id();
+  size_t npairs = a.npairs;
+  size_t lbase = 0;
+  if (a.range_b) {
+    lbase = *a.range_b;
+    npairs = *a.range_e - lbase;
+  }
+  bool live = false, done = false, warm = false;
+  size_t k = 0;
+  int it = 0;
+  Ctx2 c = {};
+  Simplex s;
+  GJKRun g;
+  GJKOut r;
+  g.dir = f3{0.f, 0.f, 0.f};
+  auto begin = [&](f3 d0) {
+    f3 dir;
+    float nl;
+    if (!try_normalize(d0, NCX_FLT_EPS, &dir, &nl)) dir = f3{1.f, 0.f, 0.f};
+    gjk_begin(g, s, r, dir);
+  };
+  auto write = [&](float d) {
+    a.dist[k] = d;
+    if (a.iters) a.iters[k] = it;
+  };
+  for (;;) {
+    const uint64_t idle = __ballot(!live && !done), lm = __ballot(live);
+    if ((idle | lm) == 0) break;
+    if (idle && (lm == 0 || __popcll(idle) >= DW_REFILL)) {
+      uint32_t t = 0;
+      const int first = __builtin_ctzll(idle);
+      if (lane == first) t = atomicAdd(a.work, (uint32_t)__popcll(idle));
+      t = (uint32_t)__builtin_amdgcn_readlane((int)t, first);
+      if (!live && !done) {
+        const size_t q = (size_t)t + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+        if (q >= npairs) {
+          done = true;
+        } else {
+          k = a.list ? a.list[lbase + q] : (uint32_t)q;
+          const uint32_t i1 = a.ia[k], i2 = a.ib[k];
+          if (i1 >= a.nshapes || i2 >= a.nshapes) {
+            atomicOr(a.bad_index, 1u);
+          } else {
+            c.g1 = load_shape(a.shapes, i1);
+            c.g2 = load_shape(a.shapes, i2);
+            c.m1 = load_pose(a.poses, i1);
+            c.m2 = load_pose(a.poses, i2);
+            it = 0;
+            f3 d0 = c.m1.t - c.m2.t;
+            if (c.g1.type == NCX_BALL && c.g2.type == NCX_BALL) {
+              const float d2 = norm_sq(c.m2.t - c.m1.t), sr = c.g1.a + c.g2.a;
+              write(d2 <= sr * sr ? 0.f : __builtin_sqrtf(d2) - sr);
+            } else {
+              const f3 idir = load_init_dir(a, k);
+              warm = idir.x != 0.f || idir.y != 0.f || idir.z != 0.f;
+              if (warm) d0 = idir;
+              begin(d0);
+              live = true;
+            }
+          }
+        }
+      }
+    }
+    if (__ballot(live) == 0) continue;
+    const CSO cso = cso_wave<DW_G>(c, g.dir, a.P, live);
+    if (live && gjk_step<false>(g, s, cso, NCX_FLT_MAX, warm ? a.max_iter : 10000, r)) {
+      it += r.iters;
+      if (warm && r.status == GJK_S_CAP && a.max_iter < 10000) {
+        warm = false;
+        begin(c.m1.t - c.m2.t);
+      } else {
+        write(r.status == GJK_S_CLOSEST ? norm(r.p1 - r.p2) : 0.f);
+        live = false;
+      }
     }
   }
 }
@@ -755,13 +846,13 @@ static int rerun_overflows(ContactTiers& T, ncx_ctx* ctx, KArgs a, uint32_t n, c
 // record on the 44-vertex arena (variants 0-2), and G = 8, 16 on the 24-vertex arena (variants
 // 3-4); every variant holds 8 records per block.  The small arena's hold more records per CU and
 // send more of them to the second tier, which the tuner times with them.  Distance queries have no
-// arena: 128-thread variants with 8, 16, 32, 4 or 2 lanes per pair.
+// arena: 128-thread variants with 8, 16, 32 or 4 lanes per pair, and one pair a lane (variant 4).
 static const int T1_NVARIANTS[2] = {NCX_T1_VARIANTS, NCX_T1_VARIANTS};
-static const int T1_VARIANT_G[2][NCX_T1_VARIANTS] = {{8, 16, 32, 8, 16}, {8, 16, 32, 4, 2}};
+static const int T1_VARIANT_G[2][NCX_T1_VARIANTS] = {{8, 16, 32, 8, 16}, {8, 16, 32, 4, 1}};
 static const int T1_VARIANT_BS[2][NCX_T1_VARIANTS] = {{64, 128, 256, 64, 128}, {128, 128, 128, 128, 128}};
-// contact: the resident blocks (LDS); distance: twice the resident blocks (VGPRs: 8 waves)
+// contact: the resident blocks (LDS); distance: twice the resident blocks (VGPRs: 8 waves), or they
 static const unsigned T1_BLOCKS_PER_CU[2][NCX_T1_VARIANTS] = {{T1_BLOCKS, T1_BLOCKS, T1_BLOCKS, T1S_BLOCKS, T1S_BLOCKS},
-                                                               {8, 8, 8, 8, 8}};
+                                                               {8, 8, 8, 8, 4}};
 // Lanes per pair of the GJK kernel by vertex-count bucket: without hulls the supports are closed
 // forms and a group's lanes would only repeat each other.
 static const int GJK_BUCKET_G[NCX_NBUCKETS] = {1, 4, 4, 8};
@@ -787,7 +878,7 @@ static int launch_distance(int variant, ncx_ctx* ctx, const KArgs& a, size_t n) 
     case 0: hipLaunchKernelGGL((k_distance<8, 128>), dim3(blocks), dim3(128), 0, ctx->stream, a); break;
     case 2: hipLaunchKernelGGL((k_distance<32, 128>), dim3(blocks), dim3(128), 0, ctx->stream, a); break;
     case 3: hipLaunchKernelGGL((k_distance<4, 128>), dim3(blocks), dim3(128), 0, ctx->stream, a); break;
-    case 4: hipLaunchKernelGGL((k_distance<2, 128>), dim3(blocks), dim3(128), 0, ctx->stream, a); break;
+    case 4: hipLaunchKernelGGL((k_distance_wave<128>), dim3(blocks), dim3(128), 0, ctx->stream, a); break;
     default: hipLaunchKernelGGL((k_distance<16, 128>), dim3(blocks), dim3(128), 0, ctx->stream, a); break;
   }
   NCX_HIP_CHECK(hipGetLastError());

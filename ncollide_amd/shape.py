@@ -112,7 +112,7 @@ class ShapeSet:
     # first-tier variants: (lanes per pair, EPA arena vertices)
     VARIANTS = ((8, 44), (16, 44), (32, 44), (8, 24), (16, 24))
     # distance queries have no EPA arena: lanes per pair of each variant
-    DISTANCE_VARIANTS = ((8, 0), (16, 0), (32, 0), (4, 0), (2, 0))
+    DISTANCE_VARIANTS = ((8, 0), (16, 0), (32, 0), (4, 0), (1, 0))
 
     def tuning(self, query="contact"):
         """The autotuner's choice per vertex-count bucket (no hull, <= 32, <= 96, more vertices):
