@@ -197,78 +197,12 @@ struct MDArgs {
   uint32_t* work;  // query counter (zero at launch)
 };
 
-// Bounds on the distance to the query shape, in the mesh frame: c its origin there, rot its
-// rotation, radius its bounding radius about the origin.  They skip boxes and triangles whose
-// distance provably cannot be below the best so far: GJK's result for a triangle is the norm of a
-// point of the Minkowski difference, so it is not below any bound on it, up to the rounding of
-// coordinates that `slack` (times their size) covers.  The boxes' own bound (msum_dist) is loose
-// where the shape does not fill its box: with it alone a query over a terrain of 0.1 cells ran GJK
-// on most triangles under the shape's box.
-struct MDBound {
-  f3 c;
-  quat rot;
-  float radius, size;
-};
-#define MD_SLACK (32.f * NCX_FLT_EPS)
-
-__device__ __forceinline__ float abs_sum(f3 v) { return fabsf(v.x) + fabsf(v.y) + fabsf(v.z); }
-
-// Distance from the shape's bounding ball to a box.
-__device__ __forceinline__ float md_box_bound(const MDBound& b, f3 mn, f3 mx) {
-  const f3 d = f3{fmaxf(fmaxf(mn.x - b.c.x, b.c.x - mx.x), 0.f), fmaxf(fmaxf(mn.y - b.c.y, b.c.y - mx.y), 0.f),
-                  fmaxf(fmaxf(mn.z - b.c.z, b.c.z - mx.z), 0.f)};
-  const float l = norm(d);
-  return (l - b.radius) - MD_SLACK * (l + b.size);
-}
-
-// The shape's support value along the unit direction u, about its origin.
-__device__ __forceinline__ float md_extent(const MDBound& b, const ShapeD& g, f3 u, const Pool& P, f3& at) {
-  if (g.type == NCX_BALL) return b.radius;
-  const f3 l = qrot_inv(b.rot, u);
-  if (g.type == NCX_CUBOID) return fabsf(g.a * l.x) + fabsf(g.b * l.y) + fabsf(g.c * l.z);
-  if (g.type == NCX_CAPSULE) return fabsf(g.a * l.y) + fabsf(g.b);
-  const uint32_t v = g.off + hull_support_id<1>(P, g.off, g.cnt, l, 0);
-  const f3 p = f3{P.x[v], P.y[v], P.z[v]};
-  at = qrot(b.rot, p);
-  return dot(p, l);
-}
-
-// A lower bound on the distance of a triangle and the shape: their separation along directions
-// from points of the shape to the triangle's points closest to them.  Any direction gives a bound;
-// these are the shape's origin (exact for a ball), then, once or twice, the point of the shape
-// closest to the triangle's point (a cuboid, a capsule's segment) or the support point (a hull).
-__device__ __forceinline__ float md_tri_bound(const MDBound& b, const ShapeD& g, f3 A, f3 B, f3 C, const Pool& P) {
-  const f3 a = A - b.c, bb = B - b.c, cc = C - b.c;
-  const float slack = MD_SLACK * (abs_sum(a) + abs_sum(bb) + abs_sum(cc) + b.size);
-  const int rounds = g.type == NCX_BALL ? 1 : (g.type == NCX_CONVEX_HULL ? 2 : 3);
-  f3 s = f3{0.f, 0.f, 0.f};
-  float bound = -NCX_FLT_MAX;
-  for (int i = 0; i < rounds; ++i) {
-    Loc loc;
-    f3 u;
-    float nl;
-    const f3 q = proj_triangle(a - s, bb - s, cc - s, loc);
-    if (!try_normalize(q, 0.f, &u, &nl)) break;
-    f3 at = s;
-    const float h = md_extent(b, g, u, P, at);
-    bound = fmaxf(bound, fminf(fminf(dot(a, u), dot(bb, u)), dot(cc, u)) - h);
-    if (g.type == NCX_CONVEX_HULL) {
-      s = at;
-    } else {
-      const f3 l = qrot_inv(b.rot, q + s);
-      const f3 n = g.type == NCX_CUBOID ? f3{fabsf(g.a), fabsf(g.b), fabsf(g.c)} : f3{0.f, fabsf(g.a), 0.f};
-      s = qrot(b.rot, f3{fminf(fmaxf(l.x, -n.x), n.x), fminf(fmaxf(l.y, -n.y), n.y), fminf(fmaxf(l.z, -n.z), n.z)});
-    }
-  }
-  return bound - slack;
-}
-
 #define MD_G 16
 #define MD_BLOCK 128
 #define MD_STACK 400
 #define MD_RAW 64
 #define MD_KEEP 32
-#define MD_BLOCKS_PER_CU 4u  // resident: 254 VGPRs, two wavefronts per SIMD
+#define MD_BLOCKS_PER_CU 4u  // resident: two wavefronts per SIMD
 
 template <int G> __device__ __forceinline__ float group_min(float v) {
   v = fminf(v, __uint_as_float(lane_across<1>(__float_as_uint(v))));
@@ -277,19 +211,49 @@ template <int G> __device__ __forceinline__ float group_min(float v) {
   if constexpr (G >= 16) v = fminf(v, __uint_as_float(lane_across<8>(__float_as_uint(v))));
   return v;
 }
+template <int G> __device__ __forceinline__ uint32_t group_min(uint32_t v) {
+  v = min(v, lane_across<1>(v));
+  v = min(v, lane_across<2>(v));
+  if constexpr (G >= 8) v = min(v, lane_across<4>(v));
+  if constexpr (G >= 16) v = min(v, lane_across<8>(v));
+  return v;
+}
+
+// The answer so far of one query.  The reference takes the triangles by increasing cost m (msum_dist
+// of their box), those of equal cost by id here, and stops at the first whose cost is not below the
+// least distance d so far.  GJK in f32 can report a distance below the cost, zero above all, for a
+// triangle that is large next to the shape; the reference then stops at that triangle if it comes
+// to it.  So its answer is the d of the triangle with the least (max(d, m), m, id): a triangle whose
+// cost is above that maximum comes after the one that has it, and no order of visiting changes
+// which one that is.
+struct MDBest {
+  float cut, m, d;  // the maximum, the cost, the distance
+  uint32_t id;
+  __device__ __forceinline__ void start() {
+    cut = d = NCX_FLT_MAX;
+    m = -1.f;  // a cost of NCX_FLT_MAX is not below the first distance either
+    id = 0u;
+  }
+  // whether a triangle or a box of cost c can still matter; a zero cost with a zero distance ends it
+  __device__ __forceinline__ bool reaches(float c) const { return c < cut || (c == cut && c <= m && cut > 0.f); }
+  __device__ __forceinline__ bool reaches(float c, uint32_t i) const {
+    return c < cut || (c == cut && cut > 0.f && (c < m || (c == m && i < id)));
+  }
+};
 
 // Distance of each query, one group of G lanes per query: a search of the tree that skips boxes and
-// triangles whose distance cannot be below the best so far; GJK on a triangle stops once its own
-// lower bound says so.
+// triangles whose cost says that the reference's search does not come to them.  Nothing but the cost
+// may skip a triangle: bounds on the true distance are closer (with them and with GJK stopped at
+// them 65,536 mixed shapes over a terrain of 131,072 triangles took 4.7 ms), but GJK's result can
+// lie below the true distance, and which triangles such a bound skipped depended on the order in
+// which lanes came to them.
 // What bounds it: the latency of node and triangle fetches and of GJK's steps, which a query needs
 // a few hundred of, one after another.  So the lanes of a group work on different things: each
-// takes a node of the group's stack (in LDS, nearer children on top), or a triangle to bound, or a
+// takes a node of the group's stack (in LDS, nearer children on top), or a triangle to test, or a
 // triangle to run GJK on by itself.  The three kinds of step are kept apart, in lists of LDS, and
 // run when most groups of the wavefront have enough of them, because a step that one lane takes
 // costs the wavefront as much as one that all do.
-// 65,536 mixed shapes over a terrain of 131,072 triangles: 50 ms with one search per 2 lanes and the
-// boxes' bound alone, 22 ms with the bounds above, 15 ms with the kinds of step apart, 5.3 ms with
-// 8 lanes on different nodes and triangles, 4.8 ms with 16.
+// The shapes over a terrain above: 50 ms with one search per 2 lanes, 8.1 ms so.
 template <int G>
 __global__ __launch_bounds__(MD_BLOCK) void k_md(MDArgs a) {
   constexpr int GROUPS = 64 / G, REFILL = GROUPS / 4;
@@ -307,15 +271,15 @@ __global__ __launch_bounds__(MD_BLOCK) void k_md(MDArgs a) {
   m1.q = quat{a.mesh_pose.qi, a.mesh_pose.qj, a.mesh_pose.qk, a.mesh_pose.qw};
   bool live = false, done = false;
   uint32_t q = 0;
-  int sp = 0, nr = 0, nk = 0;  // stack, raw triangles, bounded triangles
-  float best = NCX_FLT_MAX;
+  int sp = 0, nr = 0, nk = 0;  // stack, raw triangles, tested triangles
+  MDBest best;
+  best.start();
   Ctx2 c;
   c.m1 = m1;
   c.g1.type = SHAPE_TRIANGLE;
   c.g1.off = 0;
   c.g1.cnt = 0;
   c.g1.a = c.g1.b = c.g1.c = 0.f;
-  MDBound bd;
   f3 shift, margin;
   auto mask_of = [&](bool v) { return (uint32_t)(__ballot(v) >> gbase) & gmask; };
   for (;;) {
@@ -345,16 +309,12 @@ __global__ __launch_bounds__(MD_BLOCK) void k_md(MDArgs a) {
           shape_aabb_g<G>(c.g2, ls, a.P, gl, bmn, bmx);
           shift = -((bmn + bmx) * 0.5f);  // -ls_aabb2.center() (aabb.rs:95-97)
           margin = (bmx - bmn) * 0.5f;     // ls_aabb2.half_extents() (aabb.rs:101-104)
-          bd.c = ls.t;
-          bd.rot = ls.q;
-          bd.radius = __uint_as_float(a.shapes[s].pad[0]);
-          bd.size = abs_sum(ls.t) + abs_sum(m1.t) + abs_sum(c.m2.t) + bd.radius;
-          best = NCX_FLT_MAX;
+          best.start();
           nk = 0;
           sp = a.ntri > 1 ? 1 : 0;
           nr = a.ntri > 1 ? 0 : 1;
           if (gl == 0) {
-            stk[0] = uint2{0u, __float_as_uint(-NCX_FLT_MAX)};
+            stk[0] = uint2{0u, __float_as_uint(0.f)};
             raw[0] = 0u;
           }
         }
@@ -374,21 +334,20 @@ __global__ __launch_bounds__(MD_BLOCK) void k_md(MDArgs a) {
         uint2 e = uint2{0u, 0u};
         if (have) e = stk[sp - 1 - gl];
         sp -= p;
-        have = have && __uint_as_float(e.y) < best;
+        have = have && best.reaches(__uint_as_float(e.y));
         bool inner0 = false, inner1 = false, leaf0 = false, leaf1 = false;
         uint32_t c0 = 0, c1 = 0;
         float k0 = 0.f, k1 = 0.f;
         if (have) {
           const LNode nd = a.nodes[e.x];
-          auto key = [&](f3 mn, f3 mx) { return fmaxf(msum_dist(mn, mx, shift, margin), md_box_bound(bd, mn, mx)); };
-          const float cl = key(f3{nd.lminx, nd.lminy, nd.lminz}, f3{nd.lmaxx, nd.lmaxy, nd.lmaxz});
-          const float cr = key(f3{nd.rminx, nd.rminy, nd.rminz}, f3{nd.rmaxx, nd.rmaxy, nd.rmaxz});
+          const float cl = msum_dist(f3{nd.lminx, nd.lminy, nd.lminz}, f3{nd.lmaxx, nd.lmaxy, nd.lmaxz}, shift, margin);
+          const float cr = msum_dist(f3{nd.rminx, nd.rminy, nd.rminz}, f3{nd.rmaxx, nd.rmaxy, nd.rmaxz}, shift, margin);
           const bool lfirst = cl <= cr;
           c0 = lfirst ? nd.child_l : nd.child_r;
           c1 = lfirst ? nd.child_r : nd.child_l;
           k0 = lfirst ? cl : cr;
           k1 = lfirst ? cr : cl;
-          const bool h0 = k0 < best, h1 = k1 < best;
+          const bool h0 = best.reaches(k0), h1 = best.reaches(k1);
           leaf0 = h0 && (c0 & NCX_LEAF_BIT);
           leaf1 = h1 && (c1 & NCX_LEAF_BIT);
           inner0 = h0 && !leaf0;
@@ -411,27 +370,22 @@ __global__ __launch_bounds__(MD_BLOCK) void k_md(MDArgs a) {
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       if (2 * __popcll(am) < __popcll(__ballot(live))) break;
     }
-    // bounds of the triangles reached
+    // costs of the triangles reached
     if (live && nr > 0 && nk + G <= MD_KEEP) {
       const int p = min(G, nr);
       bool ok = gl < p;
       uint32_t k = 0;
       if (ok) k = raw[nr - 1 - gl];
       nr -= p;
-      float bound = 0.f;
+      float m = 0.f;
       if (ok) {
-        f3 ta, tb, tc;
-        tri_vertices(a.P, k, ta, tb, tc);
-        const f3 mn = f3{fminf(fminf(ta.x, tb.x), tc.x), fminf(fminf(ta.y, tb.y), tc.y), fminf(fminf(ta.z, tb.z), tc.z)};
-        const f3 mx = f3{fmaxf(fmaxf(ta.x, tb.x), tc.x), fmaxf(fmaxf(ta.y, tb.y), tc.y), fmaxf(fmaxf(ta.z, tb.z), tc.z)};
-        ok = msum_dist(mn, mx, shift, margin) < best;
-        if (ok) {
-          bound = md_tri_bound(bd, c.g2, ta, tb, tc, a.P);
-          ok = !(bound > best);
-        }
+        f3 mn, mx;
+        tri_box(a.tris, k, mn, mx);
+        m = msum_dist(mn, mx, shift, margin);
+        ok = best.reaches(m);
       }
       const uint32_t km = mask_of(ok);
-      if (ok) keep[nk + __popc(km & below)] = uint2{k, __float_as_uint(bound)};
+      if (ok) keep[nk + __popc(km & below)] = uint2{k, __float_as_uint(m)};
       nk += __popc(km);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -442,32 +396,42 @@ __global__ __launch_bounds__(MD_BLOCK) void k_md(MDArgs a) {
     if (rm && 2 * __popcll(rm) >= __popcll(__ballot(more))) {
       if (ready) {
         const int p = min(G, nk);
-        bool ok = gl < p;
+        const bool mine = gl < p;
         uint2 e = uint2{0u, 0u};
-        if (ok) e = keep[nk - 1 - gl];
+        if (mine) e = keep[nk - 1 - gl];
         nk -= p;
+        const float m = __uint_as_float(e.y);
         float d = NCX_FLT_MAX;
-        if (ok && !(__uint_as_float(e.y) > best)) {
+        uint32_t id = 0xFFFFFFFFu;
+        if (mine) id = __float_as_uint(a.tris[3 * (size_t)e.x].w);
+        if (mine && best.reaches(m, id)) {
           // query::distance(m1, triangle, m2, g2): distance_support_map_support_map (GJK from
           // m1.t - m2.t, distance_support_map_support_map.rs:25-53)
-          f3 ta, tb, tc;
-          tri_vertices(a.P, e.x, ta, tb, tc);
           c.g1.off = e.x;
           f3 dir;
           float nl;
           if (!try_normalize(c.m1.t - c.m2.t, NCX_FLT_EPS, &dir, &nl)) dir = f3{1.f, 0.f, 0.f};
           Simplex sx;
-          const float limit = best + MD_SLACK * (best + abs_sum(ta) + abs_sum(tb) + abs_sum(tc) + bd.size);
-          const GJKOut r = gjk<1>(c, dir, limit, sx, a.P, 0, 10000);
-          if (r.status != GJK_S_NOINTER)  // else farther than the best
-            d = r.status == GJK_S_CLOSEST ? norm(r.p1 - r.p2) : 0.f;
+          const GJKOut r = gjk<1>(c, dir, NCX_FLT_MAX, sx, a.P, 0, 10000);
+          d = r.status == GJK_S_CLOSEST ? norm(r.p1 - r.p2) : 0.f;
         }
-        d = group_min<G>(d);
-        if (d < best) best = d;
+        // the least (max(d, m), m, id) of the lanes; a distance that is no number counts as none
+        const bool has = d < NCX_FLT_MAX;
+        const float cut = has ? fmaxf(d, m) : NCX_FLT_MAX, gcut = group_min<G>(cut);
+        const float gm = group_min<G>(has && cut == gcut ? m : NCX_FLT_MAX);
+        const bool cand = has && cut == gcut && m == gm;
+        const uint32_t gid = group_min<G>(cand ? id : 0xFFFFFFFFu);
+        const float gd = group_min<G>(cand && id == gid ? d : NCX_FLT_MAX);
+        if (gcut < best.cut || (gcut == best.cut && (gm < best.m || (gm == best.m && gid < best.id)))) {
+          best.cut = gcut;
+          best.m = gm;
+          best.id = gid;
+          best.d = gd;
+        }
       }
     }
     if (live && sp == 0 && nr == 0 && nk == 0) {
-      if (gl == 0) a.dist[q] = best;
+      if (gl == 0) a.dist[q] = best.d;
       live = false;
     }
   }

@@ -618,7 +618,7 @@ __device__ __forceinline__ uint32_t pair_key(const ncx_shape* __restrict__ shape
 }
 
 // Bounding radius of each shape about its local origin, into pad[0] of its device record, for the
-// sort key and the mesh distance search's bounds.
+// sort key.
 __global__ __launch_bounds__(256) void k_shape_radius(ncx_shape* __restrict__ shapes, size_t n, Pool P) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
