@@ -394,7 +394,9 @@ int ncx_world_stored_aabbs(ncx_world* world, const float** soa_dev);
  * ncx_world_first_interference_with_rays: first_interference_with_ray (glue/query.rs:200-224 ->
  * dbvt_broad_phase.rs:433-460, RayIntersectionCostFnVisitor ray_intersection_cost_fn_visitor.rs:
  * 64-107): per ray the hit with the least toi (then the least handle: the reference keeps the
- * first of equal-toi hits its heap pops), handle UINT32_MAX and toi -1 on a miss.  Batches of
+ * first of equal-toi hits its heap pops), handle UINT32_MAX and toi -1 on a miss.  A hit before its
+ * own stored box's entry (a cast's rounding on a shape the ray grazes) counts only if no other is as
+ * early as that entry: the least (max(toi, entry), toi, handle) is returned.  Batches of
  * 1,024 rays or more are searched in an order sorted by origin and direction octant, with
  * about 16 bytes per ray of sort buffers kept by the world; results go to each ray's own slot.
  * ncx_world_interferences_with_aabbs: glue::interferences_with_aabb (glue/query.rs) = the stored

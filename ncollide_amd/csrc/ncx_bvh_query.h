@@ -7,8 +7,8 @@
 // Each lane walks the tree depth-first with its own stack (the tree is at most LBVH_MAX_DEPTH
 // levels deep, so the stack never holds more entries than that).  The collectors run twice: a
 // count pass, then, after a scan, a write pass to each query's slots.  The first-hit search
-// visits the nearer child first and skips boxes entered after the best hit so far; the hit kept
-// is the least (toi, handle), so the result does not depend on the visiting order.
+// visits the nearer child first and skips boxes entered after the best hit so far, with a result
+// that does not depend on the visiting order (k_bq_first_ray).
 #pragma once
 #include "ncx_gjk.h"
 
@@ -157,7 +157,13 @@ __global__ __launch_bounds__(BQ_BLOCK) void k_bq_collect(BQArgs a) {
 }
 
 // First hit of each ray among the proxies' shapes (solid = true, toi <= max_toi): the least
-// (toi, handle) over the leaves whose box the ray enters no later than the best hit so far.
+// (toi, handle) over the leaves whose box the ray enters no later than the best hit so far, taken by
+// the boxes' entry tois as the reference's best-first search does.  A cast can report a toi below
+// its own box's entry -- GJK's on a capsule or hull by up to its absolute tolerance of 1e-3, a ball's
+// closed form where the ray starts hundreds of radii away -- and such a hit counts only if no other
+// is as early as its box's entry.  So the hit kept is the one with the least (max(toi, entry), toi,
+// handle), and a box is skipped when its entry is past that maximum: a rule without an order, while
+// the leaves come in an order that depends on the wavefront's other rays.
 // What bounds it: the ray casts on capsules and hulls (GJK, 7 to 20 iterations), and divergence --
 // the rays of a wavefront reach them at different times, and a cast that one lane does alone takes
 // as long as one that all do.  So one lane walks the tree for one ray; balls and cuboids (closed
@@ -183,10 +189,12 @@ static __global__ __launch_bounds__(BQ_BLOCK, 3) void k_bq_first_ray(BQArgs a) {
   bool live = false, done = false, walk = false;
   uint32_t qi = 0, node = 0, best_h = BQ_NONE, kh0 = 0, kh1 = 0;
   int sp = 0, nk = 0;
-  float best_t = 0.f, kt0 = 0.f, kt1 = 0.f;
+  float cut = 0.f, best_t = 0.f, kt0 = 0.f, kt1 = 0.f;
   f3 o = f3{0.f, 0.f, 0.f}, dir = o, best_n = o;
-  auto hit = [&](uint32_t h, float t, f3 n) {
-    if (t < best_t || (t == best_t && h < best_h)) {
+  auto hit = [&](uint32_t h, float entry, float t, f3 n) {
+    const float c = t < entry ? entry : t;
+    if (c < cut || (c == cut && (t < best_t || (t == best_t && h < best_h)))) {
+      cut = c;
       best_t = t;
       best_h = h;
       best_n = n;
@@ -208,7 +216,7 @@ static __global__ __launch_bounds__(BQ_BLOCK, 3) void k_bq_first_ray(BQArgs a) {
       float t;
       f3 n;
       uint32_t feat;
-      if (shape_ray_cast_closed(g, m, o, dir, a.max_toi, true, t, n, feat)) hit(h, t, n);
+      if (shape_ray_cast_closed(g, m, o, dir, a.max_toi, true, t, n, feat)) hit(h, entry, t, n);
     }
   };
   auto push = [&](uint32_t child, float entry) {
@@ -238,7 +246,7 @@ static __global__ __launch_bounds__(BQ_BLOCK, 3) void k_bq_first_ray(BQArgs a) {
           qi = a.perm ? a.perm[gi] : gi;
           o = f3{a.q[0][qi], a.q[1][qi], a.q[2][qi]};
           dir = f3{a.q[3][qi], a.q[4][qi], a.q[5][qi]};
-          best_t = a.max_toi;
+          cut = best_t = a.max_toi;
           best_h = BQ_NONE;
           best_n = f3{0.f, 0.f, 0.f};
           sp = nk = 0;
@@ -265,8 +273,8 @@ static __global__ __launch_bounds__(BQ_BLOCK, 3) void k_bq_first_ray(BQArgs a) {
           const bool hl = bq_ray_box(o, dir, a.max_toi, nd.lminx, nd.lminy, nd.lminz, nd.lmaxx, nd.lmaxy, nd.lmaxz, cl);
           const bool hr = bq_ray_box(o, dir, a.max_toi, nd.rminx, nd.rminy, nd.rminz, nd.rmaxx, nd.rmaxy, nd.rmaxz, cr);
           const bool lfirst = hl && (!hr || cl <= cr);
-          const bool h0 = (lfirst ? hl : hr) && (lfirst ? cl : cr) <= best_t;
-          const bool h1 = (lfirst ? hr : hl) && (lfirst ? cr : cl) <= best_t;
+          const bool h0 = (lfirst ? hl : hr) && (lfirst ? cl : cr) <= cut;
+          const bool h1 = (lfirst ? hr : hl) && (lfirst ? cr : cl) <= cut;
           const uint32_t c0 = lfirst ? nd.child_l : nd.child_r, c1 = lfirst ? nd.child_r : nd.child_l;
           const float t1 = lfirst ? cr : cl;
           if (h0) {
@@ -287,7 +295,7 @@ static __global__ __launch_bounds__(BQ_BLOCK, 3) void k_bq_first_ray(BQArgs a) {
             if (sp < BQ_LDS_STACK) e = lstk[sp][threadIdx.x];
             else e = deep[sp - BQ_LDS_STACK];
             next_t = __uint_as_float(e.y);
-            if (!(next_t <= best_t)) continue;
+            if (!(next_t <= cut)) continue;
             next = e.x;
           }
           if (!(next & NCX_LEAF_BIT)) break;
@@ -309,13 +317,13 @@ static __global__ __launch_bounds__(BQ_BLOCK, 3) void k_bq_first_ray(BQArgs a) {
       kh0 = kh1;
       kt0 = kt1;
       --nk;
-      if (entry <= best_t) {
+      if (entry <= cut) {
         float t;
         f3 n;
         uint32_t feat;
         if (shape_ray_cast<1>(load_shape(a.shapes, h), load_pose(a.poses, h), o, dir, a.max_toi, true, a.P, 0, snap, t,
                               n, feat))
-          hit(h, t, n);
+          hit(h, entry, t, n);
       }
     }
     if (live && nk == 0 && !walk) {

@@ -40,3 +40,56 @@ def test_world_first_rays_edges(ctx, orc, nshapes, nrays, box):
         assert np.array_equal(h.cpu().numpy().view(np.uint32), rh)
         assert np.array_equal(t.cpu().numpy().view(np.uint32), rt.view(np.uint32))
         assert np.array_equal(n.cpu().numpy().view(np.uint32), rn.view(np.uint32))
+
+
+def _entries(boxes, o, d):
+    """AABB::toi_with_ray (solid) of boxes the rays hit, in f32."""
+    with np.errstate(divide="ignore", invalid="ignore"):
+        inv = np.float32(1) / d
+        a, b = (boxes[:, :3] - o) * inv, (boxes[:, 3:] - o) * inv
+    return np.where(d != 0, np.minimum(a, b), 0).max(1).clip(min=0)
+
+
+@pytest.mark.parametrize("size,away,early_hits", [(1.0, 3.0, 100), (0.05, 0.3, 30000), (8.0, 30.0, 0), (0.5, 100.0, 1000)])
+def test_hits_before_their_boxes(ctx, orc, size, away, early_hits):
+    """Casts that report a toi below their own box's entry (grazing capsules and hulls, small ones above
+    all; balls from far away) in a crowd with tight boxes: the hit is the one with the least
+    (max(toi, entry), toi, handle), whatever rays share a wavefront."""
+    rng = np.random.default_rng(int(10 * size))
+    n, nrays = 3000, 20000
+    w = workloads.full_pipeline(seed=9, n=n, box=10.0, nclusters=1)
+    rec, pool = w["records"], (w["pool"] * size).astype(np.float32)
+    for k in ("p0", "p1", "p2"):
+        rec[k] *= size
+    t = rng.uniform(0, 6.0 * size, (n, 3))
+    p = workloads.poses8(t, workloads.uniform_quats(rng, n)).astype(np.float32)
+    ss = ncx.ShapeSet(records=rec, pool=pool, ctx=ctx)
+    world = World(ss, margin=0.0, prediction=0.0, max_pairs=1 << 21)
+    world.set_contacts(False)
+    poses = torch.as_tensor(p, device=ctx.device)
+    world.step(poses)
+    world.sync()
+    boxes = world.stored_aabbs().cpu().numpy().T.copy()
+    ro = (3.0 * size + rng.normal(0, away, (nrays, 3))).astype(np.float32)
+    rd = ((p[rng.integers(0, n, nrays), :3] + rng.normal(0, 0.3 * size, (nrays, 3)) - ro)
+          * rng.uniform(0.2, 1.5, (nrays, 1))).astype(np.float32)
+    oss = oracle_shapes(orc, rec, pool)
+    cnt, h, toi, nrm = orc.world_rays(oss, to_oracle_poses(p), boxes, ro, rd, np.float32(20.0), 1)
+    ray = np.repeat(np.arange(nrays), cnt)
+    entry = _entries(boxes[h], ro[ray], rd[ray])
+    order = np.lexsort((h, toi, np.maximum(toi, entry), ray))
+    first = order[np.unique(ray[order], return_index=True)[1]]
+    rh, rt, rn = np.full(nrays, 0xFFFFFFFF, np.uint32), np.full(nrays, -1, np.float32), np.zeros((nrays, 3), np.float32)
+    rh[ray[first]], rt[ray[first]], rn[ray[first]] = h[first], toi[first], nrm[first]
+    assert (toi < entry).sum() >= early_hits
+    for k in (np.arange(nrays), rng.permutation(nrays)):  # the second time with other rays beside each
+        gh, gt, gn = world.first_interference_with_rays(poses, ro[k], rd[k], 20.0)
+        assert np.array_equal(gh.cpu().numpy().view(np.uint32), rh[k])
+        assert np.array_equal(gt.cpu().numpy().view(np.uint32), rt[k].view(np.uint32))
+        assert np.array_equal(gn.cpu().numpy().view(np.uint32), rn[k].view(np.uint32))
+    # away from such hits the rule is the least (toi, handle) of all
+    bh, bt, _ = orc.world_rays(oss, to_oracle_poses(p), boxes, ro, rd, np.float32(20.0), 0)
+    assert size != 0.05 or (bt != rt).any()  # rays where the rule decides
+    early = np.zeros(nrays, bool)
+    early[ray[toi < entry]] = True
+    assert np.array_equal(bh[~early], rh[~early]) and np.array_equal(bt[~early], rt[~early])
