@@ -533,7 +533,7 @@ extern "C" int ncx_shapes_create(ncx_ctx* ctx, const ncx_shape* shapes, size_t n
                   "ncx_shapes_create: hull range outside the point pool");
   }
   ncx_shapes* S = new ncx_shapes;
-  S->buckets = 0;
+  S->buckets = n ? 0u : 1u;  // a set without shapes: the launch that finds every pair's index bad
   for (size_t i = 0; i < n; ++i) S->types |= 1u << shapes[i].type;
   for (size_t i = 0; i < n; ++i)
     S->buckets |= 1u << (shapes[i].type == NCX_CONVEX_HULL ? count_bucket(shapes[i].hull_count) : 0u);

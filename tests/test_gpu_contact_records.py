@@ -102,3 +102,18 @@ def test_bad_index_is_refused(types, npairs):
                  lambda: query.time_of_impact(ss, p, v, ia, ib, 1.0)):
         with pytest.raises(ncx.NcxError):
             call()
+
+
+@pytest.mark.parametrize("npairs", [1, 5000, 20000])
+def test_set_without_shapes_refuses_pairs(npairs):
+    import torch
+    import ncollide_amd as ncx
+    from ncollide_amd import query
+    from ncollide_amd.shape import SHAPE_DTYPE
+    ss = ncx.ShapeSet(records=np.zeros(0, SHAPE_DTYPE), pool=np.zeros((0, 3), np.float32))
+    p = torch.zeros((1, 8), device="cuda")
+    i = np.zeros(npairs, np.int32)
+    for call in (lambda: query.contact(ss, p, i, i, 0.0), lambda: query.distance(ss, p, i, i),
+                 lambda: query.time_of_impact(ss, p, torch.zeros((1, 3), device="cuda"), i, i, 1.0)):
+        with pytest.raises(ncx.NcxError):
+            call()
