@@ -55,6 +55,7 @@ struct DevBuf {
     size_t nb = nbytes < 256 ? 256 : nbytes;
     hipError_t e = hipMalloc(&p, nb);
     if (e != hipSuccess) {
+      (void)hipGetLastError();  // the check after a later call's launch is not to find it
       ncx_set_error(std::string("hipMalloc: ") + hipGetErrorString(e));
       return NCX_E_HIP;
     }

@@ -765,10 +765,13 @@ int contact_tiers_reserve(ContactTiers& t, ncx_ctx* ctx, size_t cap, size_t nrec
   }
   cap = std::min<size_t>(std::max<size_t>(cap, 4096), (size_t)1 << 24);
   if (cap <= t.cap) return NCX_OK;
-  t.ovf.release();
-  t.cap = 0;
-  int rc = t.ovf.reserve(4 * (NCX_OVF_HEADER + 4 * cap));
+  // the present lists stay where larger ones cannot be had: later calls, the queries without
+  // overflows among them, use the header
+  DevBuf lists;
+  int rc = lists.reserve(4 * (NCX_OVF_HEADER + 4 * cap));
   if (rc) return rc;
+  t.ovf.release();
+  t.ovf = lists;
   t.cap = (uint32_t)cap;
   return NCX_OK;
 }

@@ -1,0 +1,80 @@
+"""Host code of the batched queries when device memory runs out, without a GPU: the library on a
+stand-in for the HIP runtime (hip_stub.c) whose allocations above a limit fail."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+CHILD = """
+import ctypes as C, json, sys
+import numpy as np
+stub = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+from ncollide_amd import _lib
+lib = _lib.load()
+
+
+class Ctx(C.Structure):  # ncx_ctx
+    _fields_ = [("device", C.c_int), ("stream", C.c_void_p), ("num_cus", C.c_int)]
+
+
+ctx = Ctx(0, None, 256)
+limit = C.c_size_t.in_dll(stub, "stub_limit")
+count = lambda name: C.c_int.in_dll(stub, name).value
+rec = np.zeros((8, 8), np.uint32)  # balls
+shapes = C.c_void_p()
+assert lib.ncx_shapes_create(C.byref(ctx), rec.ctypes.data, 8, None, None, None, 0, C.byref(shapes)) == 0
+poses = np.zeros((8, 8), np.float32)
+p = poses.ctypes.data
+error = lambda: lib.ncx_last_error().decode()
+
+
+def contact(n):
+    ix = np.zeros(n, np.uint32)
+    out = np.zeros(12 * n, np.uint8)
+    return lib.ncx_contact_batch(shapes, p, ix.ctypes.data, ix.ctypes.data, n, 0.0, None, *[out.ctypes.data] * 5, None)
+
+
+def distance(n):
+    ix = np.zeros(n, np.uint32)
+    return lib.ncx_distance_batch(shapes, p, ix.ctypes.data, ix.ctypes.data, n, np.zeros(n, np.float32).ctypes.data, None)
+
+
+def impact(n):
+    ix = np.zeros(n, np.uint32)
+    out = np.zeros(12 * n, np.uint8)
+    return lib.ncx_time_of_impact_batch(shapes, p, p, ix.ctypes.data, ix.ctypes.data, n, 1.0, 0.0,
+                                        *[out.ctypes.data] * 7)
+
+
+"""
+
+
+def run(tmp_path, body):
+    stub = str(tmp_path / "hip_stub.so")
+    subprocess.check_call(["gcc", "-O1", "-shared", "-fPIC", "-o", stub, os.path.join(HERE, "hip_stub.c")])
+    r = subprocess.run([sys.executable, "-c", CHILD + body, stub], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return json.loads(r.stdout.splitlines()[-1])
+
+
+@pytest.mark.parametrize("query", ["distance", "contact"])
+@pytest.mark.parametrize("npairs", [100, 20000])
+def test_time_of_impact_after_a_refused_batch(tmp_path, npairs, query):
+    """A batch whose lists cannot grow is refused and leaves the set usable: the next query's header is
+    not at address zero."""
+    out = run(tmp_path, f"""
+limit.value = 1 << 22  # the lists of 2^19 pairs take 8 MiB
+refused = {query}(1 << 19)
+message = error()
+limit.value = (1 << 64) - 1
+rc = impact({npairs})
+print(json.dumps([refused, message, rc, count("stub_null_fills"), count("stub_launches")]))
+""")
+    refused, message, rc, null_fills, launches = out
+    assert refused != 0 and "hipMalloc" in message
+    assert (rc, null_fills) == (0, 0) and launches > 0
