@@ -339,8 +339,8 @@ int ncx_mlp_predict_dirs(ncx_mlp* mlp, const ncx_pose* poses_dev, const float* d
  * use_graph != 0, refit steps and rebuild steps (after the first step) each replay a captured
  * hipGraph.  Outputs are capacity-`max_pairs` device arrays.  Device memory: about 2.3 KB per
  * shape (2 KB of it buffers each proxy's first 512 pair partners for the pair search) plus, per pair
- * of `max_pairs`, the outputs, the contact work lists, a 112-byte EPA record, and a saved EPA run
- * for every 32nd pair (at most 2^19 of them). */
+ * of `max_pairs`, the outputs and the contact work lists, and for at most 2^26 pairs at a time (fewer
+ * where memory is short) a 112-byte EPA record, with a saved EPA run for every 32nd of them. */
 typedef struct ncx_world ncx_world;
 int ncx_world_create(ncx_ctx* ctx, ncx_shapes* shapes, float margin, float prediction, size_t max_pairs,
                      ncx_world** world);

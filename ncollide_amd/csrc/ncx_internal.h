@@ -73,8 +73,8 @@ struct DevBuf {
 // Layout of ContactTiers::ovf (uint32 words): a header, then the EPA records whose run outgrew
 // the first-tier arena, those that outgrew the second tier, the third, and the fourth (cap
 // entries each).
-// Header words [0, NCX_OVF_TIER_WORDS) are the tiers' counts and the launches' numbers of EPA
-// records (cleared between tuning samples),
+// Header words [0, NCX_OVF_TIER_WORDS) are the tiers' counts, the launches' numbers of EPA records,
+// and what is kept of a launch's earlier parts (cleared between tuning samples),
 // [NCX_OVF_TIER_WORDS, NCX_OVF_COUNTS) the partition's (which the samples read): each vertex-count
 // bucket's range in the partitioned list, and each sort key's count and scatter cursor.  From
 // NCX_WORK_BASE on come the work counters of the launches (the tuning samples' GJK, the
@@ -83,7 +83,8 @@ struct DevBuf {
 constexpr uint32_t NCX_OVERLAP_BINS = 8;  // 4 and 16 bins ordered the scene's pairs no better
 constexpr uint32_t NCX_NKEYS = 64 * NCX_OVERLAP_BINS;  // sort keys: vertex-count bucket x 16 shape-type pairs x overlap bins
 constexpr uint32_t NCX_OVF_T1_COUNT = 0, NCX_OVF_BAD = 1, NCX_OVF_T2_COUNT = 2, NCX_OVF_T3_COUNT = 3,
-                   NCX_OVF_T4_COUNT = 4, NCX_REC_COUNT = 5, NCX_REC_COUNT_TUNE = 9, NCX_OVF_TIER_WORDS = 16,
+                   NCX_OVF_T4_COUNT = 4, NCX_REC_COUNT = 5, NCX_REC_COUNT_TUNE = 9, NCX_OVF_EARLIER = 10, NCX_OVF_FULL = 11,
+                   NCX_OVF_TIER_WORDS = 16,
                    NCX_BKT_RANGE = 16, NCX_KEY_CNT = 24,
                    NCX_KEY_FILL = NCX_KEY_CNT + NCX_NKEYS, NCX_OVF_COUNTS = NCX_KEY_FILL + NCX_NKEYS;
 constexpr uint32_t NCX_WORK_SET = 64, NCX_WORK_BASE = NCX_OVF_COUNTS, NCX_WORK_TUNE = 0, NCX_WORK_T2 = 1, NCX_WORK_T3 = 2,
@@ -94,7 +95,8 @@ constexpr uint32_t NCX_WORK_SET = 64, NCX_WORK_BASE = NCX_OVF_COUNTS, NCX_WORK_T
 constexpr int NCX_NBUCKETS = 4;
 static_assert(NCX_OVF_T4_COUNT < NCX_OVF_TIER_WORDS && NCX_OVF_TIER_WORDS <= NCX_BKT_RANGE &&
                   NCX_BKT_RANGE + 2 * NCX_NBUCKETS <= NCX_KEY_CNT && NCX_NKEYS == 16 * NCX_OVERLAP_BINS * NCX_NBUCKETS &&
-                  NCX_REC_COUNT + NCX_NBUCKETS <= NCX_REC_COUNT_TUNE && NCX_REC_COUNT_TUNE < NCX_OVF_TIER_WORDS &&
+                  NCX_REC_COUNT + NCX_NBUCKETS <= NCX_REC_COUNT_TUNE && NCX_REC_COUNT_TUNE < NCX_OVF_EARLIER &&
+                  NCX_OVF_FULL < NCX_OVF_TIER_WORDS &&
                   NCX_WORK_BKT + NCX_NBUCKETS <= NCX_WORK_EPA && NCX_WORK_EPA + NCX_NBUCKETS <= NCX_WORK_SETS,
               "overflow header layout");
 // The work counter of launch k.
@@ -116,9 +118,11 @@ struct ContactTiers {
   KArgs* last = nullptr;
   DevBuf epa;        // the EPA kernels' memory:
   float* sup = nullptr;     //   support points of the polytopes in flight
-  EpaRec* rec = nullptr;    //   records, one per pair at most
+  EpaRec* rec = nullptr;    //   nrec records, one per intersecting pair of a part of the launch
   uint8_t* sus0 = nullptr;  //   saved runs handed from T1 to T2
   size_t nrec = 0;
+  size_t rec_asked = 0;     // the most records asked for
+  bool parts = false;       // the last launch took its pairs in more than one part
   DevBuf sus[4];     // saved EPA runs handed on: (unused), T2 -> T3, T3 -> T4, T4 -> device-memory tier
   uint32_t* t1_list() const { return ovf.as<uint32_t>() + NCX_OVF_HEADER; }
   uint32_t* t2_list() const { return ovf.as<uint32_t>() + NCX_OVF_HEADER + cap; }

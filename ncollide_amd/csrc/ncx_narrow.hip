@@ -42,12 +42,12 @@ struct KArgs {
   uint8_t* arena;       // device-memory tier: EPA arenas of vcap vertices and fcap faces
   uint32_t vcap, fcap;
   EpaRec* rec;               // EPA records: GJK writes them, the EPA kernels read them
-  const uint32_t* rec_base;  // optional device offset into rec of this launch's records
   uint32_t* rec_count;       // their number
   float* sup;                // per EPA group: its polytope's support points, 6 floats a vertex
   uint32_t* ovf_count;  // EPA runs that outgrew the arena
   uint32_t* ovf_list;   // their records (first ovf_cap of them)
   uint32_t ovf_cap;
+  int ovf_pairs;        // the list holds the runs' pairs instead
   int distance_mode;
   uint32_t nshapes;
   uint32_t* bad_index;  // set to 1 when a pair names a shape >= nshapes
@@ -55,6 +55,7 @@ struct KArgs {
   uint32_t* work;         // work counter (zero at launch): pairs and records are taken from it
   const uint32_t* range_b;  // optional device begin and end into list: a run of buckets
   const uint32_t* range_e;
+  uint32_t part_lo, part_hi;  // the part of that list the launch takes (contacts)
   const uint8_t* sus_load;  // saved EPA runs of the list's ENTRY_SAVED entries, slot = list position
   size_t sus_load_bytes;
   uint8_t* sus_save;        // slots for runs this launch suspends (LDS tiers only; null: none)
@@ -140,12 +141,13 @@ __global__ __launch_bounds__(GJK_BS, 2) void k_contact_gjk(KArgs a) {
   const int lane = threadIdx.x & 63, gl = lane & (G - 1);
   size_t npairs = a.npairs;
   if (a.n_dev) npairs = min(npairs, (size_t)*a.n_dev);
-  size_t lbase = 0;
+  size_t lbase = 0, rbase = 0;
   if (a.range_b) {
-    lbase = *a.range_b;
-    npairs = *a.range_e - lbase;
+    lbase = max(*a.range_b, a.part_lo);
+    const size_t end = min(*a.range_e, a.part_hi);
+    npairs = end > lbase ? end - lbase : 0;
+    rbase = lbase - a.part_lo;
   }
-  const size_t rbase = a.rec_base ? *a.rec_base : 0;
   for (;;) {
     const size_t q = next_pairs<G>(a.work, lane);
     if (__ballot(q < npairs) == 0) break;
@@ -231,7 +233,8 @@ __device__ __forceinline__ void epa_write(const KArgs& a, uint32_t k, uint32_t k
 // lanes, one record per group at a time.  Every pass of the loop runs one iteration of each group's record; groups without one take
 // the next records together, with one atomic per wavefront, once REFILL of them wait or none runs.
 // SAVES: a run about to outgrow the arena is saved for the next tier.  LISTED: the records come
-// from the overflow list of the tier before (entries may be saved runs), otherwise from rec_base on.
+// from the overflow list of the tier before (entries may be saved runs), otherwise those that the GJK
+// launch of the same bucket wrote, from the place of its first pair in the part on.
 template <int G, int BS, class L, int REFILL, bool SAVES, bool LISTED>
 __global__ __launch_bounds__(BS, 1) void k_epa(KArgs a) {
   static_assert(ilog2_floor(L::HC) <= (uint32_t)G, "the heap steps need a lane per heap level");
@@ -242,7 +245,7 @@ __global__ __launch_bounds__(BS, 1) void k_epa(KArgs a) {
   A.p = lds + (threadIdx.x / G) * L::BYTES;
   float* const sup = a.sup + ((size_t)blockIdx.x * (BS / G) + threadIdx.x / G) * (6 * (size_t)L::VC);
   uint32_t n = LISTED ? min(*a.n_dev, a.ovf_cap) : *a.rec_count;
-  const uint32_t rbase = !LISTED && a.rec_base ? *a.rec_base : 0u;
+  const uint32_t rbase = !LISTED && a.range_b ? max(*a.range_b, a.part_lo) - a.part_lo : 0u;
   bool live = false, done = false;
   Ctx2 c;
   EpaState<L> s;
@@ -293,7 +296,7 @@ __global__ __launch_bounds__(BS, 1) void k_epa(KArgs a) {
               epa_write_saved<G>(a.sus_save + (size_t)slot * a.sus_save_bytes, A, sup, s, gl);
             }
           }
-          if (gl == 0 && slot < a.ovf_cap) a.ovf_list[slot] = rec | (saved ? ENTRY_SAVED : 0u);
+          if (gl == 0 && slot < a.ovf_cap) a.ovf_list[slot] = a.ovf_pairs ? k : rec | (saved ? ENTRY_SAVED : 0u);
         } else if (gl == 0) {
           f3 p1 = f3{0.f, 0.f, 0.f}, p2 = p1, nn = f3{0.f, 1.f, 0.f};
           if (st == EPA_FACE) {
@@ -740,20 +743,36 @@ static_assert(ArenaT1::FC + 2 <= ArenaT1::HC && ArenaT1S::HC <= ArenaT1::HC, "a 
 static_assert(ArenaT2::FC + 2 <= ArenaT2::HC && ArenaT3::FC + 2 <= ArenaT3::HC && ArenaT4::FC + 2 <= ArenaT4::HC,
               "a saved run's faces");
 
+// Records of a launch: for one of more pairs it goes over them in parts.  A part of 2^26 pairs has
+// 7.5 GB of records; fewer where that much memory cannot be had, down to REC_LEAST (15 MB).  A part
+// costs about 0.3 ms also where a scene has no pairs for it (three parts of 2^24 pairs: a step of a
+// 1,048,576-shape scene with room for 42 M pairs 42.0 -> 42.7 ms).
+static const size_t REC_MOST = (size_t)1 << 26, REC_LEAST = (size_t)1 << 17;
+
 // Overflow lists of at least cap entries each (at most 2^24: a call with more overflowing pairs
-// fails with NCX_E_CAPACITY), the saved-run slots, and EPA records of nrec pairs (0: none, for
+// fails with NCX_E_CAPACITY), the saved-run slots, and EPA records for nrec pairs (0: none, for
 // distances).
 int contact_tiers_reserve(ContactTiers& t, ncx_ctx* ctx, size_t cap, size_t nrec) {
-  if (nrec > t.nrec) {
-    // one allocation: support points, records, the first tier's saved runs
-    const size_t sup = (size_t)ctx->num_cus * EPA_SUP_FLOATS_PER_CU * 4;
-    const size_t slots = std::min<size_t>(SUS_CAP[0], nrec / 32);
+  nrec = std::min(nrec, REC_MOST);
+  if (nrec > t.nrec && nrec > t.rec_asked) {
+    // one allocation: support points, records, the first tier's saved runs; a quarter more than there
+    // were, so that batches that grow a little from call to call seldom come here
+    const size_t sup = (size_t)ctx->num_cus * EPA_SUP_FLOATS_PER_CU * 4, asked = nrec;
+    nrec = std::min(std::max(nrec, t.nrec + t.nrec / 4), REC_MOST);
     t.epa.release();
-    t.nrec = 0;
-    int rc = t.epa.reserve(sup + nrec * sizeof(EpaRec) + slots * SUS_BYTES[0]);
-    if (rc) return rc;
+    t.nrec = t.rec_asked = 0;
+    for (;;) {
+      const size_t slots = std::min<size_t>(SUS_CAP[0], nrec / 32);
+      const int rc = t.epa.reserve(sup + nrec * sizeof(EpaRec) + slots * SUS_BYTES[0]);
+      if (!rc) {
+        t.sus0_cap = (uint32_t)slots;
+        break;
+      }
+      if (nrec <= REC_LEAST) return rc;
+      nrec = std::max(nrec / 2, REC_LEAST);
+    }
     t.nrec = nrec;
-    t.sus0_cap = (uint32_t)slots;
+    t.rec_asked = asked;
     t.sup = t.epa.as<float>();
     t.rec = (EpaRec*)(t.epa.as<uint8_t>() + sup);
     t.sus0 = (uint8_t*)(t.rec + nrec);
@@ -781,7 +800,7 @@ void contact_tiers_release(ContactTiers& t) {
   t.blist.release();
   t.bkey.release();
   t.epa.release();
-  t.nrec = 0;
+  t.nrec = t.rec_asked = 0;
   t.bcap = 0;
   t.cap = 0;
   t.sus0_cap = 0;
@@ -790,7 +809,12 @@ void contact_tiers_release(ContactTiers& t) {
   t.last = nullptr;
 }
 
-// Re-runs the n records listed at list_src (device) with device-memory arenas 8x larger per round
+__global__ void k_iota_u32(uint32_t* __restrict__ p, uint32_t n) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = i;
+}
+
+// Re-runs the n records listed at list_src (device; null: the first n) with device-memory arenas 8x larger per round
 // (starting from 8 x the last tier's vcap/fcap) until none overflows; host-driven (synchronises
 // the stream).  Chunks keep each round's arenas <= 2 GiB.  The first round continues the runs
 // the last LDS tier saved (sus_src, slot = list position); device-memory rounds do not suspend.
@@ -801,7 +825,12 @@ static int rerun_overflows(ContactTiers& T, ncx_ctx* ctx, KArgs a, uint32_t n, c
   DevBuf lst;
   int rc;
   if ((rc = lst.reserve((size_t)n * 4))) return rc;
-  NCX_HIP_CHECK(hipMemcpyAsync(lst.p, list_src, (size_t)n * 4, hipMemcpyDeviceToDevice, ctx->stream));
+  if (list_src) {
+    NCX_HIP_CHECK(hipMemcpyAsync(lst.p, list_src, (size_t)n * 4, hipMemcpyDeviceToDevice, ctx->stream));
+  } else {
+    hipLaunchKernelGGL(k_iota_u32, dim3(ceil_div(n, 256)), dim3(256), 0, ctx->stream, lst.as<uint32_t>(), n);
+    NCX_HIP_CHECK(hipGetLastError());
+  }
   while (n > 0) {
     vcap *= 8;
     fcap *= 8;
@@ -939,13 +968,16 @@ static KArgs tier_args(ContactTiers& T, const KArgs& a, int t) {
   KArgs b = a;
   b.range_b = nullptr;
   b.range_e = nullptr;
-  b.rec_base = nullptr;
   b.list = lists[t - 1];
   b.n_dev = counts[t - 1];
   b.ovf_count = counts[t];
   b.ovf_list = lists[t];
   b.work = ncx_work_set(ovf, works[t]);
   set_sus(T, b, t);
+  if (t == 3 && T.parts) {  // the next part takes the records: contacts_resolve_overflow makes them again
+    b.ovf_pairs = 1;
+    b.sus_save_cap = 0;
+  }
   return b;
 }
 
@@ -990,6 +1022,19 @@ static int clear_tier_counters(ncx_ctx* ctx, uint32_t* hdr) {
   static_assert(NCX_WORK_TUNE == 0 && NCX_WORK_T2 == 1 && NCX_WORK_T3 == 2 && NCX_WORK_T4 == 3 && NCX_WORK_TUNE_EPA == 4,
                 "work sets");
   return fill_u32(ctx, ncx_work_set(hdr, 0), 5 * NCX_WORK_SET, 0u);
+}
+
+// Between the parts of a launch: the counts and work counters start again; the pairs that outgrew T1
+// are summed, a list that overflowed is noted, and what outgrew T4 stays listed.
+__global__ __launch_bounds__(256) void k_next_part(uint32_t* __restrict__ hdr, uint32_t cap) {
+  for (uint32_t i = threadIdx.x; i < NCX_WORK_SETS; i += 256) hdr[NCX_WORK_BASE + i * NCX_WORK_SET] = 0u;
+  if (threadIdx.x == 0) {
+    const uint32_t t1 = hdr[NCX_OVF_T1_COUNT], t2 = hdr[NCX_OVF_T2_COUNT], t3 = hdr[NCX_OVF_T3_COUNT];
+    hdr[NCX_OVF_EARLIER] += t1;
+    if (t1 > cap || t2 > cap || t3 > cap) hdr[NCX_OVF_FULL] = 1u;
+    hdr[NCX_OVF_T1_COUNT] = hdr[NCX_OVF_T2_COUNT] = hdr[NCX_OVF_T3_COUNT] = 0u;
+    for (int b = 0; b < NCX_NBUCKETS; ++b) hdr[NCX_REC_COUNT + b] = 0u;
+  }
 }
 
 #define TUNE_MIN_PAIRS 4096u
@@ -1115,7 +1160,8 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
   a.vcap = ArenaT4::VC;
   a.fcap = ArenaT4::FC;
   a.rec = T.rec;
-  a.rec_base = nullptr;
+  a.part_lo = 0u;
+  a.part_hi = 0xFFFFFFFFu;
   a.sup = T.sup;
   a.ovf_count = ovf + NCX_OVF_T1_COUNT;
   a.ovf_list = T.t1_list();
@@ -1131,6 +1177,7 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
   // Partition (sort by key) unless the batch is small: below 16,384 pairs the three partition
   // kernels and the launches per bucket cost more (about 60 us) than the order saves.
   const bool partition = tune_now || npairs >= NCX_PARTITION_MIN_PAIRS;
+  T.parts = false;
   if (partition) {
     if ((rc = partition_launch(S, T, ctx, a.poses, a.ia, a.ib, npairs, n_dev))) return rc;
     KArgs t = a;
@@ -1139,6 +1186,7 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
     t.npairs = npairs;
     if (tune_now && (rc = autotune(S, T, ctx, t, mode))) return rc;
   }
+  NCX_REQUIRE(mode == 1 || T.nrec >= (partition ? 1 : npairs), "contact launch: EPA records not allocated");
   if (!partition) {
     // one launch over all pairs, in their own order
     const int big = 31 - __builtin_clz(S->buckets | 1u);  // the variant of the set's largest hulls
@@ -1154,28 +1202,40 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
     if (rc) return rc;
   } else {
     // distance: one launch per run of consecutive buckets sharing a variant, over the partitioned
-    // list; contact: one GJK and one EPA launch per bucket, its records from its own range on
-    for (int b0 = 0; b0 < NCX_NBUCKETS;) {
-      if (mode == 0 && !(S->buckets >> b0 & 1u)) {  // no shape of the set makes such a pair
-        ++b0;
-        continue;
+    // list; contact: one GJK and one EPA launch per bucket, its records from its own range on, for
+    // each part of the list that the records suffice for
+    const size_t part = mode == 0 ? T.nrec : npairs;
+    T.parts = npairs > part;
+    for (size_t lo = 0; lo < npairs; lo += part) {
+      if (lo) {
+        // the part before
+        if ((rc = launch_upper_tiers(ctx, T, a, std::min(likely, part)))) return rc;
+        hipLaunchKernelGGL(k_next_part, dim3(1), dim3(256), 0, ctx->stream, ovf, T.cap);
+        NCX_HIP_CHECK(hipGetLastError());
       }
-      const int v = S->tune[mode][b0] >= 0 ? S->tune[mode][b0] : 1;
-      int b1 = b0;
-      while (mode == 1 && b1 + 1 < NCX_NBUCKETS && (S->tune[mode][b1 + 1] >= 0 ? S->tune[mode][b1 + 1] : 1) == v) ++b1;
-      KArgs ab = a;
-      ab.list = T.blist.as<uint32_t>();
-      ab.n_dev = nullptr;
-      ab.npairs = npairs;
-      ab.range_b = ovf + NCX_BKT_RANGE + 2 * b0;
-      ab.range_e = ovf + NCX_BKT_RANGE + 2 * b1 + 1;
-      ab.work = ncx_work_set(ovf, NCX_WORK_BKT + b0);
-      ab.rec_base = ab.range_b;
-      ab.rec_count = ovf + NCX_REC_COUNT + b0;
-      if (mode == 1) rc = launch_distance(v, ctx, ab, npairs);
-      else rc = launch_contact_t1(v, GJK_BUCKET_G[b0], ctx, ab, likely, ab.work, ncx_work_set(ovf, NCX_WORK_EPA + b0));
-      if (rc) return rc;
-      b0 = b1 + 1;
+      a.part_lo = (uint32_t)lo;
+      a.part_hi = (uint32_t)std::min(npairs, lo + part);
+      for (int b0 = 0; b0 < NCX_NBUCKETS;) {
+        if (mode == 0 && !(S->buckets >> b0 & 1u)) {  // no shape of the set makes such a pair
+          ++b0;
+          continue;
+        }
+        const int v = S->tune[mode][b0] >= 0 ? S->tune[mode][b0] : 1;
+        int b1 = b0;
+        while (mode == 1 && b1 + 1 < NCX_NBUCKETS && (S->tune[mode][b1 + 1] >= 0 ? S->tune[mode][b1 + 1] : 1) == v) ++b1;
+        KArgs ab = a;
+        ab.list = T.blist.as<uint32_t>();
+        ab.n_dev = nullptr;
+        ab.npairs = npairs;
+        ab.range_b = ovf + NCX_BKT_RANGE + 2 * b0;
+        ab.range_e = ovf + NCX_BKT_RANGE + 2 * b1 + 1;
+        ab.work = ncx_work_set(ovf, NCX_WORK_BKT + b0);
+        ab.rec_count = ovf + NCX_REC_COUNT + b0;
+        if (mode == 1) rc = launch_distance(v, ctx, ab, npairs);
+        else rc = launch_contact_t1(v, GJK_BUCKET_G[b0], ctx, ab, likely, ab.work, ncx_work_set(ovf, NCX_WORK_EPA + b0));
+        if (rc) return rc;
+        b0 = b1 + 1;
+      }
     }
   }
   if (mode == 0 && (rc = launch_upper_tiers(ctx, T, a, likely))) return rc;
@@ -1207,6 +1267,31 @@ int contacts_launch_device_count(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, c
   return launch_tiers(S, T, ctx, a, cap, n_dev, may_tune);
 }
 
+// After a launch in parts, whose records are gone: GJK again for the n pairs listed past T4, then their
+// EPA from the start on device-memory arenas.
+static int rerun_pairs(ContactTiers& T, ncx_ctx* ctx, uint32_t n) {
+  uint32_t* hdr = T.ovf.as<uint32_t>();
+  for (uint32_t o = 0; o < n; o += (uint32_t)T.nrec) {
+    KArgs g = *T.last;
+    g.list = T.t4_list() + o;
+    g.npairs = std::min<size_t>(n - o, T.nrec);
+    g.n_dev = nullptr;
+    g.ovf_pairs = 0;
+    g.rec_count = hdr + NCX_REC_COUNT;
+    g.work = ncx_work_set(hdr, NCX_WORK_BKT);
+    int rc;
+    if ((rc = fill_u32(ctx, g.rec_count, 1, 0u)) || (rc = fill_u32(ctx, g.work, 1, 0u))) return rc;
+    hipLaunchKernelGGL(k_contact_gjk<GJK_SMALL_G>, dim3(capped_blocks(ctx, GJK_BLOCKS_PER_CU, g.npairs, GJK_BS / GJK_SMALL_G)),
+                       dim3(GJK_BS), 0, ctx->stream, g);
+    NCX_HIP_CHECK(hipGetLastError());
+    uint32_t recs = 0;
+    NCX_HIP_CHECK(hipMemcpyAsync(&recs, g.rec_count, 4, hipMemcpyDeviceToHost, ctx->stream));
+    NCX_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+    if ((rc = rerun_overflows(T, ctx, g, recs, nullptr, ArenaT4::VC, ArenaT4::FC, nullptr, 0))) return rc;
+  }
+  return NCX_OK;
+}
+
 // After the last launch_tiers on T has completed on ctx's stream: fails on a bad pair index or on
 // more overflows than the lists hold, re-runs what T4 could not hold with device-memory arenas,
 // and reports how many pairs needed more than the T1 arena.
@@ -1216,12 +1301,13 @@ int contacts_resolve_overflow(ContactTiers& T, ncx_ctx* ctx, size_t* n_large) {
   NCX_HIP_CHECK(hipMemcpyAsync(hdr, T.ovf.p, sizeof(hdr), hipMemcpyDeviceToHost, ctx->stream));
   NCX_HIP_CHECK(hipStreamSynchronize(ctx->stream));
   NCX_REQUIRE(hdr[NCX_OVF_BAD] == 0, "contact batch: a pair index is not a shape of the set");
-  if (hdr[NCX_OVF_T1_COUNT] > T.cap || hdr[NCX_OVF_T2_COUNT] > T.cap || hdr[NCX_OVF_T3_COUNT] > T.cap ||
-      hdr[NCX_OVF_T4_COUNT] > T.cap) {
+  if (hdr[NCX_OVF_FULL] || hdr[NCX_OVF_T1_COUNT] > T.cap || hdr[NCX_OVF_T2_COUNT] > T.cap ||
+      hdr[NCX_OVF_T3_COUNT] > T.cap || hdr[NCX_OVF_T4_COUNT] > T.cap) {
     ncx_set_error("contact batch: more EPA arena overflows in one call than the overflow list holds");
     return NCX_E_CAPACITY;
   }
-  if (n_large) *n_large = hdr[NCX_OVF_T1_COUNT];
+  if (n_large) *n_large = hdr[NCX_OVF_EARLIER] + hdr[NCX_OVF_T1_COUNT];
+  if (T.parts) return rerun_pairs(T, ctx, hdr[NCX_OVF_T4_COUNT]);
   return rerun_overflows(T, ctx, *T.last, hdr[NCX_OVF_T4_COUNT], T.t4_list(), ArenaT4::VC, ArenaT4::FC, T.sus[3].as<uint8_t>(),
                          SUS_BYTES[3]);
 }

@@ -390,7 +390,8 @@ template <bool DIL> static void launch_toi(ncx_ctx* ctx, int G, const TOIArgs& a
 // Lanes per pair, for sets with hulls of up to 96 vertices and larger ones.
 #define TOI_G 2
 #define TOI_LARGE_G 4
-static const size_t CAST_CHUNK = (size_t)1 << 30;
+// Queries of one launch: bounds the scratch memory (8 bytes a pair, 4 a ray).
+static const size_t CAST_CHUNK = (size_t)1 << 26;
 
 extern "C" int ncx_time_of_impact_batch(ncx_shapes* s, const ncx_pose* poses_dev, const float* vel_dev,
                                         const uint32_t* ia_dev, const uint32_t* ib_dev, size_t npairs, float max_toi,
@@ -412,7 +413,8 @@ extern "C" int ncx_time_of_impact_batch(ncx_shapes* s, const ncx_pose* poses_dev
         return rc;
     return NCX_OK;
   }
-  const bool partition = npairs >= NCX_PARTITION_MIN_PAIRS;
+  // the order is worth its memory, but not a refusal
+  const bool partition = npairs >= NCX_PARTITION_MIN_PAIRS && contact_tiers_reserve_list(s->tiers, npairs) == NCX_OK;
   if (partition) rc = pairs_partition(s, s->tiers, ctx, poses_dev, ia_dev, ib_dev, npairs, nullptr);
   else rc = fill_u32(ctx, s->tiers.ovf.as<uint32_t>(), NCX_OVF_HEADER, 0u);
   if (rc) return rc;
@@ -456,19 +458,24 @@ extern "C" int ncx_shapes_cast_rays(ncx_shapes* s, const ncx_pose* poses_dev, co
   if (n == 0) return NCX_OK;
   ncx_ctx* ctx = s->ctx;
   int rc;
-  if (n > CAST_CHUNK) {  // the lists and counters are 32-bit
-    for (size_t o = 0; o < n; o += CAST_CHUNK) {
+  // an error flag, the two lists' lengths and work counters on lines of their own, the lists; fewer
+  // rays at a time where there is no memory for all
+  size_t chunk = std::min(n, CAST_CHUNK);
+  while ((rc = s->qerr.reserve(4 * (5 * SR_STRIDE + chunk)))) {
+    if (chunk <= 4096) return rc;
+    chunk = std::max<size_t>(chunk / 2, 4096);
+  }
+  if (n > chunk) {
+    for (size_t o = 0; o < n; o += chunk) {
       const float* soa[6];
       for (int d = 0; d < 6; ++d) soa[d] = ray_soa_dev[d] + o;
-      if ((rc = ncx_shapes_cast_rays(s, poses_dev, shape_dev + o, soa, std::min(CAST_CHUNK, n - o), max_toi, solid,
+      if ((rc = ncx_shapes_cast_rays(s, poses_dev, shape_dev + o, soa, std::min(chunk, n - o), max_toi, solid,
                                      toi_dev + o, normal_dev + 3 * o, feature_dev + o)))
         return rc;
     }
     return NCX_OK;
   }
-  // an error flag, the two lists' lengths and work counters on lines of their own, the lists
-  if ((rc = s->qerr.reserve(4 * (5 * SR_STRIDE + n))) || (rc = fill_u32(ctx, s->qerr.as<uint32_t>(), 5 * SR_STRIDE, 0u)))
-    return rc;
+  if ((rc = fill_u32(ctx, s->qerr.as<uint32_t>(), 5 * SR_STRIDE, 0u))) return rc;
   SRArgs a;
   a.shapes = s->shapes.as<ncx_shape>();
   a.P = Pool{s->hx.as<float>(), s->hy.as<float>(), s->hz.as<float>()};

@@ -25,6 +25,8 @@ int hipFree(void* p) { free(p); return 0; }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void* stream) { memmove(d, s, n); return 0; }
 int hipStreamSynchronize(void* s) { return 0; }
 int hipGetLastError(void) { int e = last_error; last_error = 0; return e; }
+int hipEventCreate(void** e) { *e = NULL; return 0; }
+int hipEventDestroy(void* e) { return 0; }
 const char* hipGetErrorString(int e) { return e == 2 ? "out of memory" : "error"; }
 int __hipPushCallConfiguration(dim3_ g, dim3_ b, size_t sh, void* s) { cfg_grid = g; cfg_block = b; return 0; }
 int __hipPopCallConfiguration(dim3_* g, dim3_* b, size_t* sh, void** s) {

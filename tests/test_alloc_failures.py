@@ -51,6 +51,14 @@ def impact(n):
                                         *[out.ctypes.data] * 7)
 
 
+def rays(n):
+    ix = np.zeros(n, np.uint32)
+    col = np.zeros(n, np.float32).ctypes.data
+    out = np.zeros(12 * n, np.uint8)
+    return lib.ncx_shapes_cast_rays(shapes, p, ix.ctypes.data, (C.c_void_p * 6)(*[col] * 6), n, 1.0, 1,
+                                    *[out.ctypes.data] * 3)
+
+
 """
 
 
@@ -78,3 +86,18 @@ print(json.dumps([refused, message, rc, count("stub_null_fills"), count("stub_la
     refused, message, rc, null_fills, launches = out
     assert refused != 0 and "hipMalloc" in message
     assert (rc, null_fills) == (0, 0) and launches > 0
+
+
+@pytest.mark.parametrize("call,least,little", [("contact", 20, 27), ("rays", 12, 20), ("impact", 0, 20)])
+def test_batches_of_little_memory(tmp_path, call, least, little):
+    """Contacts take their pairs in parts, and rays theirs in chunks, where there is no memory for all of
+    them at once; times of impact do without their order.  With none at all the first two are refused."""
+    body = f"""
+limit.value = 1 << {{}}
+a = count("stub_launches")
+print(json.dumps([{call}(1 << 20), count("stub_launches") - a]))
+"""
+    none, few, all_ = (run(tmp_path, body.format(k)) for k in (least, little, 62))
+    assert (none[0] == 0) == (call == "impact")
+    assert few[0] == all_[0] == 0
+    assert few[1] < all_[1] if call == "impact" else few[1] > all_[1]
