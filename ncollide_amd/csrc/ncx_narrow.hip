@@ -435,7 +435,8 @@ __global__ __launch_bounds__(BS, 3) void k_distance(KArgs a) {
 // time from one hull.  262,144 hull pairs of up to 256 vertices, whole batch: 2.37 ms in groups,
 // 1.76 ms so (groups of 4 and 16: 2.1 and 1.78 ms; a wavefront's lanes that wait for new pairs at 4
 // or 16 idle ones, the same).  It needs 64 pairs a wavefront to pay, so the autotuner chooses it or a
-// group's kernel for each vertex-count bucket by timing both on a sample.
+// group's kernel for each vertex-count bucket by timing both on a sample, for batches that fill the
+// chip (bucket_variant).
 #define DW_G 8
 #define DW_REFILL 16  // idle lanes before the wavefront takes more pairs
 template <int BS>
@@ -899,6 +900,24 @@ extern "C" int ncx_shapes_set_tuning(ncx_shapes* s, int query, const int32_t* ch
   return NCX_OK;
 }
 
+// The variant of a batch's pairs of one bucket.  The tuner's samples are large; one pair a lane needs
+// enough pairs to fill the chip (distances, 8 lanes a pair or the best other variant against one
+// pair a lane: 300 pairs of 256-vertex hulls 65 and 186 us, 16,384 185 and 287; 16,384 of 64-vertex
+// hulls 110 and 148, of mixed shapes 129 and 154; 32,768 of mixed shapes 167 and 174, 65,536 204 and
+// 184 us), so that smaller batches take the fastest of the others on the samples, and those too
+// small to partition 8 lanes a pair.
+#define DW_VARIANT 4
+#define DW_MIN_PAIRS 32768u
+static int bucket_variant(const ncx_shapes* S, int mode, int b, size_t npairs) {
+  const int v = S->tune[mode][b] >= 0 ? S->tune[mode][b] : 1;
+  if (mode == 0 || v != DW_VARIANT || npairs >= DW_MIN_PAIRS) return v;
+  int best = 0;
+  if (npairs >= NCX_PARTITION_MIN_PAIRS)
+    for (int u = 1; u < DW_VARIANT; ++u)
+      if (S->tune_ms[mode][b][u] > 0.f && S->tune_ms[mode][b][u] < S->tune_ms[mode][b][best]) best = u;
+  return best;
+}
+
 static unsigned capped_blocks(ncx_ctx* ctx, unsigned per_cu, size_t n, size_t per_block) {
   return (unsigned)std::max<size_t>(1, std::min<size_t>((size_t)ctx->num_cus * per_cu, (n + per_block - 1) / per_block));
 }
@@ -1190,7 +1209,7 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
   if (!partition) {
     // one launch over all pairs, in their own order
     const int big = 31 - __builtin_clz(S->buckets | 1u);  // the variant of the set's largest hulls
-    const int v = S->tune[mode][big] >= 0 ? S->tune[mode][big] : 1;
+    const int v = bucket_variant(S, mode, big, npairs);
     KArgs ab = a;
     ab.list = nullptr;
     ab.n_dev = n_dev;
@@ -1220,9 +1239,9 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
           ++b0;
           continue;
         }
-        const int v = S->tune[mode][b0] >= 0 ? S->tune[mode][b0] : 1;
+        const int v = bucket_variant(S, mode, b0, npairs);
         int b1 = b0;
-        while (mode == 1 && b1 + 1 < NCX_NBUCKETS && (S->tune[mode][b1 + 1] >= 0 ? S->tune[mode][b1 + 1] : 1) == v) ++b1;
+        while (mode == 1 && b1 + 1 < NCX_NBUCKETS && bucket_variant(S, mode, b1 + 1, npairs) == v) ++b1;
         KArgs ab = a;
         ab.list = T.blist.as<uint32_t>();
         ab.n_dev = nullptr;

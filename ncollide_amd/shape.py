@@ -109,7 +109,7 @@ class ShapeSet:
     def types(self):
         return self.records["type"]
 
-    # first-tier variants: (lanes per pair, EPA arena vertices)
+    # first-tier variants: (lanes per EPA run, EPA arena vertices)
     VARIANTS = ((8, 44), (16, 44), (32, 44), (8, 24), (16, 24))
     # distance queries have no EPA arena: lanes per pair of each variant
     DISTANCE_VARIANTS = ((8, 0), (16, 0), (32, 0), (4, 0), (1, 0))
