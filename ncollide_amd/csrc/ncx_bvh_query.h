@@ -127,7 +127,7 @@ __global__ __launch_bounds__(BQ_BLOCK) void k_bq_collect(BQArgs a) {
     const float* b = a.leaf_soa;
     float c;
     if (bq_test<K>(qv, a.max_toi, b[0], b[1], b[2], b[3], b[4], b[5], c)) emit(0);
-  } else {
+  } else if (a.nleaves > 1) {
     uint32_t stk[BQ_STACK];
     int sp = 0;
     uint32_t node = 0;
@@ -252,7 +252,7 @@ static __global__ __launch_bounds__(BQ_BLOCK, 3) void k_bq_first_ray(BQArgs a) {
           sp = nk = 0;
           node = 0;
           walk = a.nleaves > 1;
-          if (!walk) {
+          if (a.nleaves == 1) {
             const float* b = a.leaf_soa;
             float c;
             if (bq_ray_box(o, dir, a.max_toi, b[0], b[1], b[2], b[3], b[4], b[5], c)) leaf(0, c);

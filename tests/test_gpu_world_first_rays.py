@@ -93,3 +93,16 @@ def test_hits_before_their_boxes(ctx, orc, size, away, early_hits):
     early = np.zeros(nrays, bool)
     early[ray[toi < entry]] = True
     assert np.array_equal(bh[~early], rh[~early]) and np.array_equal(bt[~early], rt[~early])
+
+
+def test_world_without_shapes(ctx):
+    ss = ncx.ShapeSet(records=np.zeros(0, ncx.shape.SHAPE_DTYPE), pool=np.zeros((0, 3), np.float32), ctx=ctx)
+    world = World(ss, margin=0.0, prediction=0.0, max_pairs=1024)
+    poses = torch.zeros((1, 8), device=ctx.device)
+    world.step(poses)
+    assert world.sync()[0] == 0
+    o, d = np.zeros((70, 3), np.float32), np.ones((70, 3), np.float32)
+    h, t, n = world.first_interference_with_rays(poses, o, d, 10.0)
+    assert (h.cpu().numpy().view(np.uint32) == 0xFFFFFFFF).all() and (t == -1).all() and (n == 0).all()
+    assert world.interferences_with_rays(poses, o, d, 10.0)[1].numel() == 0
+    assert world.interferences_with_aabbs(np.array([[-9, -9, -9, 9, 9, 9]], np.float32))[1].numel() == 0
