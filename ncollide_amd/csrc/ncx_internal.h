@@ -123,7 +123,7 @@ struct ContactTiers {
   size_t nrec = 0;
   size_t rec_asked = 0;     // the most records asked for
   bool parts = false;       // the last launch took its pairs in more than one part
-  DevBuf sus[4];     // saved EPA runs handed on: (unused), T2 -> T3, T3 -> T4, T4 -> device-memory tier
+  DevBuf sus[3];     // saved EPA runs handed on: T2 -> T3, T3 -> T4, T4 -> device-memory tier
   uint32_t* t1_list() const { return ovf.as<uint32_t>() + NCX_OVF_HEADER; }
   uint32_t* t2_list() const { return ovf.as<uint32_t>() + NCX_OVF_HEADER + cap; }
   uint32_t* t3_list() const { return ovf.as<uint32_t>() + NCX_OVF_HEADER + 2 * (size_t)cap; }

@@ -778,9 +778,9 @@ int contact_tiers_reserve(ContactTiers& t, ncx_ctx* ctx, size_t cap, size_t nrec
     t.rec = (EpaRec*)(t.epa.as<uint8_t>() + sup);
     t.sus0 = (uint8_t*)(t.rec + nrec);
   }
-  for (int i = 1; i < 4; ++i) {
+  for (int i = 0; i < 3; ++i) {
     if (t.sus[i].p) continue;
-    int rc = t.sus[i].reserve((size_t)SUS_CAP[i] * SUS_BYTES[i]);
+    int rc = t.sus[i].reserve((size_t)SUS_CAP[i + 1] * SUS_BYTES[i + 1]);
     if (rc) return rc;
   }
   cap = std::min<size_t>(std::max<size_t>(cap, 4096), (size_t)1 << 24);
@@ -805,7 +805,7 @@ void contact_tiers_release(ContactTiers& t) {
   t.bcap = 0;
   t.cap = 0;
   t.sus0_cap = 0;
-  for (int i = 0; i < 4; ++i) t.sus[i].release();
+  for (int i = 0; i < 3; ++i) t.sus[i].release();
   delete t.last;
   t.last = nullptr;
 }
@@ -946,8 +946,7 @@ static int launch_contact_t1(int variant, int G, ncx_ctx* ctx, const KArgs& a, s
   switch (G) {
     case 1: hipLaunchKernelGGL(k_contact_gjk<1>, dim3(gb), dim3(GJK_BS), 0, ctx->stream, g); break;
     case 4: hipLaunchKernelGGL(k_contact_gjk<4>, dim3(gb), dim3(GJK_BS), 0, ctx->stream, g); break;
-    case 8: hipLaunchKernelGGL(k_contact_gjk<8>, dim3(gb), dim3(GJK_BS), 0, ctx->stream, g); break;
-    default: hipLaunchKernelGGL(k_contact_gjk<16>, dim3(gb), dim3(GJK_BS), 0, ctx->stream, g); break;
+    default: hipLaunchKernelGGL(k_contact_gjk<8>, dim3(gb), dim3(GJK_BS), 0, ctx->stream, g); break;
   }
   NCX_HIP_CHECK(hipGetLastError());
   KArgs e = a;
@@ -967,7 +966,7 @@ static int launch_contact_t1(int variant, int G, ncx_ctx* ctx, const KArgs& a, s
 
 // Saved-run buffers of LDS tier `tier` (0 = T1): it continues the runs T(tier) saved and saves
 // its own suspended runs for the next tier.
-static uint8_t* sus_slots(const ContactTiers& T, int tier) { return tier == 0 ? T.sus0 : T.sus[tier].as<uint8_t>(); }
+static uint8_t* sus_slots(const ContactTiers& T, int tier) { return tier == 0 ? T.sus0 : T.sus[tier - 1].as<uint8_t>(); }
 
 static void set_sus(ContactTiers& T, KArgs& b, int tier) {
   b.sus_load = tier > 0 ? sus_slots(T, tier - 1) : nullptr;
@@ -1327,7 +1326,7 @@ int contacts_resolve_overflow(ContactTiers& T, ncx_ctx* ctx, size_t* n_large) {
   }
   if (n_large) *n_large = hdr[NCX_OVF_EARLIER] + hdr[NCX_OVF_T1_COUNT];
   if (T.parts) return rerun_pairs(T, ctx, hdr[NCX_OVF_T4_COUNT]);
-  return rerun_overflows(T, ctx, *T.last, hdr[NCX_OVF_T4_COUNT], T.t4_list(), ArenaT4::VC, ArenaT4::FC, T.sus[3].as<uint8_t>(),
+  return rerun_overflows(T, ctx, *T.last, hdr[NCX_OVF_T4_COUNT], T.t4_list(), ArenaT4::VC, ArenaT4::FC, sus_slots(T, 3),
                          SUS_BYTES[3]);
 }
 

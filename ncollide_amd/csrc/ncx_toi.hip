@@ -382,8 +382,7 @@ template <bool DIL> static void launch_toi(ncx_ctx* ctx, int G, const TOIArgs& a
   switch (G) {
     case 1: hipLaunchKernelGGL((k_toi<1, DIL>), nb, bs, 0, ctx->stream, a); break;
     case 2: hipLaunchKernelGGL((k_toi<2, DIL>), nb, bs, 0, ctx->stream, a); break;
-    case 4: hipLaunchKernelGGL((k_toi<4, DIL>), nb, bs, 0, ctx->stream, a); break;
-    default: hipLaunchKernelGGL((k_toi<8, DIL>), nb, bs, 0, ctx->stream, a); break;
+    default: hipLaunchKernelGGL((k_toi<4, DIL>), nb, bs, 0, ctx->stream, a); break;
   }
 }
 
