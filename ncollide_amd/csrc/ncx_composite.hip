@@ -197,11 +197,11 @@ struct MDArgs {
   uint32_t* work;  // query counter (zero at launch)
 };
 
-#define MD_G 16
+#define MD_G 32
 #define MD_BLOCK 128
 #define MD_STACK 400
-#define MD_RAW 64
-#define MD_KEEP 32
+#define MD_RAW 128
+#define MD_KEEP 64
 #define MD_BLOCKS_PER_CU 4u  // resident: two wavefronts per SIMD
 
 template <int G> __device__ __forceinline__ float group_min(float v) {
@@ -209,6 +209,7 @@ template <int G> __device__ __forceinline__ float group_min(float v) {
   v = fminf(v, __uint_as_float(lane_across<2>(__float_as_uint(v))));
   if constexpr (G >= 8) v = fminf(v, __uint_as_float(lane_across<4>(__float_as_uint(v))));
   if constexpr (G >= 16) v = fminf(v, __uint_as_float(lane_across<8>(__float_as_uint(v))));
+  if constexpr (G >= 32) v = fminf(v, __uint_as_float(lane_across<16>(__float_as_uint(v))));
   return v;
 }
 template <int G> __device__ __forceinline__ uint32_t group_min(uint32_t v) {
@@ -216,6 +217,7 @@ template <int G> __device__ __forceinline__ uint32_t group_min(uint32_t v) {
   v = min(v, lane_across<2>(v));
   if constexpr (G >= 8) v = min(v, lane_across<4>(v));
   if constexpr (G >= 16) v = min(v, lane_across<8>(v));
+  if constexpr (G >= 32) v = min(v, lane_across<16>(v));
   return v;
 }
 
@@ -253,16 +255,17 @@ struct MDBest {
 // triangle to run GJK on by itself.  The three kinds of step are kept apart, in lists of LDS, and
 // run when most groups of the wavefront have enough of them, because a step that one lane takes
 // costs the wavefront as much as one that all do.
-// The shapes over a terrain above: 50 ms with one search per 2 lanes, 8.1 ms so.
+// The shapes over a terrain above: 50 ms with one search per 2 lanes, 7.1 ms so (8 and 16 lanes a
+// query 17 and 8.2 ms; lists twice as long 7.7 ms, three wavefronts on a SIMD 9.4 with 16 lanes).
 template <int G>
 __global__ __launch_bounds__(MD_BLOCK) void k_md(MDArgs a) {
-  constexpr int GROUPS = 64 / G, REFILL = GROUPS / 4;
-  static_assert(MD_RAW >= 4 * G && MD_KEEP >= 2 * G && MD_STACK >= LBVH_MAX_DEPTH + 2 * G, "list sizes");
+  constexpr int GROUPS = 64 / G, REFILL = std::max(1, GROUPS / 4);
+  static_assert(G >= 4 && G <= 32 && MD_RAW >= 4 * G && MD_KEEP >= 2 * G && MD_STACK >= LBVH_MAX_DEPTH + 2 * G, "list sizes");
   __shared__ uint2 stacks[MD_BLOCK / G][MD_STACK];
   __shared__ uint32_t raws[MD_BLOCK / G][MD_RAW];
   __shared__ uint2 keeps[MD_BLOCK / G][MD_KEEP];
   const int lane = threadIdx.x & 63, gl = lane & (G - 1), gbase = lane & ~(G - 1);
-  const uint32_t gmask = (1u << G) - 1u, below = (1u << gl) - 1u;
+  const uint32_t gmask = ~0u >> (32 - G), below = (1u << gl) - 1u;
   uint2* const stk = stacks[threadIdx.x / G];
   uint32_t* const raw = raws[threadIdx.x / G];
   uint2* const keep = keeps[threadIdx.x / G];
