@@ -139,7 +139,7 @@ struct ncx_shapes {
   DevBuf shapes;      // ncx_shape[n]
   DevBuf hx, hy, hz;  // hull pool
   ContactTiers tiers; // for ncx_contact_batch / ncx_distance_batch
-  DevBuf qerr;        // error flag of the time-of-impact, ray-cast and composite queries
+  DevBuf qerr;        // ray casts: error flag, the lists of rays by shape kind and their counters
   const float4* tri = nullptr;  // triangles of the Triangle parts (a mesh's combined set only)
   // polygonal faces, edges and adjacency of the hulls (ConvexHull::try_new), built on the first
   // contact-manifold call: per shape (face base, face count, edge base, 0); per face normal and

@@ -577,7 +577,7 @@ extern "C" int ncx_shapes_destroy(ncx_shapes* s) {
 }
 
 // The autotuner's state for one query (0 contact, 1 distance): per vertex-count bucket the
-// chosen variant (0, 1, 2 = 8, 16, 32 lanes per pair; -1 untuned) and each variant's sample time.
+// chosen variant (T1_VARIANT_G; -1 untuned) and each variant's sample time.
 extern "C" int ncx_shapes_tuning(ncx_shapes* s, int query, int32_t* choice, float* sample_ms) {
   NCX_REQUIRE(s && choice && (query == 0 || query == 1), "ncx_shapes_tuning: bad argument");
   for (int b = 0; b < NCX_NBUCKETS; ++b) {
@@ -1103,7 +1103,7 @@ static int autotune(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, const KArgs& b
         if (mode == 1) rc = launch_distance(v, ctx, a, ns);
         else rc = launch_contact_t1(v, GJK_BUCKET_G[b], ctx, a, ns, a.work, ncx_work_set(hdr, NCX_WORK_TUNE_EPA));
         if (rc) break;
-        // the variant's first-tier overflows cost a second-tier run: time it too
+        // the variant's first-tier overflows cost runs in the later tiers: time them too
         if (mode == 0 && (rc = launch_upper_tiers(ctx, T, a, ns))) break;
         NCX_HIP_CHECK(hipEventRecord(e1, ctx->stream));
         NCX_HIP_CHECK(hipEventSynchronize(e1));

@@ -116,8 +116,8 @@ class ShapeSet:
 
     def tuning(self, query="contact"):
         """The autotuner's choice per vertex-count bucket (no hull, <= 32, <= 96, more vertices):
-        the variant (lanes per pair, first-tier EPA arena vertices, 0 for distance) or None before
-        tuning, and each variant's sample time (ms; 0 for variants not tried)."""
+        the variant (lanes per EPA run and its first-tier arena's vertices, or lanes per distance pair
+        and 0) or None before tuning, and each variant's sample time (ms; 0 for variants not tried)."""
         table = self.VARIANTS if query == "contact" else self.DISTANCE_VARIANTS
         nv = len(table)
         choice = (C.c_int32 * 4)()
@@ -127,7 +127,8 @@ class ShapeSet:
 
     def set_tuning(self, variants, query="contact"):
         """Pins the first-tier variant of each bucket: a list of 4 indices into VARIANTS (None =
-        tune on the next large batch).  Results do not depend on the variant."""
+        tune on the next large batch).  Results do not depend on the variant.  Distance batches of
+        fewer than 32,768 pairs take another variant in the place of one lane a pair."""
         choice = (C.c_int32 * 4)(*[-1 if v is None else int(v) for v in variants])
         _lib.check(self.ctx.lib.ncx_shapes_set_tuning(self.h, 0 if query == "contact" else 1, choice))
 

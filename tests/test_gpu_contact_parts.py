@@ -53,7 +53,7 @@ def test_scene_of_two_parts(ctx):
     poses = torch.as_tensor(workloads.poses8(t, workloads.uniform_quats(rng, n)).astype(np.float32), device=ctx.device)
     ss = ncx.ShapeSet(records=rec, pool=w["pool"], ctx=ctx)
     world = World(ss, margin=0.01, prediction=0.0, max_pairs=2 * PART)
-    for step in range(2):  # the first step is not captured
+    for step in range(4):  # the first step is not captured
         world.step(poses)
         r = world.results()
         assert PART < r["ia"].numel() < 2 * PART
