@@ -563,6 +563,14 @@ extern "C" int ncx_mesh_distance_batch(ncx_mesh* m, const ncx_pose* mesh_pose, n
   NCX_REQUIRE(mesh_pose && poses_dev && shape_dev && dist_dev, "ncx_mesh_distance_batch: null argument");
   NCX_REQUIRE(n < 0xFFFFFFFFull, "ncx_mesh_distance_batch: too many queries");
   if (n == 0) return NCX_OK;
+  // the query counter counts past n by what the waiting wavefronts ask for, in 32 bits
+  const size_t chunk = (size_t)1 << 30;
+  if (n > chunk) {
+    for (size_t o = 0; o < n; o += chunk)
+      if ((rc = ncx_mesh_distance_batch(m, mesh_pose, s, poses_dev, shape_dev + o, std::min(chunk, n - o), dist_dev + o)))
+        return rc;
+    return NCX_OK;
+  }
   ncx_ctx* ctx = m->ctx;
   if ((rc = m->ctot.reserve(16)) || (rc = fill_u32(ctx, m->ctot.as<uint32_t>(), 3, 0u))) return rc;
   MDArgs a = {};

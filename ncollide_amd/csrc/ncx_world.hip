@@ -960,6 +960,19 @@ extern "C" int ncx_world_first_interference_with_rays(ncx_world* w, const ncx_po
   NCX_REQUIRE(n < 0xFFFFFFFFull, "ncx_world_first_interference_with_rays: too many rays");
   for (int d = 0; d < 6; ++d) NCX_REQUIRE(ray_soa_dev[d], "ncx_world_first_interference_with_rays: null ray array");
   if (n == 0) return NCX_OK;
+  int rc;
+  // the ray counter counts past n by what the waiting wavefronts ask for, in 32 bits
+  const size_t chunk = (size_t)1 << 30;
+  if (n > chunk) {
+    for (size_t o = 0; o < n; o += chunk) {
+      const float* soa[6];
+      for (int d = 0; d < 6; ++d) soa[d] = ray_soa_dev[d] + o;
+      if ((rc = ncx_world_first_interference_with_rays(w, poses_dev, soa, std::min(chunk, n - o), max_toi, handle_dev + o,
+                                                       toi_dev + o, normal_dev + 3 * o)))
+        return rc;
+    }
+    return NCX_OK;
+  }
   BQArgs a = world_bq_args(w, poses_dev);
   for (int d = 0; d < 6; ++d) a.q[d] = ray_soa_dev[d];
   a.nq = (uint32_t)n;
@@ -967,7 +980,6 @@ extern "C" int ncx_world_first_interference_with_rays(ncx_world* w, const ncx_po
   a.handles = handle_dev;
   a.toi = toi_dev;
   a.nrm = normal_dev;
-  int rc;
   if ((rc = w->qtot.reserve(16)) || (rc = fill_u32(w->ctx, w->qtot.as<uint32_t>() + 1, 2, 0u))) return rc;
   a.err = w->qtot.as<uint32_t>() + 1;
   a.work = w->qtot.as<uint32_t>() + 2;

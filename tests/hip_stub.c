@@ -23,6 +23,7 @@ int hipMalloc(void** p, size_t n) {
 }
 int hipFree(void* p) { free(p); return 0; }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void* stream) { memmove(d, s, n); return 0; }
+int hipMemcpy(void* d, const void* s, size_t n, int kind) { memmove(d, s, n); return 0; }
 int hipStreamSynchronize(void* s) { return 0; }
 int hipGetLastError(void) { int e = last_error; last_error = 0; return e; }
 int hipEventCreate(void** e) { *e = NULL; return 0; }

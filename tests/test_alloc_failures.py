@@ -101,3 +101,18 @@ print(json.dumps([{call}(1 << 20), count("stub_launches") - a]))
     assert (none[0] == 0) == (call == "impact")
     assert few[0] == all_[0] == 0
     assert few[1] < all_[1] if call == "impact" else few[1] > all_[1]
+
+
+def test_counters_do_not_wrap(tmp_path):
+    """The kernels' query counters are 32 bits wide and pass the number of queries by a few thousand before
+    the last wavefront ends: 2^32 - 2 mesh distances go in chunks that leave room for that."""
+    launches = run(tmp_path, """
+pts = np.array([[0, 0, 0], [1, 0, 0], [0, 1, 0]], np.float32)
+tri = np.array([[0, 1, 2]], np.uint32)
+mesh = C.c_void_p()
+assert lib.ncx_trimesh_create(C.byref(ctx), pts.ctypes.data, 3, tri.ctypes.data, 1, C.byref(mesh)) == 0, error()
+a = count("stub_launches")
+assert lib.ncx_mesh_distance_batch(mesh, p, shapes, p, p, (1 << 32) - 2, p) == 0, error()
+print(json.dumps(count("stub_launches") - a))
+""")
+    assert launches == 4 * 2  # a fill and a search each
