@@ -815,9 +815,9 @@ __global__ void k_iota_u32(uint32_t* __restrict__ p, uint32_t n) {
   if (i < n) p[i] = i;
 }
 
-// Re-runs the n records listed at list_src (device; null: the first n) with device-memory arenas 8x larger per round
-// (starting from 8 x the last tier's vcap/fcap) until none overflows; host-driven (synchronises
-// the stream).  Chunks keep each round's arenas <= 2 GiB.  The first round continues the runs
+// Re-runs the n records listed at list_src (device; null: the first n) with device-memory arenas 8x
+// larger per round (starting from 8 x the last tier's vcap/fcap) until none overflows; host-driven
+// (synchronises the stream).  Chunks keep each round's arenas <= 2 GiB.  The first round continues the runs
 // the last LDS tier saved (sus_src, slot = list position); device-memory rounds do not suspend.
 static int rerun_overflows(ContactTiers& T, ncx_ctx* ctx, KArgs a, uint32_t n, const uint32_t* list_src,
                            uint32_t vcap, uint32_t fcap, const uint8_t* sus_src, size_t sus_bytes) {
@@ -1195,6 +1195,7 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
   // Partition (sort by key) unless the batch is small: below 16,384 pairs the three partition
   // kernels and the launches per bucket cost more (about 60 us) than the order saves.
   const bool partition = tune_now || npairs >= NCX_PARTITION_MIN_PAIRS;
+  NCX_REQUIRE(mode == 1 || T.nrec >= (partition ? 1 : npairs), "contact launch: EPA records not allocated");
   T.parts = false;
   if (partition) {
     if ((rc = partition_launch(S, T, ctx, a.poses, a.ia, a.ib, npairs, n_dev))) return rc;
@@ -1204,7 +1205,6 @@ static int launch_tiers(ncx_shapes* S, ContactTiers& T, ncx_ctx* ctx, KArgs a, s
     t.npairs = npairs;
     if (tune_now && (rc = autotune(S, T, ctx, t, mode))) return rc;
   }
-  NCX_REQUIRE(mode == 1 || T.nrec >= (partition ? 1 : npairs), "contact launch: EPA records not allocated");
   if (!partition) {
     // one launch over all pairs, in their own order
     const int big = 31 - __builtin_clz(S->buckets | 1u);  // the variant of the set's largest hulls
